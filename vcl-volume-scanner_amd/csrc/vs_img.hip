@@ -122,10 +122,42 @@ __global__ __launch_bounds__(kTileThreads) void k_pyr_down(const SessParams *__r
 // (z_yooji_image_processor.cpp:119-227): n = normalize(dz/dx, dz/dy, -1) from
 // central differences, 1-pixel border skipped, |dx| or |dy| < 1e-7 rejected,
 // and grazing normals (-n_z <= cos 60 deg) invalidate vertex and normal.
-// Evaluated on the input vertex map (order-independent form).
+struct VnPixel {
+    f3 c, n;                       // vertex; normal (when `normal`)
+    bool valid, normal, grazing;   // depth > 0; accepted normal; rejected as grazing
+};
+__device__ __forceinline__ VnPixel vn_pixel(const float *D, const float *K, int W, int H, int x, int y) {
+    auto vert = [&](int xx, int yy, f3 &v) -> bool {
+        float d = ldg(D, (size_t)yy * W + xx);
+        if (d <= 0.0f) return false;
+        v = {d * ((float)xx - K[2]) / K[0], d * ((float)yy - K[3]) / K[1], d};
+        return true;
+    };
+    VnPixel r;
+    r.normal = r.grazing = false;
+    r.valid = vert(x, y, r.c);
+    if (r.valid && x >= 1 && x < W - 1 && y >= 1 && y < H - 1) {
+        f3 x1, x2, y1, y2;
+        if (vert(x - 1, y, x1) && vert(x + 1, y, x2) && vert(x, y - 1, y1) && vert(x, y + 1, y2)) {
+            float dx = x2.x - x1.x, dy = y2.y - y1.y;
+            if (fabsf(dx) >= 1.0e-7f && fabsf(dy) >= 1.0e-7f) {
+                float gx = (x2.z - x1.z) / dx, gy = (y2.z - y1.z) / dy;
+                float nn = sqrtf(gx * gx + gy * gy + 1.0f);
+                r.n = {gx / nn, gy / nn, -1.0f / nn};
+                r.grazing = -r.n.z <= 0.5f;
+                r.normal = !r.grazing;
+            }
+        }
+    }
+    return r;
+}
+// Without `inv`: every pixel evaluated on the input vertex map (the
+// order-independent form). With it (the reference loop's in-place order,
+// below): one bit per pixel, rows of `nw` 64-bit words, set where the loop
+// invalidates the vertex.
 __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__restrict__ SP,
                                                         const WorkItem *__restrict__ work, int l, float *vtx,
-                                                        float *nrm) {
+                                                        float *nrm, const unsigned long long *inv, int nw) {
     const WorkItem wi = work[blockIdx.x];
     const SessParams &P = SP[wi.sess];
     const LevelDesc &L = P.lev[l];
@@ -133,39 +165,23 @@ __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__rest
     const int x = (wi.tile % L.tiles_x) * kTileW + threadIdx.x % kTileW;
     const int y = (wi.tile / L.tiles_x) * kTileH + threadIdx.x / kTileW;
     if (x >= W || y >= H) return;
-    const float *D = P.filt[l];
-    const float *K = L.K;
-    auto vert = [&](int xx, int yy, f3 &v) -> bool {
-        float d = ldg(D, (size_t)yy * W + xx);
-        if (d <= 0.0f) return false;
-        v = {d * ((float)xx - K[2]) / K[0], d * ((float)yy - K[3]) / K[1], d};
-        return true;
-    };
+    VnPixel r = vn_pixel(P.filt[l], L.K, W, H, x, y);
+    bool gone = r.grazing;
+    if (inv) {
+        auto bit = [&](int xx, int yy) -> bool {
+            return xx >= 0 && yy >= 0 && ((ldg(inv, (size_t)yy * nw + (xx >> 6)) >> (xx & 63)) & 1ull);
+        };
+        gone = bit(x, y);
+        r.normal &= !(bit(x - 1, y) || bit(x, y - 1));
+    }
+    const bool v = r.valid && !gone;
     const size_t t = (size_t)y * W + x;
-    f3 c;
-    bool vc = vert(x, y, c);
-    float o[6] = {-100.f, -100.f, -100.f, -100.f, -100.f, -100.f};
-    if (vc) {
-        o[0] = c.x; o[1] = c.y; o[2] = c.z;
-    }
-    if (vc && x >= 1 && x < W - 1 && y >= 1 && y < H - 1) {
-        f3 x1, x2, y1, y2;
-        if (vert(x - 1, y, x1) && vert(x + 1, y, x2) && vert(x, y - 1, y1) && vert(x, y + 1, y2)) {
-            float dx = x2.x - x1.x, dy = y2.y - y1.y;
-            if (fabsf(dx) >= 1.0e-7f && fabsf(dy) >= 1.0e-7f) {
-                float gx = (x2.z - x1.z) / dx, gy = (y2.z - y1.z) / dy;
-                float nn = sqrtf(gx * gx + gy * gy + 1.0f);
-                float nx = gx / nn, ny = gy / nn, nz = -1.0f / nn;
-                if (-nz <= 0.5f) {
-                    o[0] = o[1] = o[2] = -100.f;
-                } else {
-                    o[3] = nx; o[4] = ny; o[5] = nz;
-                }
-            }
-        }
-    }
-    vtx[3 * t + 0] = o[0]; vtx[3 * t + 1] = o[1]; vtx[3 * t + 2] = o[2];
-    nrm[3 * t + 0] = o[3]; nrm[3 * t + 1] = o[4]; nrm[3 * t + 2] = o[5];
+    stg(vtx, 3 * t + 0, v ? r.c.x : -100.f);
+    stg(vtx, 3 * t + 1, v ? r.c.y : -100.f);
+    stg(vtx, 3 * t + 2, v ? r.c.z : -100.f);
+    stg(nrm, 3 * t + 0, r.normal ? r.n.x : -100.f);
+    stg(nrm, 3 * t + 1, r.normal ? r.n.y : -100.f);
+    stg(nrm, 3 * t + 2, r.normal ? r.n.z : -100.f);
 }
 
 // The reference CPU loop's in-place order (enm_Estimate_Normal_Map,
@@ -174,81 +190,91 @@ __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__rest
 // raster order see its vertex as -100. A grazing pixel is invalidated only
 // when neither its left nor its upper neighbour was:
 //     inv(i, j) = c(i, j) & !inv(i, j-1) & !inv(i-1, j)
-// where c marks the grazing pixels of the order-independent pass (k_vnmap,
-// which has written vtx/nrm already). A grazing pixel that is not
-// invalidated keeps its vertex (its normal was never computed), and a pixel
-// whose left or upper neighbour is invalidated loses its normal. One wave
-// walks the rows: it reads a row's flags as 64-bit ballots, resolves the
-// recurrence along the row word by word (runs of c alternate, starting
-// invalidated unless the pixel before was), and applies the fix-ups.
-__global__ __launch_bounds__(64) void k_vnmap_inplace(const SessParams *__restrict__ SP, int l, float *vtx,
-                                                      float *nrm) {
+// where c marks the grazing pixels of the order-independent form. A grazing
+// pixel that is not invalidated keeps its vertex (its normal was never
+// computed), and a pixel whose left or upper neighbour is invalidated loses
+// its normal. Three launches: the bits of c, the recurrence on bits, the maps.
+// Only the recurrence is serial, one row after another, so it is kept to one
+// wave working on bits alone. (With that wave also reading the maps back and
+// resolving each row's runs one at a time in one lane it had taken 3.2 ms a
+// level: frame preparation and the maps of three levels of a 640x480 frame,
+// alone, 9.31 -> 0.19 ms.)
+
+// One wave per 64 pixels of a row: word k of row y = bits of c.
+__global__ __launch_bounds__(kTileThreads) void k_vn_graze(const SessParams *__restrict__ SP, int l,
+                                                           unsigned long long *bits, int nw) {
     const SessParams &P = SP[0];
     const LevelDesc &L = P.lev[l];
-    const int W = L.W, H = L.H, lane = threadIdx.x;
-    const int nw = (W + 63) >> 6;  // <= 128 words (frames are at most 8192 wide)
-    __shared__ unsigned long long s_up[128], s_c[128], s_n[128], s_inv[128];
-    for (int k = lane; k < nw; k += 64) s_up[k] = 0ull;
-    const float *D = P.filt[l];
-    const float *K = L.K;
-    __syncthreads();
-    for (int i = 1; i < H - 1; ++i) {
-        for (int k = 0; k < nw; ++k) {
-            const int j = (k << 6) + lane;
-            const bool in = j >= 1 && j < W - 1;
-            const size_t t = (size_t)i * W + j;
-            const float vx = in ? vtx[3 * t] : 0.0f;
-            const float nx = in ? nrm[3 * t] : -100.0f;
-            const float d = in ? ldg(D, t) : 0.0f;
-            const unsigned long long cm = __ballot(in && vx == -100.0f && d > 0.0f);
-            const unsigned long long nm = __ballot(in && nx != -100.0f);
-            if (lane == 0) {
-                s_c[k] = cm;
-                s_n[k] = nm;
+    const int item = blockIdx.x * (kTileThreads / 64) + (threadIdx.x >> 6);
+    const int y = item / nw, k = item - y * nw;
+    if (y >= L.H) return;
+    const int x = k * 64 + (threadIdx.x & 63);
+    const bool c = x < L.W && vn_pixel(P.filt[l], L.K, L.W, L.H, x, y).grazing;
+    const unsigned long long m = __ballot(c);
+    if ((threadIdx.x & 63) == 0) stg(bits, (size_t)item, m);
+}
+
+// The recurrence, in place on the bits of c: one wave, lane k holds words
+// k * N .. k * N + N - 1 of a row. Along a row, a run of r = c & ~inv(row
+// above) is invalidated at every other pixel from its first: adding the first
+// bits of the runs that start at even columns to r (one addition over the
+// whole row) clears exactly those runs, which tells the runs' parities apart.
+// The addition's carries cross lanes by the generate / propagate masks of the
+// wave. Bound: a chain of ~25 dependent instructions per row; the rows' bits
+// are loaded kAhead rows ahead of their use.
+template <int N>
+__global__ __launch_bounds__(64) void k_vn_order(unsigned long long *bits, int nw, int H) {
+    constexpr int kAhead = 16;
+    const int lane = threadIdx.x;
+    unsigned long long up[N], nxt[kAhead][N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) up[q] = 0ull;
+    auto fetch = [&](int row0) {
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a)
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const int k = lane * N + q;
+                nxt[a][q] = (k < nw && row0 + a < H) ? ldg(bits, (size_t)(row0 + a) * nw + k) : 0ull;
+            }
+    };
+    fetch(0);
+    for (int row0 = 0; row0 < H; row0 += kAhead) {
+        unsigned long long cur[kAhead][N];
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a)
+#pragma unroll
+            for (int q = 0; q < N; ++q) cur[a][q] = nxt[a][q];
+        fetch(row0 + kAhead);
+#pragma unroll
+        for (int a = 0; a < kAhead; ++a) {
+            unsigned long long r[N], sum[N];
+#pragma unroll
+            for (int q = 0; q < N; ++q) r[q] = cur[a][q] & ~up[q];
+            // last bit of the previous lane's words
+            unsigned prev = __shfl_up((unsigned)(r[N - 1] >> 63), 1, 64);
+            if (lane == 0) prev = 0u;
+            bool carry = false, prop = true;
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                const unsigned long long first = r[q] & ~((r[q] << 1) | prev);
+                const unsigned long long s = r[q] + (first & 0x5555555555555555ull);
+                sum[q] = s + (carry ? 1ull : 0ull);
+                carry = s < r[q] || sum[q] < s;
+                prop &= sum[q] == ~0ull;
+                prev = (unsigned)(r[q] >> 63);
+            }
+            const unsigned long long G = __ballot(carry), Pr = __ballot(prop);
+            bool in = ((((G << 1) + Pr) ^ Pr) >> lane) & 1ull;  // carry into this lane's first word
+#pragma unroll
+            for (int q = 0; q < N; ++q) {
+                sum[q] += in ? 1ull : 0ull;
+                in = in && sum[q] == 0ull;
+                up[q] = r[q] & ((~sum[q] & 0x5555555555555555ull) | (sum[q] & 0xAAAAAAAAAAAAAAAAull));
+                const int k = lane * N + q;
+                if (k < nw && row0 + a < H) stg(bits, (size_t)(row0 + a) * nw + k, up[q]);
             }
         }
-        __syncthreads();
-        if (lane == 0) {
-            bool carry = false;  // inv of the pixel before the word
-            for (int k = 0; k < nw; ++k) {
-                unsigned long long rest = s_c[k] & ~s_up[k], inv = 0ull;
-                while (rest) {
-                    const int s0 = __builtin_ctzll(rest);
-                    const unsigned long long from = rest >> s0;
-                    const int len = (~from == 0ull) ? 64 - s0 : __builtin_ctzll(~from);
-                    const unsigned long long run = (len >= 64 ? ~0ull : ((1ull << len) - 1ull)) << s0;
-                    const int first = s0 + ((s0 == 0 && carry) ? 1 : 0);
-                    inv |= run & ((first & 1) ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull);
-                    rest &= ~run;
-                }
-                s_inv[k] = inv;
-                carry = (inv >> 63) & 1ull;
-            }
-        }
-        __syncthreads();
-        for (int k = 0; k < nw; ++k) {
-            const int j = (k << 6) + lane;
-            if (!(j >= 1 && j < W - 1)) continue;
-            const unsigned long long inv = s_inv[k];
-            const bool c = (s_c[k] >> lane) & 1ull, nv = (s_n[k] >> lane) & 1ull;
-            const bool here = (inv >> lane) & 1ull;
-            const bool left = lane ? ((inv >> (lane - 1)) & 1ull) : (k ? ((s_inv[k - 1] >> 63) & 1ull) : false);
-            const bool up = (s_up[k] >> lane) & 1ull;
-            const size_t t = (size_t)i * W + j;
-            if (c && !here) {
-                const float d = ldg(D, t);
-                vtx[3 * t + 0] = d * ((float)j - K[2]) / K[0];
-                vtx[3 * t + 1] = d * ((float)i - K[3]) / K[1];
-                vtx[3 * t + 2] = d;
-            } else if (nv && (left || up)) {
-                nrm[3 * t + 0] = -100.0f;
-                nrm[3 * t + 1] = -100.0f;
-                nrm[3 * t + 2] = -100.0f;
-            }
-        }
-        __syncthreads();
-        for (int k = lane; k < nw; k += 64) s_up[k] = s_inv[k];
-        __syncthreads();
     }
 }
 
@@ -297,10 +323,22 @@ void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int l, hi
     if (n > 0) hipLaunchKernelGGL(k_pyr_down, dim3(n), dim3(kTileThreads), 0, s, P, work, l);
 }
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int l, float *vtx, float *nrm, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm);
+    if (n > 0)
+        hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm,
+                           (const unsigned long long *)nullptr, 0);
 }
-void launch_vnmap_inplace(const SessParams *P, int l, float *vtx, float *nrm, hipStream_t s) {
-    hipLaunchKernelGGL(k_vnmap_inplace, dim3(1), dim3(64), 0, s, P, l, vtx, nrm);
+void launch_vnmap_inplace(const SessParams *P, const WorkItem *work, int n, int l, int W, int H,
+                          unsigned long long *bits, float *vtx, float *nrm, hipStream_t s) {
+    if (n <= 0) return;
+    const int nw = vn_words(W);  // at most 128 (frames are at most 8192 wide)
+    const size_t items = (size_t)nw * H, per = kTileThreads / 64;
+    hipLaunchKernelGGL(k_vn_graze, dim3((unsigned)((items + per - 1) / per)), dim3(kTileThreads), 0, s, P, l, bits, nw);
+    if (nw <= 64)
+        hipLaunchKernelGGL(k_vn_order<1>, dim3(1), dim3(64), 0, s, bits, nw, H);
+    else
+        hipLaunchKernelGGL(k_vn_order<2>, dim3(1), dim3(64), 0, s, bits, nw, H);
+    hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm,
+                       (const unsigned long long *)bits, nw);
 }
 
 }  // namespace vs

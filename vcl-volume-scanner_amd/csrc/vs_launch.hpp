@@ -20,8 +20,11 @@ void launch_fill_u32(uint32_t *p, size_t n, uint32_t v, hipStream_t s);
 void launch_bilateral(const SessParams *P, const WorkItem *work, int n, hipStream_t s);
 void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int level, hipStream_t s);
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int level, float *vtx, float *nrm, hipStream_t s);
-// single session (P[0]): after launch_vnmap, the reference loop's in-place order
-void launch_vnmap_inplace(const SessParams *P, int level, float *vtx, float *nrm, hipStream_t s);
+// single session (P[0]), the reference loop's in-place order; bits: vn_words(W)
+// * H words of scratch
+constexpr int vn_words(int W) { return (W + 63) / 64; }
+void launch_vnmap_inplace(const SessParams *P, const WorkItem *work, int n, int level, int W, int H,
+                          unsigned long long *bits, float *vtx, float *nrm, hipStream_t s);
 
 // tracker (vs_icp.hip); nsess = sessions in the batch
 void launch_track_setup(const SessParams *P, int nsess, const double *T_init, hipStream_t s);
