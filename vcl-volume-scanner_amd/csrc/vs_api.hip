@@ -74,7 +74,7 @@ struct Layout {
     size_t total;
     size_t nvox;
     uint32_t nbricks, nwords, nsuper, nswords;
-    int sdim[3];
+    int sdim[3], sshift;
     int tiles[kMaxLevels];
 };
 
@@ -105,7 +105,8 @@ Layout make_layout(const vs_session_desc &d) {
     L.nvox = (size_t)d.vol_dim[0] * d.vol_dim[1] * d.vol_dim[2];
     L.nbricks = (uint32_t)((d.vol_dim[0] / 8) * (d.vol_dim[1] / 8) * (d.vol_dim[2] / 8));
     L.nwords = (L.nbricks + 31) / 32;
-    for (int k = 0; k < 3; ++k) L.sdim[k] = (d.vol_dim[k] / kBrick + (1 << kSuperShift) - 1) >> kSuperShift;
+    L.sshift = super_shift(d.vol_dim[0] / kBrick, d.vol_dim[1] / kBrick, d.vol_dim[2] / kBrick);
+    for (int k = 0; k < 3; ++k) L.sdim[k] = (d.vol_dim[k] / kBrick + (1 << L.sshift) - 1) >> L.sshift;
     L.nsuper = (uint32_t)(L.sdim[0] * L.sdim[1] * L.sdim[2]);
     L.nswords = (L.nsuper + 31) / 32;
     const size_t sv = d.tsdf_type == VS_TSDF_F16 ? 2 : 4, sw = d.weight_type == VS_WEIGHT_U8 ? 1 : 4;
@@ -290,7 +291,7 @@ struct Batch {
     BrickList bl{};
     uint32_t bricks = 0;    // capacity of the brick list
     uint32_t max_words = 0; // longest visible-brick bitmap of a member (32-bit words)
-    bool o32 = false;       // every member's voxel records are below 4 GB
+    int addr = kAddr64;     // how the raycast addresses the members' voxels (VoxAddr)
     int integ_grid = 1;     // default integrate grid
     Shape shape;
     std::string size_class;
@@ -392,11 +393,14 @@ struct ListSet {
     std::vector<WorkItem> tile[kMaxLevels], group[kMaxLevels];
     uint32_t bricks = 0, max_words = 0;
     size_t max_array = 0;  // largest voxel-record array of a member (bytes)
+    int max_shift = 0, sd_slices = 0;  // largest superbrick, most superbricks along z
     int levels = 0, max_iters[kMaxLevels] = {0, 0, 0};
     int count = 0, max_w = 0, max_h = 0, max_dim = 0;
     void add(int slot, const vs_session *s) {
         ++count;
         max_words = std::max(max_words, s->L.nwords);
+        max_shift = std::max(max_shift, s->L.sshift);
+        sd_slices = std::max(sd_slices, s->L.sdim[2]);
         max_array = std::max(max_array, s->L.nvox * vox_rec_bytes(s->d.tsdf_type == VS_TSDF_F16,
                                                                   s->d.weight_type == VS_WEIGHT_U8));
         max_w = std::max(max_w, s->d.width);
@@ -480,11 +484,11 @@ struct ListSet {
     // Iteration bounds, integrate grid and size class of the batch.
     vs_status settle(Batch &B, int integ_max) const {
         B.levels = levels;
-        B.sd_slices = (max_dim / kBrick + (1 << kSuperShift) - 1) >> kSuperShift;
+        B.sd_slices = sd_slices;
         for (int l = 0; l < kMaxLevels; ++l) B.max_iters[l] = max_iters[l];
         B.bricks = bricks;
         B.max_words = max_words;
-        B.o32 = max_array < (size_t(1) << 32);
+        B.addr = max_array >= (size_t(1) << 32) ? kAddr64 : max_shift > kSuperShift ? kAddr32 : kAddrSmall;
         B.integ_grid = (int)std::max<uint32_t>(1, std::min<uint32_t>(bricks, (uint32_t)integ_max));
         // size class: largest frame, largest volume edge and session count
         // rounded up to powers of two, storage types
@@ -735,10 +739,10 @@ void enqueue_step(const Batch &B, hipStream_t s, Timer *timed) {
     launch_integrate(B.dP, B.n, B.bl, B.tt, B.wt, integ_grid(B), B.sd_slices, s);
     mark(5);
     const LevelWork lw = level_work(B.dWork, B.nWork, B.levels);
-    launch_raycast_march(B.dP, lw, B.tt, B.wt, nullptr, B.shape.march, B.o32, s);
+    launch_raycast_march(B.dP, lw, B.tt, B.wt, nullptr, B.shape.march, B.addr, s);
     mark(6);
     launch_raycast_shade(B.dP, lw, B.tt, B.wt, nullptr, kShadeOpts[B.shape.shade].block,
-                         kShadeOpts[B.shape.shade].waves, B.o32, s);
+                         kShadeOpts[B.shape.shade].waves, B.addr, s);
     mark(7);
     mark(8);
     if (timed) timed->used = true;
@@ -1230,6 +1234,7 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
     P.sdist = (uint8_t *)(m + L.sdist);
     P.sdtmp = (uint8_t *)(m + L.sdtmp);
     for (int k = 0; k < 3; ++k) P.sdim[k] = L.sdim[k];
+    P.sshift = L.sshift;
     P.sband_words = (int)L.nswords;
     P.icp_part = (double *)(m + L.icp_part);
     {
@@ -1524,7 +1529,7 @@ vs_status vs_raycast(vs_session *s, int level, vs_stream stream) {
     hipStream_t h = pick(s, stream);
     const Batch &B = s->self;
     launch_fuse_ok(B.dP, 1, h);
-    launch_raycast(B.dP, B.dWork[level], B.nWork[level], level, B.tt, B.wt, B.o32, h);
+    launch_raycast(B.dP, B.dWork[level], B.nWork[level], level, B.tt, B.wt, B.addr, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }

@@ -43,14 +43,25 @@ __host__ __device__ constexpr int icp_groups(int tiles, int level) { return (til
 // field (below) is kept per superbrick and copied to each raycast
 // workgroup's LDS, whose 16 KB hold the 32^3 superbricks of a 512^3 grid;
 // smaller cells bound the band regions more tightly (a band superbrick of
-// 32^3 voxels left the march ~6 brick-sized boxes per ray inside it).
-constexpr int kSuperShift = 1;                   // log2(bricks per superbrick edge)
-constexpr int kSuper = kBrick << kSuperShift;    // superbrick edge (voxels)
+// 32^3 voxels left the march ~6 brick-sized boxes per ray inside it). A grid
+// of more cells takes the smallest superbrick that fits the copy (32^3
+// voxels up to 1024^3, 64^3 up to 2048^3; SessParams::sshift). Without a
+// field of its own, the raycast of a 1024^3 grid skipped one brick at a
+// time (a 1280x960 frame fused and rendered once more: 2.84 ms, now 1.28).
+constexpr int kSuperShift = 1;                   // log2(bricks per superbrick edge) of the grids that fit
 // Superbrick distance field: per superbrick the L-infinity distance (in
 // superbricks, capped at kDistMax) to the nearest band superbrick, 4 bits
-// each; sessions of up to kDistCells superbricks (512^3 voxels) have one.
+// each, at most kDistCells superbricks.
 constexpr int kDistMax = 15;
 constexpr int kDistCells = 32768;
+// log2(bricks per superbrick edge) of a grid of bx x by x bz bricks (each at
+// most 256: the cells fit by shift 3)
+inline int super_shift(int bx, int by, int bz) {
+    int sh = kSuperShift;
+    auto n = [&](int b) { return (size_t)((b + (1 << sh) - 1) >> sh); };
+    while (n(bx) * n(by) * n(bz) > (size_t)kDistCells) ++sh;
+    return sh;
+}
 
 struct LevelDesc {
     int W, H;
@@ -131,13 +142,14 @@ struct alignas(16) SessParams {
     uint32_t *bocc;          // bricks holding any weight > 0 (monotone)
     // Band bits (set-only, so a superset): a brick whose bit is clear holds
     // only voxels of weight 0 or value exactly 1.0, which the raycast's march
-    // steps through like empty space; a superbrick (2^3 bricks = 16^3 voxels)
+    // steps through like empty space; a superbrick (2^sshift bricks an edge)
     // whose bit is clear holds no band brick.
     uint32_t *bband;
     uint32_t *sband;
     uint8_t *sdist;          // superbrick distance field, 2 superbricks per byte (low nibble first)
     uint8_t *sdtmp;          // its rebuild's scratch: one byte per superbrick
     int sdim[3];             // superbricks per axis
+    int sshift;              // log2(bricks per superbrick edge)
     int sband_words;         // 32-bit words of sband
     double *icp_part;        // ICP group partials (kIcpVals per group of level-0 tiles)
     // World coordinate of each voxel centre along each axis, the reference's
@@ -312,7 +324,7 @@ __device__ __forceinline__ int brick_of(const SessParams &P, int x, int y, int z
 }
 // superbrick of brick (bx, by, bz)
 __device__ __forceinline__ int super_of_brick(const SessParams &P, int bx, int by, int bz) {
-    return ((bz >> kSuperShift) * P.sdim[1] + (by >> kSuperShift)) * P.sdim[0] + (bx >> kSuperShift);
+    return ((bz >> P.sshift) * P.sdim[1] + (by >> P.sshift)) * P.sdim[0] + (bx >> P.sshift);
 }
 
 // Voxel records. A voxel's value and weight share one record, so a lookup

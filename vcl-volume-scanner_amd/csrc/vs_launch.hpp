@@ -55,10 +55,14 @@ void launch_vis_mark(const SessParams *P, const WorkItem *work, int n, int nsess
 // sd_slices: the most superbricks along z of any session (distance field)
 void launch_integrate(const SessParams *P, int nsess, BrickList bl, int tsdf_type, int weight_type, int grid,
                       int sd_slices, hipStream_t s);
-// o32: every session's voxel records are below 4 GB (the march and the
-// shading then address them with 32-bit offsets)
+// How the raycast addresses the sessions of a launch: 32-bit offsets when
+// every session's voxel records are below 4 GB, and then a compile-time
+// superbrick size when every session has the one of grids up to 512^3 (whose
+// records are at most 1 GB). The form for mixed and large grids reads the
+// superbrick size per session.
+enum VoxAddr { kAddrSmall = 0, kAddr32 = 1, kAddr64 = 2 };
 void launch_raycast(const SessParams *P, const WorkItem *work, int n, int level, int tsdf_type, int weight_type,
-                    bool o32, hipStream_t s);
+                    int addr, hipStream_t s);
 // a single session's model maps of `level` (npx pixels) into caller buffers
 // (each nullable): depth, vertex and normal (3 floats per pixel), image
 void launch_maps_out(const SessParams *P, int level, size_t npx, float *depth, float *vtx, float *nrm, uint8_t *img,
@@ -82,12 +86,12 @@ LevelWork level_work(const WorkItem *const work[kMaxLevels], const int n[kMaxLev
 void launch_sdist(const SessParams *P, int nsess, int sd_slices, int force, hipStream_t s);
 // Ray block of one wave in the raycast kernels (same results for each).
 enum RayBlock { kRay8x8 = 0, kRay16x4 = 1, kRay32x2 = 2 };
-// o32 as for launch_raycast
+// addr: VoxAddr
 void launch_raycast_march(const SessParams *P, const LevelWork &lw, int tsdf_type, int weight_type,
-                          unsigned long long *stats, int ray_block, bool o32, hipStream_t s);
-// waves: the waves per SIMD its registers aim for (4 or 5); o32 as for launch_raycast
+                          unsigned long long *stats, int ray_block, int addr, hipStream_t s);
+// waves: the waves per SIMD its registers aim for (4 or 5); addr: VoxAddr
 void launch_raycast_shade(const SessParams *P, const LevelWork &lw, int tsdf_type, int weight_type,
-                          unsigned long long *stats, int ray_block, int waves, bool o32, hipStream_t s);
+                          unsigned long long *stats, int ray_block, int waves, int addr, hipStream_t s);
 // volume maintenance (single session, P points at its parameters)
 void launch_volume_init(const SessParams *P, size_t nvox, int tsdf_type, int weight_type, uint32_t nwords,
                         int sd_slices, hipStream_t s);

@@ -457,7 +457,7 @@ constexpr int kSdistThreads = 1024, kSdistChunk = 2 * kSdistThreads;
 
 __device__ __forceinline__ bool sdist_todo(const SessParams &P, int force) {
     const int n = P.sdim[0] * P.sdim[1] * P.sdim[2];
-    return n > 0 && n <= kDistCells && (force || ldg(&P.st->sdist_dirty, 0));
+    return n > 0 && (force || ldg(&P.st->sdist_dirty, 0));
 }
 
 // min of rd(c) and, over 0 < |t| < kDistMax with pos + t in [0, len), of
@@ -541,14 +541,15 @@ __device__ __forceinline__ bool below3(int x, int y, int z, int nx, int ny, int 
     return (int)((unsigned)x < (unsigned)nx) & (int)((unsigned)y < (unsigned)ny) & (int)((unsigned)z < (unsigned)nz);
 }
 
-template <class TV, class TW>
+// AD (VoxAddr): 32- or 64-bit record offsets, superbrick size known or read
+// from the session.
+template <class TV, class TW, int AD>
 struct Vol {
+    static constexpr bool O32 = AD != kAddr64;
     const SessParams &P;
     const void *vx;  // voxel records
     // superbrick distance field: the workgroup's LDS copy (4 bits per
-    // superbrick). A session without one gets zeros (every superbrick counts
-    // as a band one and only the brick bits decide); the index is masked to
-    // the copy's size either way.
+    // superbrick); the index is masked to the copy's size
     const VS_LDS uint8_t *sdist;
     // of the last brick looked up (a ray's consecutive taps mostly stay in
     // one brick; the bitmaps are read-only during the launch), in one
@@ -557,6 +558,8 @@ struct Vol {
     // = the brick is a band one
     static constexpr unsigned kIdx = 0x01FFFFFFu, kBrickBand = 1u << 31;
     mutable unsigned cbf = kIdx;
+    // log2(voxels per superbrick edge)
+    __device__ __forceinline__ int super_log2() const { return 3 + (AD == kAddrSmall ? kSuperShift : P.sshift); }
     __device__ __forceinline__ int cb() const { return (int)(cbf & kIdx); }
     __device__ __forceinline__ int dist() const { return (int)((cbf >> 25) & 15u); }
     __device__ __forceinline__ bool band(int x, int y, int z) const {
@@ -565,7 +568,7 @@ struct Vol {
         const unsigned b = __umul24(__umul24((unsigned)z >> 3, (unsigned)P.bdim[1]) + ((unsigned)y >> 3),
                                     (unsigned)P.bdim[0]) + ((unsigned)x >> 3);
         if (b != (cbf & kIdx)) {
-            constexpr int ss = 3 + kSuperShift;
+            const int ss = super_log2();
             const unsigned sb = __umul24(__umul24((unsigned)z >> ss, (unsigned)P.sdim[1]) + ((unsigned)y >> ss),
                                          (unsigned)P.sdim[0]) + ((unsigned)x >> ss);
             const unsigned d = (sdist[(sb >> 1) & (kDistCells / 2 - 1)] >> ((sb & 1u) * 4u)) & 15u;
@@ -588,7 +591,6 @@ struct Vol {
         return ok;
     }
     // voxel (x, y, z) in range; O32: 32-bit offsets (records below 4 GB)
-    template <bool O32>
     __device__ __forceinline__ bool load_at(int x, int y, int z, float &out) const {
         if (!O32) return load(vox_index(P, x, y, z), out);
         typedef VoxRec<TV, TW> R;
@@ -599,7 +601,6 @@ struct Vol {
     }
     // voxel b * 512 + l (brick index b, in-brick offset l < 512); O32 as for
     // load_at
-    template <bool O32>
     __device__ __forceinline__ bool load_bl(unsigned b, unsigned l, float &out) const {
         if (!O32) return load((size_t)b * kBrickVox + l, out);
         typedef VoxRec<TV, TW> R;
@@ -626,7 +627,6 @@ struct Vol {
     // [lo, lo + size)^3 (a superbrick or brick without band bit) reads 1.0,
     // size = -1 when the position is outside the grid (moving towards it),
     // size = 0 otherwise.
-    template <bool O32>
     __device__ __forceinline__ int nearest(f3 v, f3 rd, float &out, int3 &lo, int &size) const {
         out = 1.0f;
         size = 0;
@@ -650,12 +650,12 @@ struct Vol {
             // superbrick); d > 0: the (2d-1)^3 superbricks centred here,
             // which hold no band brick
             const int d = dist();
-            const int sh = d == 0 ? 3 : 3 + kSuperShift, r = max(d - 1, 0), unit = 1 << sh;
+            const int sh = d == 0 ? 3 : super_log2(), r = max(d - 1, 0), unit = 1 << sh;
             lo = make_int3(((x >> sh) - r) * unit, ((y >> sh) - r) * unit, ((z >> sh) - r) * unit);
             size = (2 * r + 1) * unit;
             return 0;
         }
-        return load_bl<O32>((unsigned)cb(), (unsigned)(((z & 7) << 6) | ((y & 7) << 3) | (x & 7)), out) ? 1 : 0;
+        return load_bl((unsigned)cb(), (unsigned)(((z & 7) << 6) | ((y & 7) << 3) | (x & 7)), out) ? 1 : 0;
     }
     // ---- instrumented form only: the bytes the reference's own lookups
     // request, tap by tap, in its order and with its early exits.
@@ -707,7 +707,6 @@ struct Vol {
     // 1.0. The 2x2x2 stencil is range-checked as a whole and its 8 values and
     // weights are loaded together; a voxel of an empty brick has weight 0, so
     // no occupancy lookup is needed here.
-    template <bool O32>
     __device__ __forceinline__ bool trilinear(f3 v, float &out) const {
         out = 1.0f;
         if (!finite3(v)) return false;
@@ -736,7 +735,7 @@ struct Vol {
         for (int k = 0; k < 8; ++k) {
             const unsigned b = Bz[k >> 2] + By[(k >> 1) & 1] + Bx[k & 1];
             const unsigned l = Lz[k >> 2] | Ly[(k >> 1) & 1] | Lx[k & 1];
-            ok &= load_bl<O32>(b, l, f[k]);
+            ok &= load_bl(b, l, f[k]);
         }
         if (!ok) return false;
         const float fi = (1.0f - ry) * ((1.0f - rx) * f[0] + rx * f[1]) + ry * ((1.0f - rx) * f[2] + rx * f[3]);
@@ -806,22 +805,22 @@ __device__ __forceinline__ int steps_outside(f3 v, f3 d, const int *vdim) {
 struct RayStats {
     unsigned n_near = 0, n_tri = 0, n_out = 0, n_w0 = 0;
     unsigned long long b_near = 0, b_tri = 0;
-    template <class TV, class TW>
-    __device__ __forceinline__ void nearest(const Vol<TV, TW> &V, f3 v) {
+    template <class TV, class TW, int AD>
+    __device__ __forceinline__ void nearest(const Vol<TV, TW, AD> &V, f3 v) {
         ++n_near;
         const int c = V.ref_nearest(v, b_near);
         n_out += c == 0;
         n_w0 += c == 1;
     }
-    template <class TV, class TW>
-    __device__ __forceinline__ void trilinear(const Vol<TV, TW> &V, f3 v) {
+    template <class TV, class TW, int AD>
+    __device__ __forceinline__ void trilinear(const Vol<TV, TW, AD> &V, f3 v) {
         ++n_tri;
         V.ref_trilinear(v, b_tri);
     }
 };
 
-template <class TV, class TW, bool STATS, bool O32>
-__device__ __forceinline__ bool cast_ray(const Vol<TV, TW> &V, const RayConst &C, const float *Tcg, float px,
+template <class TV, class TW, bool STATS, int AD>
+__device__ __forceinline__ bool cast_ray(const Vol<TV, TW, AD> &V, const RayConst &C, const float *Tcg, float px,
                                          float py, f3 &hit, RayStats &rs) {
     const float dist_min = C.dist_cc - C.r_cube, dist_max = C.dist_cc + C.r_cube;
     const f3 pe = transform(Tcg, back_project(px, py, C.K, dist_max));
@@ -879,7 +878,7 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW> &V, const RayConst &C
         // instrumented form keeps marching to count the reference's taps.
         int3 lo;
         int size;
-        if (V.template nearest<O32>(vox, rd, tsdf, lo, size) < 0 && !STATS) return false;
+        if (V.nearest(vox, rd, tsdf, lo, size) < 0 && !STATS) return false;
         if (!STATS && size != 0) {
             // 1.0 here and in the region around: skip the steps that stay
             // inside it (tsdf is 1.0, so the next step is the same S each time)
@@ -912,7 +911,7 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW> &V, const RayConst &C
         }
         if (fabsf(tsdf) < 1.0f) {
             if (STATS) rs.trilinear(V, vox);
-            V.template trilinear<O32>(vox, tsdf);
+            V.trilinear(vox, tsdf);
             if (tsdf < 0.0f) {
                 if (coarse) return false;
                 behind = true;
@@ -929,7 +928,7 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW> &V, const RayConst &C
     float step = C.step_scale * tsdf;
     vox = add(vox, scale(step, rd));
     if (STATS) rs.trilinear(V, vox);
-    V.template trilinear<O32>(vox, tsdf);
+    V.trilinear(vox, tsdf);
     step = C.step_scale * tsdf;
     vox = add(vox, scale(step, rd));
     hit = voxel_to_world(V.P, vox);
@@ -938,8 +937,8 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW> &V, const RayConst &C
 
 // d_csnt_Compute_Surface_Normal_from_TSDF: central differences of trilinear
 // values from 32 taps around the hit.
-template <bool O32, class TV, class TW>
-__device__ __forceinline__ bool surface_normal(const Vol<TV, TW> &V, f3 p, f3 &n) {
+template <class TV, class TW, int AD>
+__device__ __forceinline__ bool surface_normal(const Vol<TV, TW, AD> &V, f3 p, f3 &n) {
     f3 vox;
     if (!world_to_voxel(V.P, p, vox)) return false;
     const int ox = (int)vox.x, oy = (int)vox.y, oz = (int)vox.z;
@@ -955,13 +954,13 @@ __device__ __forceinline__ bool surface_normal(const Vol<TV, TW> &V, f3 p, f3 &n
     float fm[4], fr[12], bk[12], bm[4];
     bool ok = true;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ok &= V.template load_at<O32>(ox + dx1[i], oy + dy1[i], oz - 1, fm[i]);
+    for (int i = 0; i < 4; ++i) ok &= V.load_at(ox + dx1[i], oy + dy1[i], oz - 1, fm[i]);
 #pragma unroll
-    for (int i = 0; i < 12; ++i) ok &= V.template load_at<O32>(ox + dx2[i], oy + dy2[i], oz, fr[i]);
+    for (int i = 0; i < 12; ++i) ok &= V.load_at(ox + dx2[i], oy + dy2[i], oz, fr[i]);
 #pragma unroll
-    for (int i = 0; i < 12; ++i) ok &= V.template load_at<O32>(ox + dx2[i], oy + dy2[i], oz + 1, bk[i]);
+    for (int i = 0; i < 12; ++i) ok &= V.load_at(ox + dx2[i], oy + dy2[i], oz + 1, bk[i]);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ok &= V.template load_at<O32>(ox + dx1[i], oy + dy1[i], oz + 2, bm[i]);
+    for (int i = 0; i < 4; ++i) ok &= V.load_at(ox + dx1[i], oy + dy1[i], oz + 2, bm[i]);
     if (!ok) return false;
     auto Lz = [&](int i) { return (1.0f - rz) * fr[i] + rz * bk[i]; };
     float a4[4], b4[4], a2[2], b2[2];
@@ -1007,8 +1006,8 @@ __device__ __forceinline__ bool surface_normal(const Vol<TV, TW> &V, f3 p, f3 &n
 // lookup fail, which leaves (0, 0, 0) (the caller ignores the return,
 // :1171-1175). The stencil is range-checked as a whole and its 16 loads are
 // issued together.
-template <class TV, class TW>
-__device__ __forceinline__ uint32_t rgb_interpolated(const Vol<TV, TW> &V, const uint32_t *col, f3 v) {
+template <class TV, class TW, int AD>
+__device__ __forceinline__ uint32_t rgb_interpolated(const Vol<TV, TW, AD> &V, const uint32_t *col, f3 v) {
     if (!(fabsf(v.x) < 2147483520.0f && fabsf(v.y) < 2147483520.0f && fabsf(v.z) < 2147483520.0f)) return 0u;
     const int ox = (int)v.x, oy = (int)v.y, oz = (int)v.z;
     if (!V.in_grid(ox, oy, oz) || !V.in_grid(ox + 1, oy + 1, oz + 1)) return 0u;
@@ -1077,9 +1076,8 @@ __device__ __forceinline__ void ray_pixel(int t, int &px, int &py) {
 // 8 waves per SIMD (at most 64 VGPRs): the march is VALU-bound with dependent
 // taps, and the extra waves hide the taps' latency better than the few
 // registers the compiler would add beyond 64.
-// O32: the lookups take 32-bit offsets from the voxel-record base (every
-// session of the launch has its records below 4 GB), as in k_raycast_shade.
-template <class TV, class TW, bool STATS, int RB, bool O32>
+// AD: VoxAddr of the launch.
+template <class TV, class TW, bool STATS, int RB, int AD>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_raycast(
     const SessParams *__restrict__ SP, LevelWork lw, unsigned long long *stats) {
     __shared__ uint32_t s_dist[kDistCells / 8];
@@ -1090,12 +1088,8 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
     const LevelDesc &L = P.lev[level];
     if (!st->fuse_ok || level >= P.levels || tile_out(L, wi.tile)) return;
     const int ncell = P.sdim[0] * P.sdim[1] * P.sdim[2];
-    if (ncell <= kDistCells) {
-        const uint32_t *src = (const uint32_t *)P.sdist;
-        for (int i = threadIdx.x; i < (ncell + 7) / 8; i += kTileThreads) s_dist[i] = ldg(src, i);
-    } else {
-        for (int i = threadIdx.x; i < kDistCells / 8; i += kTileThreads) s_dist[i] = 0u;
-    }
+    const uint32_t *src = (const uint32_t *)P.sdist;
+    for (int i = threadIdx.x; i < (ncell + 7) / 8; i += kTileThreads) s_dist[i] = ldg(src, i);
     __syncthreads();
     int px, py;
     ray_pixel<RB>(threadIdx.x, px, py);
@@ -1113,11 +1107,11 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
     C.step_scale = P.step_scale;
     C.total_max = P.total_max;
     C.max_iter = P.max_iter;
-    const Vol<TV, TW> V{P, P.vox, (const VS_LDS uint8_t *)s_dist};
+    const Vol<TV, TW, AD> V{P, P.vox, (const VS_LDS uint8_t *)s_dist};
     RayStats rs;
     f3 p;
     const M34 Tc = ld_m34(st->T_cg_f);
-    const bool ok = cast_ray<TV, TW, STATS, O32>(V, C, Tc.m, (float)x, (float)y, p, rs);
+    const bool ok = cast_ray<TV, TW, STATS, AD>(V, C, Tc.m, (float)x, (float)y, p, rs);
     const size_t t = (size_t)y * L.W + x;
     if (ok) {
         st_mvtx(P.mvn[level], t, p.x, p.y, p.z);  // world hit; the shading makes it the camera-frame vertex
@@ -1140,11 +1134,11 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
 // WV: the waves per SIMD the register allocation aims for (4: the compiler's
 // own choice, ~126 VGPRs with all 64 stencil loads in flight; 5: 91, fewer
 // loads in flight); the same results for each, so the autotuner picks. (6
-// waves, 80 VGPRs, spills a few registers and was slower still.) O32: the
-// stencil's loads take 32-bit offsets from the array bases (every session
+// waves, 80 VGPRs, spills a few registers and was slower still.) AD: kAddr32
+// or kAddr64; with the former the stencil's loads take 32-bit offsets from the array bases (every session
 // of the launch has its voxel records below 4 GB): 62 VGPRs instead of 101 at
 // WV 4, the same results.
-template <class TV, class TW, bool STATS, int RB, int WV, bool O32>
+template <class TV, class TW, bool STATS, int RB, int WV, int AD>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(WV == 4 ? 1 : WV, WV == 4 ? 8 : WV)))
 void k_raycast_shade(
     const SessParams *__restrict__ SP, LevelWork lw, unsigned long long *stats) {
@@ -1164,7 +1158,7 @@ void k_raycast_shade(
     // or -100 for a miss, which is final already
     const MapXYZ h = ld_mvtx(P.mvn[level], t);
     if (h.x == -100.0f) return;
-    const Vol<TV, TW> V{P, P.vox, nullptr};
+    const Vol<TV, TW, AD> V{P, P.vox, nullptr};
     const f3 p = {h.x, h.y, h.z};
     if (STATS) {
         unsigned long long b = 0;
@@ -1172,7 +1166,7 @@ void k_raycast_shade(
         atomicAdd(stats + 7, b);
     }
     f3 n;
-    if (surface_normal<O32>(V, p, n)) {
+    if (surface_normal(V, p, n)) {
         const M34 Tg = ld_m34(st->T_gc_f);
         const float *T = Tg.m;
         const f3 pc = transform(T, p);
@@ -1423,21 +1417,20 @@ void launch_integrate(const SessParams *P, int nsess, BrickList bl, int tt, int 
 }
 
 template <class TV, class TW>
-static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, bool o32,
+static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int addr,
                     hipStream_t s) {
     const int n = lw.blocks();
     if (n <= 0) return;
-#define VS_MARCH(RB_)                                                                                          \
-    do {                                                                                                       \
-        if (o32)                                                                                               \
-            hipLaunchKernelGGL((k_raycast<TV, TW, false, RB_, true>), dim3(n), dim3(kTileThreads), 0, s, P, lw, \
-                               stats);                                                                         \
-        else                                                                                                   \
-            hipLaunchKernelGGL((k_raycast<TV, TW, false, RB_, false>), dim3(n), dim3(kTileThreads), 0, s, P, lw, \
-                               stats);                                                                         \
+#define VS_MARCH_A(RB_, AD_) \
+    hipLaunchKernelGGL((k_raycast<TV, TW, false, RB_, AD_>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats)
+#define VS_MARCH(RB_)                                        \
+    do {                                                     \
+        if (addr == kAddrSmall) VS_MARCH_A(RB_, kAddrSmall); \
+        else if (addr == kAddr32) VS_MARCH_A(RB_, kAddr32);  \
+        else VS_MARCH_A(RB_, kAddr64);                       \
     } while (0)
     if (stats)
-        hipLaunchKernelGGL((k_raycast<TV, TW, true, kRay8x8, false>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats);
+        hipLaunchKernelGGL((k_raycast<TV, TW, true, kRay8x8, kAddr64>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats);
     else if (rb == kRay16x4)
         VS_MARCH(kRay16x4);
     else if (rb == kRay32x2)
@@ -1445,23 +1438,23 @@ static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long
     else
         VS_MARCH(kRay8x8);
 #undef VS_MARCH
+#undef VS_MARCH_A
 }
 template <class TV, class TW>
 static void shade_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int waves,
-                    bool o32, hipStream_t s) {
+                    int addr, hipStream_t s) {
     const int n = lw.blocks();
     if (n <= 0) return;
-#define VS_SHADE(RB_, WV_)                                                                                      \
-    do {                                                                                                        \
-        if (o32)                                                                                                \
-            hipLaunchKernelGGL((k_raycast_shade<TV, TW, false, RB_, WV_, true>), dim3(n), dim3(kTileThreads), 0, \
-                               s, P, lw, stats);                                                                \
-        else                                                                                                    \
-            hipLaunchKernelGGL((k_raycast_shade<TV, TW, false, RB_, WV_, false>), dim3(n), dim3(kTileThreads),  \
-                               0, s, P, lw, stats);                                                             \
+#define VS_SHADE_A(RB_, WV_, AD_)                                                                              \
+    hipLaunchKernelGGL((k_raycast_shade<TV, TW, false, RB_, WV_, AD_>), dim3(n), dim3(kTileThreads), 0, s, P, lw, \
+                       stats)
+#define VS_SHADE(RB_, WV_)                                     \
+    do {                                                       \
+        if (addr != kAddr64) VS_SHADE_A(RB_, WV_, kAddr32);    \
+        else VS_SHADE_A(RB_, WV_, kAddr64);                    \
     } while (0)
     if (stats)
-        hipLaunchKernelGGL((k_raycast_shade<TV, TW, true, kRay32x2, 4, false>), dim3(n), dim3(kTileThreads), 0, s, P,
+        hipLaunchKernelGGL((k_raycast_shade<TV, TW, true, kRay32x2, 4, kAddr64>), dim3(n), dim3(kTileThreads), 0, s, P,
                            lw, stats);
     else if (rb == kRay8x8 && waves == 5)
         VS_SHADE(kRay8x8, 5);
@@ -1472,6 +1465,7 @@ static void shade_t(const SessParams *P, const LevelWork &lw, unsigned long long
     else
         VS_SHADE(kRay32x2, 4);
 #undef VS_SHADE
+#undef VS_SHADE_A
 }
 LevelWork level_work(const WorkItem *const work[kMaxLevels], const int n[kMaxLevels], int levels) {
     LevelWork lw{};
@@ -1485,12 +1479,12 @@ LevelWork level_work(const WorkItem *const work[kMaxLevels], const int n[kMaxLev
     return lw;
 }
 void launch_raycast_march(const SessParams *P, const LevelWork &lw, int tt, int wt, unsigned long long *stats,
-                          int rb, bool o32, hipStream_t s) {
-    VS_DISPATCH(tt, wt, march_t, P, lw, stats, rb, o32, s);
+                          int rb, int addr, hipStream_t s) {
+    VS_DISPATCH(tt, wt, march_t, P, lw, stats, rb, addr, s);
 }
 void launch_raycast_shade(const SessParams *P, const LevelWork &lw, int tt, int wt, unsigned long long *stats,
-                          int rb, int waves, bool o32, hipStream_t s) {
-    VS_DISPATCH(tt, wt, shade_t, P, lw, stats, rb, waves, o32, s);
+                          int rb, int waves, int addr, hipStream_t s) {
+    VS_DISPATCH(tt, wt, shade_t, P, lw, stats, rb, waves, addr, s);
 }
 static LevelWork one_level(const WorkItem *work, int n, int level) {
     LevelWork lw{};
@@ -1502,17 +1496,17 @@ static LevelWork one_level(const WorkItem *work, int n, int level) {
     }
     return lw;
 }
-void launch_raycast(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt, bool o32,
+void launch_raycast(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt, int addr,
                     hipStream_t s) {
     const LevelWork lw = one_level(work, n, level);
-    launch_raycast_march(P, lw, tt, wt, nullptr, kRay8x8, o32, s);
-    launch_raycast_shade(P, lw, tt, wt, nullptr, kRay8x8, 4, o32, s);
+    launch_raycast_march(P, lw, tt, wt, nullptr, kRay8x8, addr, s);
+    launch_raycast_shade(P, lw, tt, wt, nullptr, kRay8x8, 4, addr, s);
 }
 void launch_raycast_stats(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt,
                           unsigned long long *stats, hipStream_t s) {
     const LevelWork lw = one_level(work, n, level);
-    launch_raycast_march(P, lw, tt, wt, stats, kRay8x8, false, s);
-    launch_raycast_shade(P, lw, tt, wt, stats, kRay32x2, 4, false, s);
+    launch_raycast_march(P, lw, tt, wt, stats, kRay8x8, kAddr64, s);
+    launch_raycast_shade(P, lw, tt, wt, stats, kRay32x2, 4, kAddr64, s);
 }
 
 static int grid_for(size_t n) {
