@@ -541,6 +541,13 @@ __device__ __forceinline__ bool below3(int x, int y, int z, int nx, int ny, int 
     return (int)((unsigned)x < (unsigned)nx) & (int)((unsigned)y < (unsigned)ny) & (int)((unsigned)z < (unsigned)nz);
 }
 
+// A voxel outside the grid on an axis along which the ray moves away or not
+// at all.
+__device__ __forceinline__ bool leaves3(int x, int y, int z, int nx, int ny, int nz, f3 rd) {
+    return (int)(x < 0 && !(rd.x > 0.0f)) | (int)(x >= nx && !(rd.x < 0.0f)) | (int)(y < 0 && !(rd.y > 0.0f)) |
+           (int)(y >= ny && !(rd.y < 0.0f)) | (int)(z < 0 && !(rd.z > 0.0f)) | (int)(z >= nz && !(rd.z < 0.0f));
+}
+
 // AD (VoxAddr): 32- or 64-bit record offsets, superbrick size known or read
 // from the session.
 template <class TV, class TW, int AD>
@@ -609,6 +616,10 @@ struct Vol {
         out = ok ? R::val(r) : 1.0f;
         return ok;
     }
+    // the record of voxel b * 512 + l
+    __device__ __forceinline__ typename VoxRec<TV, TW>::T rec_bl(unsigned b, unsigned l) const {
+        return O32 ? ld_rec32<TV, TW>(vx, (b << 9) | l) : ld_rec<TV, TW>(vx, (size_t)b * kBrickVox + l);
+    }
     // d_gtvu, exactly: nearest voxel by ROUNDF; true when it has weight.
     __device__ __forceinline__ bool nearest_valid(f3 v, float &out) const {
         int x, y, z;
@@ -638,10 +649,7 @@ struct Vol {
         const int y = v.y < 0.0f ? (int)(v.y - 0.5f) : (int)(v.y + 0.5f);
         const int z = v.z < 0.0f ? (int)(v.z - 0.5f) : (int)(v.z + 0.5f);
         if (!below3(x, y, z, P.vdim[0], P.vdim[1], P.vdim[2])) {
-            if ((int)(x < 0 && !(rd.x > 0.0f)) | (int)(x >= P.vdim[0] && !(rd.x < 0.0f)) |
-                (int)(y < 0 && !(rd.y > 0.0f)) | (int)(y >= P.vdim[1] && !(rd.y < 0.0f)) |
-                (int)(z < 0 && !(rd.z > 0.0f)) | (int)(z >= P.vdim[2] && !(rd.z < 0.0f)))
-                return -1;
+            if (leaves3(x, y, z, P.vdim[0], P.vdim[1], P.vdim[2], rd)) return -1;
             size = -1;
             return 0;
         }
@@ -769,10 +777,10 @@ constexpr float kSkipMargin = 0.25f;
 
 // rounded position inside [lo, lo + size)^3 clipped to the grid:
 // v in [lo - 0.5, hi + 0.5) on each axis
-__device__ __forceinline__ int steps_in_box(f3 v, f3 d, int3 lo, int size, const int *vdim) {
+__device__ __forceinline__ int steps_in_box(f3 v, f3 d, int3 lo, int size, int nx, int ny, int nz) {
     float k = (float)kSkipMax;
     const float vv[3] = {v.x, v.y, v.z}, dd[3] = {d.x, d.y, d.z};
-    const int ll[3] = {lo.x, lo.y, lo.z};
+    const int ll[3] = {lo.x, lo.y, lo.z}, vdim[3] = {nx, ny, nz};
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         const float hi = (float)min(ll[a] + size - 1, vdim[a] - 1);
@@ -785,9 +793,10 @@ __device__ __forceinline__ int steps_in_box(f3 v, f3 d, int3 lo, int size, const
 
 // rounded position outside the grid: it stays outside while any axis does
 // (below: v <= -0.5; above: v >= vdim - 0.5)
-__device__ __forceinline__ int steps_outside(f3 v, f3 d, const int *vdim) {
+__device__ __forceinline__ int steps_outside(f3 v, f3 d, int nx, int ny, int nz) {
     float k = 0.0f;
     const float vv[3] = {v.x, v.y, v.z}, dd[3] = {d.x, d.y, d.z};
+    const int vdim[3] = {nx, ny, nz};
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         const bool below = vv[a] <= -0.5f && dd[a] > 0.0f;
@@ -798,6 +807,29 @@ __device__ __forceinline__ int steps_outside(f3 v, f3 d, const int *vdim) {
     }
     k = fminf(k, (float)kSkipMax);
     return k >= 1.0f ? (int)k : 0;
+}
+
+// k steps of S along d = S * rd, k >= 0
+__device__ __forceinline__ void skip_steps(f3 &vox, float &total, int &iter, f3 d, float S, int k) {
+    iter += k;
+    int j = k;
+    for (; j >= 4; j -= 4) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            vox = add(vox, d);
+            total += S;
+        }
+    }
+    if (j & 2) {
+        vox = add(vox, d);
+        total += S;
+        vox = add(vox, d);
+        total += S;
+    }
+    if (j & 1) {
+        vox = add(vox, d);
+        total += S;
+    }
 }
 
 // Tap statistics of the instrumented march (the reference's lookups: what
@@ -884,29 +916,11 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW, AD> &V, const RayCons
             // inside it (tsdf is 1.0, so the next step is the same S each time)
             const float S = coarse ? C.step_scale : fmaxf(C.step_scale * tsdf, 1.0f);
             const f3 d = scale(S, rd);
-            const int k = size > 0 ? steps_in_box(vox, d, lo, size, V.P.vdim) : steps_outside(vox, d, V.P.vdim);
-            {  // k = 0 changes nothing
-                iter += k;
-                int j = k;
-                for (; j >= 4; j -= 4) {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        vox = add(vox, d);
-                        total += S;
-                    }
-                }
-                if (j & 2) {
-                    vox = add(vox, d);
-                    total += S;
-                    vox = add(vox, d);
-                    total += S;
-                }
-                if (j & 1) {
-                    vox = add(vox, d);
-                    total += S;
-                }
-                if ((int)(iter > C.max_iter) | (int)(total > C.total_max)) return false;
-            }
+            const int *n = V.P.vdim;
+            const int k = size > 0 ? steps_in_box(vox, d, lo, size, n[0], n[1], n[2])
+                                   : steps_outside(vox, d, n[0], n[1], n[2]);
+            skip_steps(vox, total, iter, d, S, k);
+            if ((int)(iter > C.max_iter) | (int)(total > C.total_max)) return false;
             continue;
         }
         if (fabsf(tsdf) < 1.0f) {
@@ -932,6 +946,147 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW, AD> &V, const RayCons
     step = C.step_scale * tsdf;
     vox = add(vox, scale(step, rd));
     hit = voxel_to_world(V.P, vox);
+    return true;
+}
+
+// The same march for launches that leave the chip mostly idle, where the time
+// is the longest ray's chain of iterations (~50 of them in a 640x480 frame,
+// whether 1575 or 75 workgroups run) and a wave has a SIMD nearly to itself.
+// cast_ray's iteration took ~1.3 us there: scalar loads of the session's sizes
+// waited for one after another in the loop (kept in memory there because
+// registers for them cost the full chip more than it gained), a nest of
+// branches, and up to three dependent rounds of loads. Here the sizes stay in
+// vector registers, the tests are flags, and one round loads the band word,
+// the nearest record and the eight trilinear corners together (the corners of
+// a stencil that leaves the grid read the nearest record and count as
+// failed). Decisions and values are cast_ray's: the same FP32 operations on
+// the same operands.
+template <class TV, class TW, int AD>
+__device__ __forceinline__ bool cast_ray_latency(const Vol<TV, TW, AD> &V, const RayConst &C, const float *Tcg,
+                                                 float px, float py, f3 &hit) {
+    typedef VoxRec<TV, TW> R;
+    const SessParams &P = V.P;
+    int nx = P.vdim[0], ny = P.vdim[1], nz = P.vdim[2];
+    unsigned bd0 = (unsigned)P.bdim[0], bd1 = (unsigned)P.bdim[1], sd0 = (unsigned)P.sdim[0],
+             sd1 = (unsigned)P.sdim[1];
+    int ss = V.super_log2();
+    // opaque: held in vector registers, not loaded again
+    asm volatile("" : "+v"(nx), "+v"(ny), "+v"(nz), "+v"(bd0), "+v"(bd1), "+v"(sd0), "+v"(sd1), "+v"(ss));
+    const uint32_t *bband = P.bband;
+    const unsigned bd01 = bd0 * bd1;
+    const float dist_min = C.dist_cc - C.r_cube, dist_max = C.dist_cc + C.r_cube;
+    const f3 pe = transform(Tcg, back_project(px, py, C.K, dist_max));
+    const f3 rd = normalised(sub(pe, C.cam));
+    if (dot(rd, C.ncc) < C.cos_max) return false;
+    const f3 ps = add(C.cam, scale(dist_min, rd));
+    f3 vox;
+    world_to_voxel(P, ps, vox);
+    float tsdf;
+    const bool valid = V.nearest_valid(vox, tsdf);
+    bool coarse = !valid;
+    if (valid && !(tsdf >= 0.0f)) return false;
+    float total = 0.0f;
+    int iter = 0;
+    unsigned sv_x = 0xFFFFFFFFu, sv_y = 0xFFFFFFFFu, sv_z = 0xFFFFFFFFu, sv_t = 0xFFFFFFFFu, brent = 0;
+    enum { kRun, kMiss, kBehind, kHit };
+    int state = kRun;
+    do {
+        // cycle detection on the fine-search state, as in cast_ray
+        const unsigned bx = __float_as_uint(vox.x), by = __float_as_uint(vox.y), bz = __float_as_uint(vox.z),
+                       bt = __float_as_uint(tsdf);
+        bool miss = (int)!coarse & (int)(((bx ^ sv_x) | (by ^ sv_y) | (bz ^ sv_z) | (bt ^ sv_t)) == 0u);
+        const bool save = (int)!coarse & (int)((brent & 0xFFFFu) == (1u << (brent >> 16)));
+        sv_x = save ? bx : sv_x;
+        sv_y = save ? by : sv_y;
+        sv_z = save ? bz : sv_z;
+        sv_t = save ? bt : sv_t;
+        brent = (save ? ((brent >> 16) + 1) << 16 : brent) + (coarse ? 0u : 1u);
+        ++iter;
+        const float sm = fmaxf(fabsf(C.step_scale * tsdf), 1.0f);
+        const float step = coarse ? C.step_scale : (tsdf > 0.0f ? sm : -sm);
+        vox = add(vox, scale(step, rd));
+        total += step;
+        const bool fin = finite3(vox);
+        const f3 v = {fin ? vox.x : 0.0f, fin ? vox.y : 0.0f, fin ? vox.z : 0.0f};
+        const int x = v.x < 0.0f ? (int)(v.x - 0.5f) : (int)(v.x + 0.5f);  // ROUNDF
+        const int y = v.y < 0.0f ? (int)(v.y - 0.5f) : (int)(v.y + 0.5f);
+        const int z = v.z < 0.0f ? (int)(v.z - 0.5f) : (int)(v.z + 0.5f);
+        const bool in = (int)fin & (int)below3(x, y, z, nx, ny, nz);
+        miss = (int)miss | (int)(iter > C.max_iter) | (int)(total > C.total_max) |
+               ((int)fin & (int)!in & (int)leaves3(x, y, z, nx, ny, nz, rd));
+        const unsigned sb = __umul24(__umul24((unsigned)(z >> ss), sd1) + (unsigned)(y >> ss), sd0) + (unsigned)(x >> ss);
+        const int d = (V.sdist[(sb >> 1) & (kDistCells / 2 - 1)] >> ((sb & 1u) * 4u)) & 15u;
+        tsdf = 1.0f;
+        bool near = false, band = false;
+        if ((int)in & (int)(d == 0) & (int)!miss) {
+            const unsigned b = __umul24(__umul24((unsigned)z >> 3, bd1) + ((unsigned)y >> 3), bd0) + ((unsigned)x >> 3);
+            const unsigned l = (unsigned)(((z & 7) << 6) | ((y & 7) << 3) | (x & 7));
+            const int ox = (int)v.x, oy = (int)v.y, oz = (int)v.z;
+            const bool inner = below3(ox, oy, oz, nx - 1, ny - 1, nz - 1);
+            unsigned Bx[2], By[2], Bz[2], Lx[2], Ly[2], Lz[2];
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                Bx[a] = (unsigned)(ox + a) >> 3;
+                By[a] = __umul24((unsigned)(oy + a) >> 3, bd0);
+                Bz[a] = __umul24((unsigned)(oz + a) >> 3, bd01);
+                Lx[a] = (unsigned)(ox + a) & 7u;
+                Ly[a] = ((unsigned)(oy + a) & 7u) << 3;
+                Lz[a] = ((unsigned)(oz + a) & 7u) << 6;
+            }
+            const uint32_t word = ldg(bband, b >> 5);
+            const typename R::T rn = V.rec_bl(b, l);
+            typename R::T rc[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const unsigned cb = Bz[k >> 2] + By[(k >> 1) & 1] + Bx[k & 1];
+                const unsigned cl = Lz[k >> 2] | Ly[(k >> 1) & 1] | Lx[k & 1];
+                rc[k] = V.rec_bl(inner ? cb : b, inner ? cl : l);
+            }
+            band = (word >> (b & 31)) & 1u;
+            const float tn = R::has_w(rn) ? R::val(rn) : 1.0f;
+            near = (int)band & (int)(fabsf(tn) < 1.0f);
+            float f[8];
+            bool ok = inner;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                ok = (int)ok & (int)R::has_w(rc[k]);
+                f[k] = R::val(rc[k]);
+            }
+            const float rx = v.x - (float)ox, ry = v.y - (float)oy, rz = v.z - (float)oz;
+            const float fi = (1.0f - ry) * ((1.0f - rx) * f[0] + rx * f[1]) + ry * ((1.0f - rx) * f[2] + rx * f[3]);
+            const float bi = (1.0f - ry) * ((1.0f - rx) * f[4] + rx * f[5]) + ry * ((1.0f - rx) * f[6] + rx * f[7]);
+            const float tt = ok ? (1.0f - rz) * fi + rz * bi : 1.0f;
+            tsdf = band ? (near ? tt : tn) : 1.0f;
+        }
+        // 1.0 here and in the box around (the brick, the superbricks of the
+        // field, or the space before the grid): skip the steps inside it
+        if ((int)fin & (int)!band & (int)!miss) {
+            const float S = coarse ? C.step_scale : fmaxf(C.step_scale * 1.0f, 1.0f);
+            const f3 dv = scale(S, rd);
+            int k;
+            if (in) {
+                const int sh = d == 0 ? 3 : ss, r = max(d - 1, 0), unit = 1 << sh;
+                const int3 lo = make_int3(((x >> sh) - r) * unit, ((y >> sh) - r) * unit, ((z >> sh) - r) * unit);
+                k = steps_in_box(vox, dv, lo, (2 * r + 1) * unit, nx, ny, nz);
+            } else {
+                k = steps_outside(vox, dv, nx, ny, nz);
+            }
+            skip_steps(vox, total, iter, dv, S, k);
+            miss = (int)(iter > C.max_iter) | (int)(total > C.total_max);
+        }
+        const bool neg = (int)near & (int)(tsdf < 0.0f);
+        state = miss || (neg && coarse) ? kMiss : neg ? kBehind : (near && tsdf == 0.0f) ? kHit : kRun;
+        coarse = (int)coarse & (int)!near;
+    } while (state == kRun);
+    if (state == kMiss) return false;
+    if (state == kBehind) {
+        float step = C.step_scale * tsdf;
+        vox = add(vox, scale(step, rd));
+        V.trilinear(vox, tsdf);
+        step = C.step_scale * tsdf;
+        vox = add(vox, scale(step, rd));
+    }
+    hit = voxel_to_world(P, vox);
     return true;
 }
 
@@ -1077,10 +1232,10 @@ __device__ __forceinline__ void ray_pixel(int t, int &px, int &py) {
 // taps, and the extra waves hide the taps' latency better than the few
 // registers the compiler would add beyond 64.
 // AD: VoxAddr of the launch.
-template <class TV, class TW, bool STATS, int RB, int AD>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_raycast(
+template <class TV, class TW, bool STATS, int RB, int AD, bool LAT>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(LAT ? 4 : 8, 8))) void k_raycast(
     const SessParams *__restrict__ SP, LevelWork lw, unsigned long long *stats) {
-    __shared__ uint32_t s_dist[kDistCells / 8];
+    __shared__ __align__(16) uint32_t s_dist[kDistCells / 8];
     int level;
     const WorkItem wi = level_item(lw, level);
     const SessParams &P = SP[wi.sess];
@@ -1088,8 +1243,24 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
     const LevelDesc &L = P.lev[level];
     if (!st->fuse_ok || level >= P.levels || tile_out(L, wi.tile)) return;
     const int ncell = P.sdim[0] * P.sdim[1] * P.sdim[2];
-    const uint32_t *src = (const uint32_t *)P.sdist;
-    for (int i = threadIdx.x; i < (ncell + 7) / 8; i += kTileThreads) s_dist[i] = ldg(src, i);
+    // four 16-byte loads per thread, issued together (the field's buffer is
+    // padded to 256 bytes)
+    {
+        constexpr int kLoads = kDistCells / 32 / kTileThreads;
+        const vs_u4 *src = (const vs_u4 *)P.sdist;
+        const int nq = (ncell + 31) / 32;
+        vs_u4 q[kLoads];
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k) {
+            const int i = threadIdx.x + k * kTileThreads;
+            if (i < nq) q[k] = ldg(src, i);
+        }
+#pragma unroll
+        for (int k = 0; k < kLoads; ++k) {
+            const int i = threadIdx.x + k * kTileThreads;
+            if (i < nq) ((vs_u4 *)s_dist)[i] = q[k];
+        }
+    }
     __syncthreads();
     int px, py;
     ray_pixel<RB>(threadIdx.x, px, py);
@@ -1111,7 +1282,8 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8,
     RayStats rs;
     f3 p;
     const M34 Tc = ld_m34(st->T_cg_f);
-    const bool ok = cast_ray<TV, TW, STATS, AD>(V, C, Tc.m, (float)x, (float)y, p, rs);
+    const bool ok = LAT ? cast_ray_latency<TV, TW, AD>(V, C, Tc.m, (float)x, (float)y, p)
+                        : cast_ray<TV, TW, STATS, AD>(V, C, Tc.m, (float)x, (float)y, p, rs);
     const size_t t = (size_t)y * L.W + x;
     if (ok) {
         st_mvtx(P.mvn[level], t, p.x, p.y, p.z);  // world hit; the shading makes it the camera-frame vertex
@@ -1416,13 +1588,23 @@ void launch_integrate(const SessParams *P, int nsess, BrickList bl, int tt, int 
     launch_sdist(P, nsess, sd_slices, 0, s);
 }
 
+// Launches of up to this many workgroups (the 8 per CU that are resident at
+// once on 256 CUs) take the latency form of the march. Fused frame with a
+// 1200-workgroup preview: 1575 workgroups at 640x480 / 256^3, 532 us in the
+// wide form, 509 in the latency form; 1443 at 603x451 in colour, 615 / 550;
+// three levels of 1260, 300 and 75 workgroups (264x200x312), 155 / 117. Above
+// it the waves' own number hides their latency: 6300 and 4800 workgroups at
+// 1280x960 / 1024^3, 1177 / 1225.
+constexpr int kLatencyGroups = 2048;
 template <class TV, class TW>
 static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int addr,
                     hipStream_t s) {
     const int n = lw.blocks();
     if (n <= 0) return;
 #define VS_MARCH_A(RB_, AD_) \
-    hipLaunchKernelGGL((k_raycast<TV, TW, false, RB_, AD_>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats)
+    hipLaunchKernelGGL((k_raycast<TV, TW, false, RB_, AD_, false>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats)
+#define VS_MARCH_L(AD_) \
+    hipLaunchKernelGGL((k_raycast<TV, TW, false, kRay8x8, AD_, true>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats)
 #define VS_MARCH(RB_)                                        \
     do {                                                     \
         if (addr == kAddrSmall) VS_MARCH_A(RB_, kAddrSmall); \
@@ -1430,8 +1612,11 @@ static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long
         else VS_MARCH_A(RB_, kAddr64);                       \
     } while (0)
     if (stats)
-        hipLaunchKernelGGL((k_raycast<TV, TW, true, kRay8x8, kAddr64>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats);
-    else if (rb == kRay16x4)
+        hipLaunchKernelGGL((k_raycast<TV, TW, true, kRay8x8, kAddr64, false>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats);
+    else if (n <= kLatencyGroups) {
+        if (addr != kAddr64) VS_MARCH_L(kAddr32);
+        else VS_MARCH_L(kAddr64);
+    } else if (rb == kRay16x4)
         VS_MARCH(kRay16x4);
     else if (rb == kRay32x2)
         VS_MARCH(kRay32x2);
@@ -1439,6 +1624,7 @@ static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long
         VS_MARCH(kRay8x8);
 #undef VS_MARCH
 #undef VS_MARCH_A
+#undef VS_MARCH_L
 }
 template <class TV, class TW>
 static void shade_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int waves,
