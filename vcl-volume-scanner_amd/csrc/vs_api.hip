@@ -1337,6 +1337,11 @@ vs_status vs_session_destroy(vs_session *s) {
         return VS_OK;
     }
     (void)sync_last(s);
+    // a batched step without a caller's stream runs on its first session's
+    // stream, which the other sessions then hold as their last one: that
+    // work has just completed, and the handle ends here
+    for (vs_session *o : s->ctx->sessions)
+        if (o != s && o->last == s->stream) o->last = o->stream;
     drop_batches_with(s->ctx, s);
     free_batch_graph(s->self);
     s->timer.destroy();
