@@ -62,7 +62,7 @@ def _run(cmd):
 # libvscan.so, or the file VSCAN_LIB names):
 #   icp_lds: the ICP iteration's block sums as per-thread FP32 FMAs and LDS
 #            chunk sums instead of on the matrix cores (VS_ICP_MFMA=0)
-VARIANTS = {"icp_lds": ["-DVS_ICP_MFMA=0"]}
+VARIANTS = {"icp_lds": ["-DVS_ICP_MFMA=0", "-DVS_ICP_STEP_GROUPS=0"]}
 
 
 def build(verbose=False, variant=None):

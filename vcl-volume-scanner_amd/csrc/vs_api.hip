@@ -74,7 +74,7 @@ struct Layout {
     size_t total;
     size_t nvox;
     uint32_t nbricks, nwords, nsuper, nswords;
-    int sdim[3], sshift;
+    int sdim[3], sshift, icp_half;
     int tiles[kMaxLevels];
 };
 
@@ -132,7 +132,9 @@ Layout make_layout(const vs_session_desc &d) {
     L.sband = take((size_t)L.nswords * 4);
     L.sdist = take(((size_t)L.nsuper + 7) / 8 * 4);  // 4 bits per superbrick, whole words
     L.sdtmp = take(L.nsuper);
-    L.icp_part = take((size_t)L.tiles[0] * kIcpVals * 8);
+    L.icp_half = 0;
+    for (int l = 0; l < kMaxLevels; ++l) L.icp_half = std::max(L.icp_half, icp_groups(L.tiles[l], l) * kIcpVals);
+    L.icp_part = take((size_t)L.icp_half * 2 * 8);
     L.diag_part = take((size_t)L.tiles[0] * kIcpVals * 8);
     L.diag_mask = take((size_t)W * H);
     {
@@ -715,6 +717,23 @@ hipStream_t pick(vs_session *s, vs_stream st) {
     return h;
 }
 
+// The Gauss-Newton iterations of a batch, coarse to fine, and the pose update.
+void enqueue_track(const Batch &B, hipStream_t s) {
+    const bool one = B.nGroup[0] <= kIcpStepGroups;  // one launch per iteration
+    int seq = 0;
+    for (int l = B.levels - 1; l >= 0; --l)
+        for (int it = 0; it < B.max_iters[l]; ++it) {
+            if (one)
+                launch_icp_step(B.dP, B.dGroup[l], B.nGroup[l], l, it, ++seq, s);
+            else
+                launch_icp_iter(B.dP, B.dGroup[l], B.nGroup[l], B.n, l, it, s);
+        }
+    if (one)
+        launch_icp_finish(B.dP, B.n, s);
+    else
+        launch_track_finalize(B.dP, B.n, s);
+}
+
 // The per-frame launch sequence of a batch (so_Scan_Object order).
 void enqueue_step(const Batch &B, hipStream_t s, Timer *timed) {
     auto mark = [&](int i) {
@@ -729,9 +748,7 @@ void enqueue_step(const Batch &B, hipStream_t s, Timer *timed) {
     mark(1);
     for (int l = 1; l < B.levels; ++l) launch_pyr_down(B.dP, B.dWork[l], B.nWork[l], l, s);
     mark(2);
-    for (int l = B.levels - 1; l >= 0; --l)
-        for (int it = 0; it < B.max_iters[l]; ++it) launch_icp_iter(B.dP, B.dGroup[l], B.nGroup[l], B.n, l, it, s);
-    launch_track_finalize(B.dP, B.n, s);
+    enqueue_track(B, s);
     mark(3);
     launch_vis_clear(B.dP, B.n, B.bl, s);
     launch_vis_mark(B.dP, B.dWork[0], B.nWork[0], B.n, B.max_words, B.bl, s);
@@ -1237,6 +1254,7 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
     P.sshift = L.sshift;
     P.sband_words = (int)L.nswords;
     P.icp_part = (double *)(m + L.icp_part);
+    P.icp_half = L.icp_half;
     {
         float *wt = (float *)(m + L.wtab);
         P.wtab[0] = wt;
@@ -1491,9 +1509,7 @@ vs_status vs_track(vs_session *s, const double *T_01_init, vs_stream stream) {
     hipStream_t h = pick(s, stream);
     const Batch &B = s->self;
     launch_track_setup_forced(B.dP, 1, T_01_init, h);
-    for (int l = B.levels - 1; l >= 0; --l)
-        for (int it = 0; it < B.max_iters[l]; ++it) launch_icp_iter(B.dP, B.dGroup[l], B.nGroup[l], B.n, l, it, h);
-    launch_track_finalize(B.dP, 1, h);
+    enqueue_track(B, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }

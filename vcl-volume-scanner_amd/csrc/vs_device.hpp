@@ -69,12 +69,25 @@ struct LevelDesc {
     float K[4];  // fx, fy, cx, cy
 };
 
+// Where a session's Gauss-Newton loop stands after a launch of the one-launch
+// form of an iteration (k_icp_step): two records used in turn, the later one
+// (by seq) is current. Its group partials, not yet solved when pending >= 0,
+// are in the half of icp_part with the record's index.
+struct IcpStep {
+    double T_12[16];
+    int seq;         // launch that wrote the record (0: track setup, -1: never)
+    int pending;     // level of the unsolved partials, -1 none
+    int failed, conv_level, solves;
+    int pad[3];
+};
+
 // Mutable per-session state; lives in HBM, touched only by kernels.
 struct alignas(16) SessState {
     double T_gc[16];   // FP64 master pose (world -> camera)
     double T_cg[16];
     double T_12[16];   // tracker increment camera t0 -> t1
     double T_21[16];
+    IcpStep step[2];
     float T_gc_f[16];  // FP32 copies the kernels consume
     float T_cg_f[16];
     float T_21_f[16];
@@ -151,7 +164,8 @@ struct alignas(16) SessParams {
     int sdim[3];             // superbricks per axis
     int sshift;              // log2(bricks per superbrick edge)
     int sband_words;         // 32-bit words of sband
-    double *icp_part;        // ICP group partials (kIcpVals per group of level-0 tiles)
+    double *icp_part;        // ICP group partials (kIcpVals per group), two halves of icp_half doubles
+    int icp_half;
     // World coordinate of each voxel centre along each axis, the reference's
     // FP32 expression ((float)i + 0.5f) / vox_inv + origin[a] (d_gpw,
     // _yooji_cuda_math.h:285-302), evaluated once per session: wtab[a][i]

@@ -33,6 +33,22 @@ __device__ void matmul4d(const double *A, const double *B, double *C) {
         }
     for (int k = 0; k < 16; ++k) C[k] = t[k];
 }
+// C = A B for an A whose last row is (0, 0, 0, 1).
+__device__ __forceinline__ void affine_matmul(const double *A, const double *B, double *C) {
+    double t[12];
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            double s = A[r * 4] * B[c];
+            for (int k = 1; k < 4; ++k) s = fma(A[r * 4 + k], B[k * 4 + c], s);
+            t[r * 4 + c] = s;
+        }
+#pragma unroll
+    for (int k = 0; k < 12; ++k) C[k] = t[k];
+#pragma unroll
+    for (int k = 12; k < 16; ++k) C[k] = B[k];
+}
 // Inverse of a rigid transform: [R^T, -R^T t]. Equals the reference's general
 // 4x4 inverse (d_im_Inverse_Matrix_4x4, _yooji_math_inlines.h:404-465) on
 // rigid inputs.
@@ -49,15 +65,32 @@ __device__ void rigid_inverse(const double *T, double *Ti) {
 // SE(3) exponential of x = [w; v] (the twist update of
 // z_uitme_Update_Incremental_Tracking_with_Matrix_Exponential, pose_tracker.cu:50-149),
 // with a series branch for small |w| (the reference divides by |w|).
+// Coefficients of th^2k in sin(th) / th, (1 - cos(th)) / th^2 and
+// (th - sin(th)) / th^3: (-1)^k / (2k + 1)!, / (2k + 2)!, / (2k + 3)!.
+constexpr double kExpA[8] = {1.0, -1.0 / 6, 1.0 / 120, -1.0 / 5040, 1.0 / 362880, -1.0 / 39916800, 1.0 / 6227020800.0,
+                             -1.0 / 1307674368000.0};
+constexpr double kExpB[8] = {1.0 / 2, -1.0 / 24, 1.0 / 720, -1.0 / 40320, 1.0 / 3628800, -1.0 / 479001600,
+                             1.0 / 87178291200.0, -1.0 / 20922789888000.0};
+constexpr double kExpC[8] = {1.0 / 6, -1.0 / 120, 1.0 / 5040, -1.0 / 362880, 1.0 / 39916800, -1.0 / 6227020800.0,
+                             1.0 / 1307674368000.0, -1.0 / 355687428096000.0};
 __device__ void expmap(const double *x, double *T) {
     const double w0 = x[0], w1 = x[1], w2 = x[2];
-    const double th2 = w0 * w0 + w1 * w1 + w2 * w2, th = sqrt(th2);
+    const double th2 = w0 * w0 + w1 * w1 + w2 * w2;
     double A, B, C;
-    if (th < 1e-4) {
-        A = 1.0 - th2 / 6.0 + th2 * th2 / 120.0;
-        B = 0.5 - th2 / 24.0 + th2 * th2 / 720.0;
-        C = 1.0 / 6.0 - th2 / 120.0 + th2 * th2 / 5040.0;
+    if (th2 < 0.25) {
+        // series in th^2 to beyond double precision (0.25^8 / 17! < 1e-19);
+        // free of the cancellation in 1 - cos and th - sin, and a third of
+        // the instructions of a sine and a cosine
+        A = B = C = 0.0;
+#pragma unroll
+        for (int k = 7; k >= 0; --k) {
+            const double a = kExpA[k], b = kExpB[k], c = kExpC[k];
+            A = fma(A, th2, a);
+            B = fma(B, th2, b);
+            C = fma(C, th2, c);
+        }
     } else {
+        const double th = sqrt(th2);
         A = sin(th) / th;
         B = (1.0 - cos(th)) / th2;
         C = (th - sin(th)) / (th2 * th);
@@ -78,49 +111,60 @@ __device__ void expmap(const double *x, double *T) {
     T[12] = T[13] = T[14] = 0.0;
     T[15] = 1.0;
 }
-// Cholesky and triangular solves with the reference's pivot rule
-// (d_lld_LL_Decomposition / d_sls_Solve_Linear_System_using_LLD,
-// _yooji_cuda_math.h:489-592): entries below a pivot < 1e-8 are zeroed and the
-// solve fails (status 4) if any pivot is below 1e-8 (or not a number). With
+// The 6x6 solve with the reference's pivot rule (d_lld_LL_Decomposition /
+// d_sls_Solve_Linear_System_using_LLD, _yooji_cuda_math.h:489-592): it fails
+// (status 4) if any Cholesky pivot L_jj is below 1e-8 (or not a number). With
 // rel > 0 it also fails (status 8) when a squared pivot L_jj^2 is below
 // rel * A_jj: column j of J is then nearly a combination of the columns
 // before it (a plane leaves 3 of the 6 motions unconstrained), a near-rank
 // deficiency the absolute test cannot see at FP32 scales. The ratio is
 // invariant to the units of the rotation and translation columns.
-// Column by column, each below-diagonal entry and substitution step scaled by
-// the column's reciprocal pivot (6 FP64 divisions instead of 33 on the
-// solve's one-lane chain; the same sums in the same order).
-// Returns 0 on success.
-__device__ int cholesky_solve(const double *A, const double *b, double rel, double *x) {
-    double L[36], inv[6];
-    for (int k = 0; k < 36; ++k) L[k] = 0.0;
+// Factored as L D L^T, D_j = L_jj^2: the chain of one lane then holds one
+// reciprocal per pivot (two Newton steps on the hardware estimate, to the
+// last bit or two of FP64) where the square-root form had a square root and a
+// division. A is the upper triangle row by row (21 values). Returns 0 on
+// success.
+__device__ __forceinline__ int solve6(const double *A, const double *b, double rel, double *x) {
+    double u[6][6], l[6][6], r[6];  // u = l D below the diagonal
+    bool ok = true, weak = false;
+    int k0 = 0;
+#pragma unroll
     for (int j = 0; j < 6; ++j) {
-        double s = 0.0;
-        for (int k = 0; k < j; ++k) s += L[j * 6 + k] * L[j * 6 + k];
-        L[j * 6 + j] = sqrt(A[j * 6 + j] - s);
-        inv[j] = 1.0 / L[j * 6 + j];
-        const bool piv = fabs(L[j * 6 + j]) >= 1e-8;
+        double d = A[k0];
+#pragma unroll
+        for (int k = 0; k < j; ++k) d = fma(-u[j][k], l[j][k], d);
+        ok &= d >= 1.0e-16;
+        weak |= d < rel * A[k0];
+        double q = __builtin_amdgcn_rcp(d);
+        q = fma(q, fma(-d, q, 1.0), q);
+        q = fma(q, fma(-d, q, 1.0), q);
+        r[j] = d < 1.0e300 ? q : 0.0;
+#pragma unroll
         for (int i = j + 1; i < 6; ++i) {
-            double t = 0.0;
-            for (int k = 0; k < j; ++k) t += L[i * 6 + k] * L[j * 6 + k];
-            L[i * 6 + j] = piv ? (A[i * 6 + j] - t) * inv[j] : 0.0;
+            double t = A[k0 + i - j];
+#pragma unroll
+            for (int k = 0; k < j; ++k) t = fma(-u[i][k], l[j][k], t);
+            u[i][j] = t;
+            l[i][j] = t * r[j];
         }
+        k0 += 6 - j;
     }
-    for (int i = 0; i < 6; ++i)
-        if (!(fabs(L[i * 6 + i]) >= 1e-8)) return 4;
-    if (rel > 0.0)
-        for (int i = 0; i < 6; ++i)
-            if (L[i * 6 + i] * L[i * 6 + i] < rel * A[i * 6 + i]) return 8;
+    if (!ok) return 4;
+    if (rel > 0.0 && weak) return 8;
     double y[6];
+#pragma unroll
     for (int i = 0; i < 6; ++i) {
-        double s = 0.0;
-        for (int k = 0; k < i; ++k) s += L[i * 6 + k] * y[k];
-        y[i] = (b[i] - s) * inv[i];
+        double t = b[i];
+#pragma unroll
+        for (int k = 0; k < i; ++k) t = fma(-l[i][k], y[k], t);
+        y[i] = t;
     }
+#pragma unroll
     for (int i = 5; i >= 0; --i) {
-        double s = 0.0;
-        for (int k = i + 1; k < 6; ++k) s += L[k * 6 + i] * x[k];
-        x[i] = (y[i] - s) * inv[i];
+        double t = y[i] * r[i];
+#pragma unroll
+        for (int k = 5; k > i; --k) t = fma(-l[k][i], x[k], t);
+        x[i] = t;
     }
     return 0;
 }
@@ -332,48 +376,37 @@ __device__ __forceinline__ bool icp_skip(const SessParams &P, const SessState *s
            iter >= P.iters[level] || (ldg(&st->force_single, 0) && level != 0);
 }
 
-// One Gauss-Newton iteration at `level`, first half: the 29 sums of every
-// group of G = icp_group(level) consecutive 32x8 tiles of every session of the work
-// list (items are (session, group)), one FP64 partial per group, summed on
-// the matrix cores (above) or, with VS_ICP_MFMA=0, by per-thread FP32
-// accumulation over the group's tiles and one block reduction (block_terms).
-// No cross-workgroup synchronisation here: on a
-// multi-XCD device an agent-scope release per workgroup would write back L2
-// each time, so the reduction and the solve are the next launch
-// (k_icp_solve).
+// The group's depths (independent loads; a pixel outside the frame re-reads
+// pixel 0 and is skipped).
 template <int G>
-__global__ __launch_bounds__(kTileThreads) void k_icp_iter(const SessParams *__restrict__ SP,
-                                                           const WorkItem *__restrict__ work, int level, int iter) {
-    __shared__ float T21s[16];
-    __shared__ double red64[kIcpVals];
-    const WorkItem wi = work[blockIdx.x];
-    const SessParams &P = SP[wi.sess];
-    const SessState *st = P.st;
-    if (level >= P.levels || icp_skip(P, st, level, iter)) return;
-    const LevelDesc &L = P.lev[level];
-    const int ntiles = L.tiles_x * L.tiles_y;
-    const int t0 = wi.tile * G;
-    if (t0 >= ntiles) return;
-    if (threadIdx.x < 16) T21s[threadIdx.x] = ldg(st->T_21_f, threadIdx.x);
-    __syncthreads();
-#if !VS_ICP_MFMA
-    float acc[kIcpVals];
-#pragma unroll
-    for (int k = 0; k < kIcpVals; ++k) acc[k] = 0.0f;
-#endif
-    // the group's depths first (independent loads; a pixel outside the
-    // frame re-reads pixel 0 and is skipped), then the pixels in order
+struct GroupPixels {
     int xs[G], ys[G];
     bool in[G];
     float td[G];
+    __device__ __forceinline__ void load(const SessParams &P, int level, int t0) {
+        const LevelDesc &L = P.lev[level];
+        const int ntiles = L.tiles_x * L.tiles_y;
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const int tile = t0 + g;
-        xs[g] = (tile % L.tiles_x) * kTileW + threadIdx.x % kTileW;
-        ys[g] = (tile / L.tiles_x) * kTileH + threadIdx.x / kTileW;
-        in[g] = tile < ntiles && xs[g] < L.W && ys[g] < L.H;
-        td[g] = ldg(P.filt[level], in[g] ? (size_t)ys[g] * L.W + xs[g] : (size_t)0);
+        for (int g = 0; g < G; ++g) {
+            const int tile = t0 + g;
+            xs[g] = (tile % L.tiles_x) * kTileW + threadIdx.x % kTileW;
+            ys[g] = (tile / L.tiles_x) * kTileH + threadIdx.x / kTileW;
+            in[g] = tile < ntiles && xs[g] < L.W && ys[g] < L.H;
+            td[g] = ldg(P.filt[level], in[g] ? (size_t)ys[g] * L.W + xs[g] : (size_t)0);
+        }
     }
+};
+
+// The 29 sums of one group (G = icp_group(level) consecutive 32x8 tiles) at
+// the pose T21s (LDS), one FP64 partial into out, summed on the matrix cores
+// (above) or, with VS_ICP_MFMA=0, by per-thread FP32 accumulation over the
+// group's tiles and one block reduction (block_terms).
+template <int G>
+__device__ __forceinline__ void group_sums(const SessParams &P, int level, const GroupPixels<G> &px_, const float *T21s,
+                                           double *out) {
+    const int *xs = px_.xs, *ys = px_.ys;
+    const bool *in = px_.in;
+    const float *td = px_.td;
 #if VS_ICP_MFMA
     __shared__ float feat[kTileThreads / 64][64][8];
     __shared__ float gw[kTileThreads / 64][8][8];
@@ -422,9 +455,13 @@ __global__ __launch_bounds__(kTileThreads) void k_icp_iter(const SessParams *__r
         double s = 0.0;
 #pragma unroll
         for (int w = 0; w < kTileThreads / 64; ++w) s += (double)gw[w][i][j];
-        stg(P.icp_part, (size_t)wi.tile * kIcpVals + threadIdx.x, s);
+        stg(out, threadIdx.x, s);
     }
 #else
+    __shared__ double red64[kIcpVals];
+    float acc[kIcpVals];
+#pragma unroll
+    for (int k = 0; k < kIcpVals; ++k) acc[k] = 0.0f;
 #pragma unroll
     for (int g = 0; g < G; ++g) {
         if (in[g]) {
@@ -434,97 +471,305 @@ __global__ __launch_bounds__(kTileThreads) void k_icp_iter(const SessParams *__r
         }
     }
     block_terms(acc, red64);
-    if (threadIdx.x < kIcpVals) stg(P.icp_part, (size_t)wi.tile * kIcpVals + threadIdx.x, red64[threadIdx.x]);
+    if (threadIdx.x < kIcpVals) stg(out, threadIdx.x, red64[threadIdx.x]);
 #endif
 }
 
-// Second half: one wave per session sums the group partials in FP64 in a
-// fixed order, solves the 6x6 system and applies the SE(3) update. Lane t
-// adds groups t, t + 64, ...; then the 29 sums (padded to 32) are reduced
-// across the wave by recursive halving: at each of five exchanges a lane
-// sends half of the sums it still holds to its partner (lane ^ 32, ^ 16, ...,
-// ^ 2) and adds the partner's half of its own, so 16 + 8 + 4 + 2 + 1 values
-// cross lanes instead of 29 x 6 for 29 separate butterflies; a last exchange
-// with lane ^ 1 completes sum v = lane / 2, and lane 0 reads the 29 totals
-// with readlane. The order is fixed, so the result does not depend on the
-// batch or the schedule. (A 256-thread block with a butterfly per sum spent
-// about twice as long in this part.)
-constexpr int kSolveThreads = 64;
-__global__ __launch_bounds__(kSolveThreads) void k_icp_solve(const SessParams *__restrict__ SP, int nsess, int level,
-                                                             int iter) {
+// One Gauss-Newton iteration at `level`, first half of the two-launch form:
+// the partial of every group of every session of the work list (items are
+// (session, group)). No cross-workgroup synchronisation here: on a
+// multi-XCD device an agent-scope release per workgroup would write back L2
+// each time, so the reduction and the solve are the next launch
+// (k_icp_solve).
+template <int G>
+__global__ __launch_bounds__(kTileThreads) void k_icp_iter(const SessParams *__restrict__ SP,
+                                                           const WorkItem *__restrict__ work, int level, int iter) {
+    __shared__ float T21s[16];
+    const WorkItem wi = work[blockIdx.x];
+    const SessParams &P = SP[wi.sess];
+    const SessState *st = P.st;
+    if (level >= P.levels || icp_skip(P, st, level, iter)) return;
+    const LevelDesc &L = P.lev[level];
+    const int t0 = wi.tile * G;
+    if (t0 >= L.tiles_x * L.tiles_y) return;
+    if (threadIdx.x < 16) T21s[threadIdx.x] = ldg(st->T_21_f, threadIdx.x);
+    __syncthreads();
+    GroupPixels<G> px;
+    px.load(P, level, t0);
+    group_sums<G>(P, level, px, T21s, P.icp_part + (size_t)wi.tile * kIcpVals);
+}
+
+// The 29 totals of ng group partials in FP64, in a fixed order that depends
+// on the group count alone: thread (chunk c, term k) adds groups c, c + 32,
+// ..., then the 32 chunk sums of a term are added as a fixed tree. Neighbouring
+// threads read neighbouring terms, so a load covers whole lines, and a
+// 640x480 frame's 150 groups are one round of loads. (One wave with a group
+// per lane read 64 lines per load.) Result in tot (LDS), visible to the first
+// wave only.
+constexpr int kSumChunks = 32;
+template <int THREADS>
+__device__ __forceinline__ void sum_partials(const double *part, int ng, double (*chunk)[kIcpVals], double *tot) {
+    constexpr int U = 5, kPairs = kSumChunks * kIcpVals;
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int p0 = 0; p0 < kPairs; p0 += THREADS) {
+        const int p = p0 + t, c = p / kIcpVals, k = p - c * kIcpVals;
+        if (p < kPairs) {
+            double s = 0.0;
+            for (int g = c; g < ng; g += U * kSumChunks) {
+                double v[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) v[u] = ldg(part, (size_t)min(g + u * kSumChunks, ng - 1) * kIcpVals + k);
+#pragma unroll
+                for (int u = 0; u < U; ++u) s = g + u * kSumChunks < ng ? s + v[u] : s;
+            }
+            chunk[c][k] = s;
+        }
+    }
+    __syncthreads();
+    if (t < kIcpVals) {
+        double v[kSumChunks];
+#pragma unroll
+        for (int q = 0; q < kSumChunks; ++q) v[q] = chunk[q][t];
+#pragma unroll
+        for (int h = kSumChunks / 2; h >= 1; h >>= 1)
+#pragma unroll
+            for (int q = 0; q < h; ++q) v[q] += v[q + h];
+        tot[t] = v[0];
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One solve and SE(3) update from the 29 totals (one thread). Returns 0 when
+// T12 was updated, 1 when the step was below the convergence bound, else the
+// failure's status in `failed`.
+struct SolveResult {
+    bool updated, converged;
+    int failed;
+};
+__device__ __forceinline__ SolveResult solve_totals(const SessParams &P, const double *tot, double T12[16]) {
+    SolveResult r{false, false, 0};
+    double v[kIcpVals - 1], x6[6];
+    for (int k = 0; k < kIcpVals - 1; ++k) v[k] = tot[k];  // upper triangle, J^T r, count
+    if (P.icp_min_valid > 0 && v[27] < (double)P.icp_min_valid) {
+        r.failed = 7;
+        return r;
+    }
+    r.failed = solve6(v, v + 21, (double)P.icp_rel_pivot, x6);
+    if (r.failed != 0) return r;
+    double ninf = 0.0;
+    for (int i = 0; i < 6; ++i) ninf = fmax(ninf, fabs(x6[i]));
+    if (ninf < 5.0e-7) {
+        r.converged = true;
+        return r;
+    }
+    double E[16];
+    expmap(x6, E);
+    affine_matmul(E, T12, T12);
+    r.updated = true;
+    return r;
+}
+
+// Second half of the two-launch form: one workgroup per session sums the
+// group partials, solves the 6x6 system and applies the SE(3) update. THREADS
+// changes how many of the sums run at once, not their order.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_icp_solve(const SessParams *__restrict__ SP, int nsess, int level,
+                                                            int iter) {
+    __shared__ double chunk[kSumChunks][kIcpVals], tot[kIcpVals];
     const int s = blockIdx.x;
     if (s >= nsess) return;
     const SessParams &P = SP[s];
     SessState *st = P.st;
     if (level >= P.levels || icp_skip(P, st, level, iter)) return;
     const LevelDesc &L = P.lev[level];
-    const int ngroups = icp_groups(L.tiles_x * L.tiles_y, level);
-    const int lane = threadIdx.x;
-    double acc[32];
-#pragma unroll
-    for (int k = 0; k < 32; ++k) acc[k] = 0.0;
-    for (int t = lane; t < ngroups; t += kSolveThreads) {
-        const double *pp = P.icp_part + (size_t)t * kIcpVals;
-#pragma unroll
-        for (int k = 0; k < kIcpVals; ++k) acc[k] += ldg(pp, k);
-    }
-#pragma unroll
-    for (int h = 16; h >= 1; h >>= 1) {  // partner lane ^ 2h; keep the upper h sums when that bit is set
-        const bool up = (lane & (2 * h)) != 0;
-#pragma unroll
-        for (int i = 0; i < h; ++i) {
-            const double send = up ? acc[i] : acc[h + i];
-            const double keep = up ? acc[h + i] : acc[i];
-            acc[i] = keep + __shfl_xor(send, 2 * h, 64);
-        }
-    }
-    const double own = acc[0] + __shfl_xor(acc[0], 1, 64);  // sum (lane / 2) over all 64 lanes
-    double tot[kIcpVals];
-    {
-        const int lo = __double2loint(own), hi = __double2hiint(own);
-#pragma unroll
-        for (int k = 0; k < kIcpVals; ++k)
-            tot[k] = __hiloint2double(__builtin_amdgcn_readlane(hi, 2 * k), __builtin_amdgcn_readlane(lo, 2 * k));
-    }
-    if (lane != 0) return;
-    double ATA[36], ATb[6], x6[6];
-    int k = 0;
-    for (int i = 0; i < 6; ++i)
-        for (int j = i; j < 6; ++j) {
-            ATA[i * 6 + j] = ATA[j * 6 + i] = tot[k++];
-        }
-    for (int i = 0; i < 6; ++i) ATb[i] = tot[k++];
-    const double cnt = tot[21 + 6];
+    sum_partials<THREADS>(P.icp_part, icp_groups(L.tiles_x * L.tiles_y, level), chunk, tot);
+    if (threadIdx.x != 0) return;
     // state through global-qualified accesses (a chain of generic accesses
     // in one thread waits on both the vector-memory and the scalar counters)
     double T12[16];
     for (int i = 0; i < 16; ++i) T12[i] = ldg(st->T_12, i);
     stg(&st->solves, 0, ldg(&st->solves, 0) + 1);
-    if (P.icp_min_valid > 0 && cnt < (double)P.icp_min_valid) {
-        stg(&st->icp_failed, 0, 7);
-        return;
-    }
-    const int cs = cholesky_solve(ATA, ATb, (double)P.icp_rel_pivot, x6);
-    if (cs != 0) {
-        stg(&st->icp_failed, 0, cs);
-        return;
-    }
-    double ninf = 0.0;
-    for (int i = 0; i < 6; ++i) ninf = fmax(ninf, fabs(x6[i]));
-    if (ninf < 5.0e-7) {
+    const SolveResult r = solve_totals(P, tot, T12);
+    if (r.failed) {
+        stg(&st->icp_failed, 0, r.failed);
+    } else if (r.converged) {
         stg(&st->conv_level, 0, level);
-        return;
-    }
-    double E[16], T21[16];
-    expmap(x6, E);
-    matmul4d(E, T12, T12);
-    rigid_inverse(T12, T21);
-    for (int i = 0; i < 16; ++i) {
-        stg(st->T_12, i, T12[i]);
-        stg(st->T_21, i, T21[i]);
-        stg(st->T_21_f, i, (float)T21[i]);
+    } else {
+        double T21[16];
+        rigid_inverse(T12, T21);
+        for (int i = 0; i < 16; ++i) {
+            stg(st->T_12, i, T12[i]);
+            stg(st->T_21, i, T21[i]);
+            stg(st->T_21_f, i, (float)T21[i]);
+        }
     }
 }
+
+// The one-launch form of an iteration: every workgroup of a session first
+// solves the previous iteration's system, each for itself from the same
+// partials in the same order, and then sums its group at the new pose. It
+// costs the solve (~2 us of one wave) in every workgroup and saves a launch
+// and its gap per iteration; which form is faster depends on how many
+// workgroups share a CU (kIcpStepGroups). The kernel boundary orders the
+// partials; workgroup 0 of a session records where the loop stands for the
+// next launch, in the record and the half of icp_part that this launch's
+// workgroups do not read.
+constexpr int kStepThreads = 1024;
+struct StepShared {
+    double chunk[kSumChunks][kIcpVals], tot[kIcpVals];
+    double T12[16];
+    float T21f[16];
+    int failed, conv_level, solves;
+};
+// Brings the loop up to date into sh (all threads); returns the record it
+// started from. seq: only records of earlier launches count.
+__device__ __forceinline__ int step_resume(const SessParams &P, const SessState *st, int seq, StepShared &sh) {
+    const int s0 = ldg(&st->step[0].seq, 0), s1 = ldg(&st->step[1].seq, 0);
+    const int cur = (s1 < seq && (s0 >= seq || s1 > s0)) ? 1 : 0;
+    const IcpStep *S = &st->step[cur];
+    const int pending = ldg(&S->pending, 0);
+    if (threadIdx.x < 16) sh.T12[threadIdx.x] = ldg(S->T_12, threadIdx.x);
+    if (threadIdx.x == 16) {
+        sh.failed = ldg(&S->failed, 0);
+        sh.conv_level = ldg(&S->conv_level, 0);
+        sh.solves = ldg(&S->solves, 0);
+    }
+    if (pending >= 0) {
+        const LevelDesc &L = P.lev[pending];
+        sum_partials<kStepThreads>(P.icp_part + (size_t)cur * P.icp_half, icp_groups(L.tiles_x * L.tiles_y, pending),
+                                   sh.chunk, sh.tot);
+    } else {
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        double T12[16];
+        for (int i = 0; i < 16; ++i) T12[i] = sh.T12[i];
+        if (pending >= 0) {
+            const SolveResult r = solve_totals(P, sh.tot, T12);
+            sh.solves += 1;
+            if (r.failed) sh.failed = r.failed;
+            else if (r.converged) sh.conv_level = pending;
+            else
+                for (int i = 0; i < 16; ++i) sh.T12[i] = T12[i];
+        }
+        double T21[16];
+        rigid_inverse(T12, T21);
+        for (int i = 0; i < 16; ++i) sh.T21f[i] = (float)T21[i];
+    }
+    __syncthreads();
+    return cur;
+}
+
+// The same sums as group_sums by 16 waves: wave (c, q), c = wave % 4, evaluates
+// the pixels that wave c of group_sums has in the group's tiles q * G / 4,
+// ..., all loads at once, and leaves their rows in LDS; then wave (c, 0) runs
+// c's chain of matrix instructions over the group's rows in the same order,
+// so the sums are the same bits. A 150-group launch leaves 106 CUs idle
+// anyway; with 4 waves a workgroup walked its 8 tiles one after another
+// (640x480, level 0: 7.2 us of the iteration's 13.1; the launch-to-launch time
+// of an iteration is now 11.3).
+#if VS_ICP_MFMA
+template <int G>
+struct WidePixels {
+    static constexpr int N = G / 4;  // tiles per wave
+    int xs[N], ys[N];
+    float td[N];
+    __device__ __forceinline__ void load(const SessParams &P, int level, int t0) {
+        const LevelDesc &L = P.lev[level];
+        const int ntiles = L.tiles_x * L.tiles_y;
+        const int wave = threadIdx.x >> 6, tt = (wave & 3) * 64 + (threadIdx.x & 63);  // thread of the tile
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+            const int tile = t0 + (wave >> 2) * N + j;
+            xs[j] = (tile % L.tiles_x) * kTileW + tt % kTileW;
+            ys[j] = (tile / L.tiles_x) * kTileH + tt / kTileW;
+            const bool in = tile < ntiles && xs[j] < L.W && ys[j] < L.H;
+            const float d = ldg(P.filt[level], in ? (size_t)ys[j] * L.W + xs[j] : (size_t)0);
+            td[j] = in ? d : 0.0f;
+        }
+    }
+};
+template <int G>
+__device__ __forceinline__ void group_sums_wide(const SessParams &P, int level, const WidePixels<G> &px,
+                                                const float *T21s, double *out) {
+    constexpr int N = WidePixels<G>::N;
+    __shared__ __align__(16) float feat[4][G][64][8];
+    __shared__ float gw[4][8][8];
+    const int wave = threadIdx.x >> 6, c = wave & 3, q = wave >> 2, lane = threadIdx.x & 63;
+    IcpPre pre[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) pre[j] = icp_pre(P, level, px.xs[j], px.ys[j], px.td[j], T21s);
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+        float A[6], b;
+        const bool ok = icp_post(P, pre[j], A, b);
+        float *f = feat[c][q * N + j][lane];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) f[k] = A[k];
+        f[6] = b;
+        f[7] = ok ? 1.0f : 0.0f;
+    }
+    __syncthreads();
+    if (q == 0) {
+        const int row = ((lane & 15) >> 3) * 4 + (lane >> 4), fi = lane & 7;
+        vs_f4x g4 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int m = 0; m < 8; ++m) {
+                const float a = feat[c][g][8 * m + row][fi];
+                g4 = __builtin_amdgcn_mfma_f32_16x16x4f32(a, a, g4, 0, 0, 0);
+            }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float other = __shfl_down(g4[r], 40, 64);
+            if ((lane >> 4) < 2 && (lane & 15) < 8) gw[c][4 * (lane >> 4) + r][lane & 15] = g4[r] + other;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < kIcpVals) {
+        int i, j;
+        term_ij(threadIdx.x, i, j);
+        double s = 0.0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) s += (double)gw[w][i][j];
+        stg(out, threadIdx.x, s);
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(kStepThreads) void k_icp_step(const SessParams *__restrict__ SP,
+                                                           const WorkItem *__restrict__ work, int level, int iter,
+                                                           int seq) {
+    __shared__ StepShared sh;
+    const WorkItem wi = work[blockIdx.x];
+    const SessParams &P = SP[wi.sess];
+    SessState *st = P.st;
+    if (level >= P.levels || !ldg(&st->do_track, 0)) return;
+    const LevelDesc &L = P.lev[level];
+    const int t0 = wi.tile * G;
+    if (t0 >= L.tiles_x * L.tiles_y) return;
+    WidePixels<G> px;
+    px.load(P, level, t0);  // in flight during the solve
+    const int out = step_resume(P, st, seq, sh) ^ 1;
+    const bool skip = sh.failed || sh.conv_level == level || iter >= P.iters[level] ||
+                      (ldg(&st->force_single, 0) && level != 0);
+    if (wi.tile == 0) {
+        IcpStep *S = &st->step[out];
+        if (threadIdx.x < 16) stg(S->T_12, threadIdx.x, sh.T12[threadIdx.x]);
+        if (threadIdx.x == 16) {
+            stg(&S->seq, 0, seq);
+            stg(&S->pending, 0, skip ? -1 : level);
+            stg(&S->failed, 0, sh.failed);
+            stg(&S->conv_level, 0, sh.conv_level);
+            stg(&S->solves, 0, sh.solves);
+        }
+    }
+    if (skip) return;
+    group_sums_wide<G>(P, level, px, sh.T21f, P.icp_part + (size_t)out * P.icp_half + (size_t)wi.tile * kIcpVals);
+}
+#endif
 
 // Per-frame / per-track reset of the tracker state (one thread per session).
 // `active` (nullable: all active) marks the sessions of a slot table that have
@@ -545,8 +790,18 @@ __global__ void k_track_setup(const SessParams *__restrict__ SP, int nsess, Mat1
     st->conv_level = -1;
     st->solves = 0;
     st->force_single = has_init;
-    for (int k = 0; k < 16; ++k) st->T_12[k] = has_init ? Tinit.m[k] : ((k % 5) == 0 ? 1.0 : 0.0);
+    for (int k = 0; k < 16; ++k) {
+        const double v = has_init ? Tinit.m[k] : ((k % 5) == 0 ? 1.0 : 0.0);
+        st->T_12[k] = v;
+        st->step[0].T_12[k] = v;
+    }
     publish_T21(st);
+    st->step[0].seq = 0;
+    st->step[0].pending = -1;
+    st->step[0].failed = 0;
+    st->step[0].conv_level = -1;
+    st->step[0].solves = 0;
+    st->step[1].seq = -1;
 }
 
 __device__ void set_pose_derived(const SessParams &P, SessState *st) {
@@ -579,15 +834,7 @@ __device__ double rotation_deg(const double *T) {
 
 // Apply the tracked increment (T_gc <- T_12 T_gc, pose_tracker.cu:992-998) or
 // record the failure; decides whether the frame is integrated.
-__global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nsess) return;
-    const SessParams &P = SP[s];
-    SessState *st = P.st;
-    if (!st->active) {
-        st->fuse_ok = 0;
-        return;
-    }
+__device__ __forceinline__ void track_finalize(const SessParams &P, SessState *st) {
     int status = 0;
     if (st->do_track) {
         if (st->icp_failed) {
@@ -607,6 +854,38 @@ __global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess) {
     st->last_status = status;
     st->fuse_ok = (status == 0);
     if (status == 0) st->frames += 1;
+}
+__global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nsess) return;
+    const SessParams &P = SP[s];
+    SessState *st = P.st;
+    if (!st->active) {
+        st->fuse_ok = 0;
+        return;
+    }
+    track_finalize(P, st);
+}
+// The same after the one-launch iterations: one workgroup per session solves
+// the last one first.
+__global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *__restrict__ SP, int nsess) {
+    __shared__ StepShared sh;
+    const SessParams &P = SP[blockIdx.x];
+    SessState *st = P.st;
+    if (!st->active) {
+        if (threadIdx.x == 0) st->fuse_ok = 0;
+        return;
+    }
+    if (st->do_track) {
+        step_resume(P, st, 0x7FFFFFFF, sh);
+        if (threadIdx.x == 0) {
+            for (int i = 0; i < 16; ++i) st->T_12[i] = sh.T12[i];
+            st->icp_failed = sh.failed;
+            st->conv_level = sh.conv_level;
+            st->solves = sh.solves;
+        }
+    }
+    if (threadIdx.x == 0) track_finalize(P, st);
 }
 
 // Pose set from the host: derived copies only.
@@ -697,7 +976,30 @@ void launch_icp_iter(const SessParams *P, const WorkItem *work, int n, int nsess
         hipLaunchKernelGGL(k_icp_iter<icp_group(1)>, dim3(n), dim3(kTileThreads), 0, s, P, work, level, iter);
     else
         hipLaunchKernelGGL(k_icp_iter<icp_group(2)>, dim3(n), dim3(kTileThreads), 0, s, P, work, level, iter);
-    hipLaunchKernelGGL(k_icp_solve, dim3(nsess), dim3(kSolveThreads), 0, s, P, nsess, level, iter);
+    // 16 waves read a 1280x960 frame's 600 partials fastest when the chip is
+    // otherwise idle (fused frame with preview 1177 us with 4 waves, 1125 with
+    // 16), but have to wait for a CU with room for all of them while the other
+    // parts of a large batch fill it (64 sessions: 6.27 ms a step with 2 or 4
+    // waves, 6.35 with 8, 6.30 with 1; 24-slot server 889 us with 4 and 958
+    // with 1)
+    if (nsess <= 4)
+        hipLaunchKernelGGL(k_icp_solve<kStepThreads>, dim3(nsess), dim3(kStepThreads), 0, s, P, nsess, level, iter);
+    else
+        hipLaunchKernelGGL(k_icp_solve<kTileThreads>, dim3(nsess), dim3(kTileThreads), 0, s, P, nsess, level, iter);
+}
+void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level, int iter, int seq, hipStream_t s) {
+    if (n <= 0) return;
+#if VS_ICP_MFMA
+    if (level == 0)
+        hipLaunchKernelGGL(k_icp_step<icp_group(0)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq);
+    else if (level == 1)
+        hipLaunchKernelGGL(k_icp_step<icp_group(1)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq);
+    else
+        hipLaunchKernelGGL(k_icp_step<icp_group(2)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq);
+#endif
+}
+void launch_icp_finish(const SessParams *P, int nsess, hipStream_t s) {
+    hipLaunchKernelGGL(k_icp_finish, dim3(nsess), dim3(kStepThreads), 0, s, P, nsess);
 }
 void launch_track_finalize(const SessParams *P, int nsess, hipStream_t s) {
     hipLaunchKernelGGL(k_track_finalize, dim3((nsess + 63) / 64), dim3(64), 0, s, P, nsess);

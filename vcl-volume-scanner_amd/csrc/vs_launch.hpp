@@ -5,6 +5,9 @@
 
 #include "vs_device.hpp"
 
+#ifndef VS_ICP_STEP_GROUPS
+#define VS_ICP_STEP_GROUPS 256  // (0 with VS_ICP_MFMA=0: the form exists for the matrix-core sums only)
+#endif
 namespace vs {
 
 // image stages (vs_img.hip)
@@ -35,6 +38,16 @@ void launch_set_active(int *active, int nslots, const uint32_t bits[kMaxSlots / 
 void launch_icp_iter(const SessParams *P, const WorkItem *work, int n, int nsess, int level, int iter,
                      hipStream_t s);
 void launch_track_finalize(const SessParams *P, int nsess, hipStream_t s);
+// The one-launch form of an iteration, for launches of up to kIcpStepGroups
+// level-0 groups, a CU each for their 16-wave workgroups. Fused frame with
+// preview, two launches / one: 38 groups (320x240) 427 / 382 us, 150
+// (640x480) 489 / 442, 136 with colour 534 / 487; beyond it 600 groups
+// (1280x960) 1125 / 1246 and a 24-slot server's 2291 1295 / 1359.
+constexpr int kIcpStepGroups = VS_ICP_STEP_GROUPS;
+// seq: 1, 2, ... over the launches of one track
+void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level, int iter, int seq, hipStream_t s);
+// the last iteration's solve, then launch_track_finalize's work
+void launch_icp_finish(const SessParams *P, int nsess, hipStream_t s);
 // one system, no solve: writes 29 doubles (+ optional mask) for diagnostics
 void launch_icp_system(const SessParams *P, const WorkItem *work, int n, int level, const float *T21,
                        double *out_part, uint8_t *mask, hipStream_t s);
