@@ -33,22 +33,6 @@ __device__ void matmul4d(const double *A, const double *B, double *C) {
         }
     for (int k = 0; k < 16; ++k) C[k] = t[k];
 }
-// C = A B for an A whose last row is (0, 0, 0, 1).
-__device__ __forceinline__ void affine_matmul(const double *A, const double *B, double *C) {
-    double t[12];
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            double s = A[r * 4] * B[c];
-            for (int k = 1; k < 4; ++k) s = fma(A[r * 4 + k], B[k * 4 + c], s);
-            t[r * 4 + c] = s;
-        }
-#pragma unroll
-    for (int k = 0; k < 12; ++k) C[k] = t[k];
-#pragma unroll
-    for (int k = 12; k < 16; ++k) C[k] = B[k];
-}
 // Inverse of a rigid transform: [R^T, -R^T t]. Equals the reference's general
 // 4x4 inverse (d_im_Inverse_Matrix_4x4, _yooji_math_inlines.h:404-465) on
 // rigid inputs.
@@ -65,32 +49,15 @@ __device__ void rigid_inverse(const double *T, double *Ti) {
 // SE(3) exponential of x = [w; v] (the twist update of
 // z_uitme_Update_Incremental_Tracking_with_Matrix_Exponential, pose_tracker.cu:50-149),
 // with a series branch for small |w| (the reference divides by |w|).
-// Coefficients of th^2k in sin(th) / th, (1 - cos(th)) / th^2 and
-// (th - sin(th)) / th^3: (-1)^k / (2k + 1)!, / (2k + 2)!, / (2k + 3)!.
-constexpr double kExpA[8] = {1.0, -1.0 / 6, 1.0 / 120, -1.0 / 5040, 1.0 / 362880, -1.0 / 39916800, 1.0 / 6227020800.0,
-                             -1.0 / 1307674368000.0};
-constexpr double kExpB[8] = {1.0 / 2, -1.0 / 24, 1.0 / 720, -1.0 / 40320, 1.0 / 3628800, -1.0 / 479001600,
-                             1.0 / 87178291200.0, -1.0 / 20922789888000.0};
-constexpr double kExpC[8] = {1.0 / 6, -1.0 / 120, 1.0 / 5040, -1.0 / 362880, 1.0 / 39916800, -1.0 / 6227020800.0,
-                             1.0 / 1307674368000.0, -1.0 / 355687428096000.0};
 __device__ void expmap(const double *x, double *T) {
     const double w0 = x[0], w1 = x[1], w2 = x[2];
-    const double th2 = w0 * w0 + w1 * w1 + w2 * w2;
+    const double th2 = w0 * w0 + w1 * w1 + w2 * w2, th = sqrt(th2);
     double A, B, C;
-    if (th2 < 0.25) {
-        // series in th^2 to beyond double precision (0.25^8 / 17! < 1e-19);
-        // free of the cancellation in 1 - cos and th - sin, and a third of
-        // the instructions of a sine and a cosine
-        A = B = C = 0.0;
-#pragma unroll
-        for (int k = 7; k >= 0; --k) {
-            const double a = kExpA[k], b = kExpB[k], c = kExpC[k];
-            A = fma(A, th2, a);
-            B = fma(B, th2, b);
-            C = fma(C, th2, c);
-        }
+    if (th < 1e-4) {
+        A = 1.0 - th2 / 6.0 + th2 * th2 / 120.0;
+        B = 0.5 - th2 / 24.0 + th2 * th2 / 720.0;
+        C = 1.0 / 6.0 - th2 / 120.0 + th2 * th2 / 5040.0;
     } else {
-        const double th = sqrt(th2);
         A = sin(th) / th;
         B = (1.0 - cos(th)) / th2;
         C = (th - sin(th)) / (th2 * th);
@@ -111,60 +78,49 @@ __device__ void expmap(const double *x, double *T) {
     T[12] = T[13] = T[14] = 0.0;
     T[15] = 1.0;
 }
-// The 6x6 solve with the reference's pivot rule (d_lld_LL_Decomposition /
-// d_sls_Solve_Linear_System_using_LLD, _yooji_cuda_math.h:489-592): it fails
-// (status 4) if any Cholesky pivot L_jj is below 1e-8 (or not a number). With
+// Cholesky and triangular solves with the reference's pivot rule
+// (d_lld_LL_Decomposition / d_sls_Solve_Linear_System_using_LLD,
+// _yooji_cuda_math.h:489-592): entries below a pivot < 1e-8 are zeroed and the
+// solve fails (status 4) if any pivot is below 1e-8 (or not a number). With
 // rel > 0 it also fails (status 8) when a squared pivot L_jj^2 is below
 // rel * A_jj: column j of J is then nearly a combination of the columns
 // before it (a plane leaves 3 of the 6 motions unconstrained), a near-rank
 // deficiency the absolute test cannot see at FP32 scales. The ratio is
 // invariant to the units of the rotation and translation columns.
-// Factored as L D L^T, D_j = L_jj^2: the chain of one lane then holds one
-// reciprocal per pivot (two Newton steps on the hardware estimate, to the
-// last bit or two of FP64) where the square-root form had a square root and a
-// division. A is the upper triangle row by row (21 values). Returns 0 on
-// success.
-__device__ __forceinline__ int solve6(const double *A, const double *b, double rel, double *x) {
-    double u[6][6], l[6][6], r[6];  // u = l D below the diagonal
-    bool ok = true, weak = false;
-    int k0 = 0;
-#pragma unroll
+// Column by column, each below-diagonal entry and substitution step scaled by
+// the column's reciprocal pivot (6 FP64 divisions instead of 33 on the
+// solve's one-lane chain; the same sums in the same order).
+// Returns 0 on success.
+__device__ int cholesky_solve(const double *A, const double *b, double rel, double *x) {
+    double L[36], inv[6];
+    for (int k = 0; k < 36; ++k) L[k] = 0.0;
     for (int j = 0; j < 6; ++j) {
-        double d = A[k0];
-#pragma unroll
-        for (int k = 0; k < j; ++k) d = fma(-u[j][k], l[j][k], d);
-        ok &= d >= 1.0e-16;
-        weak |= d < rel * A[k0];
-        double q = __builtin_amdgcn_rcp(d);
-        q = fma(q, fma(-d, q, 1.0), q);
-        q = fma(q, fma(-d, q, 1.0), q);
-        r[j] = d < 1.0e300 ? q : 0.0;
-#pragma unroll
+        double s = 0.0;
+        for (int k = 0; k < j; ++k) s += L[j * 6 + k] * L[j * 6 + k];
+        L[j * 6 + j] = sqrt(A[j * 6 + j] - s);
+        inv[j] = 1.0 / L[j * 6 + j];
+        const bool piv = fabs(L[j * 6 + j]) >= 1e-8;
         for (int i = j + 1; i < 6; ++i) {
-            double t = A[k0 + i - j];
-#pragma unroll
-            for (int k = 0; k < j; ++k) t = fma(-u[i][k], l[j][k], t);
-            u[i][j] = t;
-            l[i][j] = t * r[j];
+            double t = 0.0;
+            for (int k = 0; k < j; ++k) t += L[i * 6 + k] * L[j * 6 + k];
+            L[i * 6 + j] = piv ? (A[i * 6 + j] - t) * inv[j] : 0.0;
         }
-        k0 += 6 - j;
     }
-    if (!ok) return 4;
-    if (rel > 0.0 && weak) return 8;
+    for (int i = 0; i < 6; ++i)
+        if (!(fabs(L[i * 6 + i]) >= 1e-8)) return 4;
+    if (rel > 0.0)
+        for (int i = 0; i < 6; ++i)
+            if (L[i * 6 + i] * L[i * 6 + i] < rel * A[i * 6 + i]) return 8;
     double y[6];
-#pragma unroll
     for (int i = 0; i < 6; ++i) {
-        double t = b[i];
-#pragma unroll
-        for (int k = 0; k < i; ++k) t = fma(-l[i][k], y[k], t);
-        y[i] = t;
+        double s = 0.0;
+        for (int k = 0; k < i; ++k) s += L[i * 6 + k] * y[k];
+        y[i] = (b[i] - s) * inv[i];
     }
-#pragma unroll
     for (int i = 5; i >= 0; --i) {
-        double t = y[i] * r[i];
-#pragma unroll
-        for (int k = 5; k > i; --k) t = fma(-l[k][i], x[k], t);
-        x[i] = t;
+        double s = 0.0;
+        for (int k = i + 1; k < 6; ++k) s += L[k * 6 + i] * x[k];
+        x[i] = (y[i] - s) * inv[i];
     }
     return 0;
 }
@@ -500,16 +456,16 @@ __global__ __launch_bounds__(kTileThreads) void k_icp_iter(const SessParams *__r
 }
 
 // The 29 totals of ng group partials in FP64, in a fixed order that depends
-// on the group count alone: thread (chunk c, term k) adds groups c, c + 32,
-// ..., then the 32 chunk sums of a term are added as a fixed tree. Neighbouring
-// threads read neighbouring terms, so a load covers whole lines, and a
-// 640x480 frame's 150 groups are one round of loads. (One wave with a group
-// per lane read 64 lines per load.) Result in tot (LDS), visible to the first
-// wave only.
-constexpr int kSumChunks = 32;
+// on the group count alone: chunk c adds groups c, c + 64, ..., then the 64
+// chunk sums of a term are added as a tree of halves. A thread takes a (chunk,
+// term) pair, so neighbouring threads read neighbouring terms and a load
+// covers whole lines. (One wave with a group per lane, its sums exchanged
+// between the lanes in the same tree, read 64 lines per load.) Result in tot
+// (LDS), visible to the first wave only.
+constexpr int kSumChunks = 64;
 template <int THREADS>
 __device__ __forceinline__ void sum_partials(const double *part, int ng, double (*chunk)[kIcpVals], double *tot) {
-    constexpr int U = 5, kPairs = kSumChunks * kIcpVals;
+    constexpr int U = 3, kPairs = kSumChunks * kIcpVals;
     const int t = threadIdx.x;
 #pragma unroll
     for (int p0 = 0; p0 < kPairs; p0 += THREADS) {
@@ -527,15 +483,24 @@ __device__ __forceinline__ void sum_partials(const double *part, int ng, double 
         }
     }
     __syncthreads();
-    if (t < kIcpVals) {
-        double v[kSumChunks];
+    // two threads per term, each half of the first level's pairs
+    if (t < 2 * 32) {
+        const int k = t & 31, side = t >> 5;
+        if (k < kIcpVals) {
+            double v[16];
 #pragma unroll
-        for (int q = 0; q < kSumChunks; ++q) v[q] = chunk[q][t];
+            for (int q = 0; q < 16; ++q) {
+                const int c = q + 16 * side;
+                v[q] = chunk[c][k] + chunk[c + 32][k];
+            }
 #pragma unroll
-        for (int h = kSumChunks / 2; h >= 1; h >>= 1)
+            for (int q = 0; q < 16; ++q) v[q] += __shfl_xor(v[q], 32, 64);
 #pragma unroll
-            for (int q = 0; q < h; ++q) v[q] += v[q + h];
-        tot[t] = v[0];
+            for (int h = 8; h >= 1; h >>= 1)
+#pragma unroll
+                for (int q = 0; q < h; ++q) v[q] += v[q + h];
+            if (side == 0) tot[k] = v[0];
+        }
     }
     __builtin_amdgcn_wave_barrier();
 }
@@ -549,13 +514,19 @@ struct SolveResult {
 };
 __device__ __forceinline__ SolveResult solve_totals(const SessParams &P, const double *tot, double T12[16]) {
     SolveResult r{false, false, 0};
-    double v[kIcpVals - 1], x6[6];
-    for (int k = 0; k < kIcpVals - 1; ++k) v[k] = tot[k];  // upper triangle, J^T r, count
-    if (P.icp_min_valid > 0 && v[27] < (double)P.icp_min_valid) {
+    double ATA[36], ATb[6], x6[6];
+    int k = 0;
+    for (int i = 0; i < 6; ++i)
+        for (int j = i; j < 6; ++j) {
+            ATA[i * 6 + j] = ATA[j * 6 + i] = tot[k++];
+        }
+    for (int i = 0; i < 6; ++i) ATb[i] = tot[k++];
+    const double cnt = tot[21 + 6];
+    if (P.icp_min_valid > 0 && cnt < (double)P.icp_min_valid) {
         r.failed = 7;
         return r;
     }
-    r.failed = solve6(v, v + 21, (double)P.icp_rel_pivot, x6);
+    r.failed = cholesky_solve(ATA, ATb, (double)P.icp_rel_pivot, x6);
     if (r.failed != 0) return r;
     double ninf = 0.0;
     for (int i = 0; i < 6; ++i) ninf = fmax(ninf, fabs(x6[i]));
@@ -565,7 +536,7 @@ __device__ __forceinline__ SolveResult solve_totals(const SessParams &P, const d
     }
     double E[16];
     expmap(x6, E);
-    affine_matmul(E, T12, T12);
+    matmul4d(E, T12, T12);
     r.updated = true;
     return r;
 }
