@@ -312,8 +312,60 @@ struct Batch {
     HostStage hs;  // host-memory frames of this batch's steps
 };
 
+// Page-locked records of the sessions (HostState), in slabs of kSlab. A slot
+// table's session may be closed while steps that write its record are in
+// flight: the record is then free again after an event behind them.
+constexpr int kSlab = 256;
+struct HostStates {
+    std::vector<HostState *> slabs, free;
+    struct Retired {
+        HostState *p;
+        hipEvent_t done;
+    };
+    std::vector<Retired> retired;
+    hipError_t take(HostState **out) {
+        for (size_t k = 0; k < retired.size();) {
+            if (hipEventQuery(retired[k].done) == hipSuccess) {
+                hipEventDestroy(retired[k].done);
+                free.push_back(retired[k].p);
+                retired[k] = retired.back();
+                retired.pop_back();
+            } else {
+                ++k;
+            }
+        }
+        if (free.empty()) {
+            HostState *s = nullptr;
+            const hipError_t e = hipHostMalloc((void **)&s, kSlab * sizeof(HostState), hipHostMallocDefault);
+            if (e != hipSuccess) return e;
+            slabs.push_back(s);
+            for (int k = kSlab - 1; k >= 0; --k) free.push_back(s + k);
+        }
+        *out = free.back();
+        free.pop_back();
+        return hipSuccess;
+    }
+    // free after the work enqueued on h so far (a record whose event cannot be made is not used again)
+    void retire(HostState *p, hipStream_t h) {
+        Retired r{p, nullptr};
+        if (hipEventCreateWithFlags(&r.done, hipEventDisableTiming) != hipSuccess) return;
+        if (hipEventRecord(r.done, h) != hipSuccess) {
+            hipEventDestroy(r.done);
+            return;
+        }
+        retired.push_back(r);
+    }
+    // after the device is idle
+    void release() {
+        for (auto &r : retired) hipEventDestroy(r.done);
+        for (HostState *s : slabs) hipHostFree(s);
+        *this = HostStates();
+    }
+};
+
 struct vs_ctx {
     int device = 0;
+    HostStates hosts;
     double *scratch = nullptr;  // this device's copy of `scratch` (vs_icp_system_noalloc)
     std::map<std::vector<vs_session *>, std::unique_ptr<Batch>> batches;
     std::vector<vs_session *> sessions;
@@ -334,6 +386,7 @@ struct vs_session {
     char *mem = nullptr;
     SessParams hp{};
     SessState *st = nullptr;
+    HostState *host = nullptr;
     hipStream_t stream = nullptr;
     hipStream_t last = nullptr;
     Batch self;
@@ -1132,6 +1185,8 @@ vs_status vs_ctx_destroy(vs_ctx *ctx) {
     std::vector<vs_session *> ss = ctx->sessions;
     for (vs_session *s : ss) vs_session_destroy(s);
     ctx->timer.destroy();
+    (void)hipDeviceSynchronize();
+    ctx->hosts.release();
     delete ctx;
     return VS_OK;
 }
@@ -1167,6 +1222,17 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
         return fail(VS_ENOMEM, "device allocation of %zu bytes failed: %s", L.total, hipGetErrorString(e));
     }
     s->pooled = pooled;
+    e = ctx->hosts.take(&s->host);
+    if (e != hipSuccess) {
+        if (pooled) {
+            hipFreeAsync(s->mem, s->stream);
+            hipStreamSynchronize(s->stream);
+        } else {
+            hipFree(s->mem);
+        }
+        hipStreamDestroy(s->stream);
+        return fail(VS_ENOMEM, "host record: %s", hipGetErrorString(e));
+    }
     char *m = s->mem;
     SessParams &P = s->hp;
     std::memset(&P, 0, sizeof(P));
@@ -1272,6 +1338,7 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
         HIP_TRY(hipMemcpy(wt, h.data(), h.size() * 4, hipMemcpyHostToDevice));
     }
     P.st = (SessState *)(m + L.state);
+    P.host = s->host;
     P.tsdf_type = d.tsdf_type;
     P.weight_type = d.weight_type;
     P.integ_mode = d.integrate_mode;
@@ -1341,6 +1408,7 @@ vs_status vs_session_destroy(vs_session *s) {
         free_batch_graph(s->self);
         s->timer.destroy();
         if (s->stream) hipStreamDestroy(s->stream);
+        s->ctx->hosts.retire(s->host, server_order(v));
         if (s->mem) {
             if (s->pooled) {
                 hipFreeAsync(s->mem, server_order(v));
@@ -1372,6 +1440,7 @@ vs_status vs_session_destroy(vs_session *s) {
             hipFree(s->mem);
         }
     }
+    s->ctx->hosts.free.push_back(s->host);
     auto &v = s->ctx->sessions;
     v.erase(std::remove(v.begin(), v.end(), s), v.end());
     delete s;
@@ -1661,8 +1730,7 @@ vs_status vs_get_frame_status(vs_session *s, int *last_status, int *frames_fused
     if (!s) return fail(VS_EINVAL, "null session");
     vs_status r = sync_last(s);
     if (r != VS_OK) return r;
-    SessState st;
-    HIP_TRY(hipMemcpy(&st, s->st, sizeof(st), hipMemcpyDeviceToHost));
+    const HostState &st = *s->host;
     if (last_status) *last_status = st.last_status;
     if (frames_fused) *frames_fused = st.frames;
     if (icp_iters) *icp_iters = st.solves;
@@ -1673,7 +1741,7 @@ vs_status vs_get_pose(vs_session *s, double T_gc[16]) {
     if (!s || !T_gc) return fail(VS_EINVAL, "null argument");
     vs_status r = sync_last(s);
     if (r != VS_OK) return r;
-    HIP_TRY(hipMemcpy(T_gc, s->st->T_gc, 16 * sizeof(double), hipMemcpyDeviceToHost));
+    std::memcpy(T_gc, s->host->T_gc, 16 * sizeof(double));
     return VS_OK;
 }
 
@@ -1942,6 +2010,7 @@ vs_status restore_session(vs_ctx *ctx, const void *buf, size_t bytes, bool poole
     if (e == hipSuccess) {
         const int32_t frames = h.frames;
         e = hipMemcpy((char *)s->st + offsetof(SessState, frames), &frames, sizeof(frames), hipMemcpyHostToDevice);
+        launch_pose_derived(s->self.dP, s->stream);  // the pose as it is, and the host's record with the count
     }
     if (e != hipSuccess) {
         vs_session_destroy(s);

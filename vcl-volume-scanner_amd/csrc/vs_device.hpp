@@ -109,6 +109,14 @@ struct alignas(16) SessState {
     unsigned long long upd_count;  // voxels updated by the last integrate
 };
 
+// What the host asks for after every frame, in page-locked host memory: the
+// kernels that change it write it there too (publish_host), so reading it
+// needs a wait but no transfer.
+struct alignas(64) HostState {
+    double T_gc[16];
+    int last_status, frames, solves, pad;
+};
+
 // One element of a model vertex or normal map: x, y, z (12 bytes, AoS like
 // the reference's float3 maps); -100 in x marks an invalid pixel.
 struct MapXYZ {
@@ -171,6 +179,7 @@ struct alignas(16) SessParams {
     // _yooji_cuda_math.h:285-302), evaluated once per session: wtab[a][i]
     const float *wtab[3];
     SessState *st;
+    HostState *host;         // the session's record in host memory
     int tsdf_type, weight_type;
     int sid;                 // index in the context's table
     // VS_INTEGRATE_COLOR sessions (integ_mode 1); null otherwise

@@ -797,6 +797,21 @@ __device__ void set_pose_derived(const SessParams &P, SessState *st) {
     st->cos_max = (s < 1.0f) ? sqrtf(1.0f - s * s) : -2.0f;
 }
 
+// The session's record in host memory (HostState), by one thread; visible to
+// the host once it has waited for the stream. A pose read back by a 128-byte
+// device-to-host copy cost ~20 us of the host's time (64-session step with the
+// poses read back 7.90 -> 6.67 ms, 640x480 scan with preview 463 -> 440 us,
+// 8 of 24 server slots 1.34 -> 1.21 ms).
+__device__ __forceinline__ void publish_host(const SessParams &P, const SessState *st) {
+    HostState *h = P.host;
+    if (!h) return;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) stg(h->T_gc, k, st->T_gc[k]);
+    stg(&h->last_status, 0, st->last_status);
+    stg(&h->frames, 0, st->frames);
+    stg(&h->solves, 0, st->solves);
+}
+
 __device__ double rotation_deg(const double *T) {
     double c = (T[0] + T[5] + T[10] - 1.0) * 0.5;
     c = fmax(-1.0, fmin(1.0, c));
@@ -825,6 +840,7 @@ __device__ __forceinline__ void track_finalize(const SessParams &P, SessState *s
     st->last_status = status;
     st->fuse_ok = (status == 0);
     if (status == 0) st->frames += 1;
+    publish_host(P, st);
 }
 __global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -861,7 +877,10 @@ __global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *_
 
 // Pose set from the host: derived copies only.
 __global__ void k_pose_derived(const SessParams *__restrict__ SP) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) set_pose_derived(SP[0], SP[0].st);
+    if (threadIdx.x == 0 && blockIdx.x == 0) {
+        set_pose_derived(SP[0], SP[0].st);
+        publish_host(SP[0], SP[0].st);
+    }
 }
 
 // Normal equations of one iteration without a solve (diagnostics/parity).

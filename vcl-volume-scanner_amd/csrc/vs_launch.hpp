@@ -40,8 +40,8 @@ void launch_icp_iter(const SessParams *P, const WorkItem *work, int n, int nsess
 void launch_track_finalize(const SessParams *P, int nsess, hipStream_t s);
 // The one-launch form of an iteration, for launches of up to kIcpStepGroups
 // level-0 groups, a CU each for their 16-wave workgroups. Fused frame with
-// preview, two launches / one: 38 groups (320x240) 443 / 395 us, 150
-// (640x480) 509 / 455, 136 with colour 550 / 495; beyond it, 600 groups
+// preview, two launches / one: 38 groups (320x240) 443 / 398 us, 150
+// (640x480) 509 / 463, 136 with colour 550 / 506; beyond it, 600 groups
 // (1280x960) 1125 / 1246 and a 24-slot server's 2291 1295 / 1359 (these two
 // with a shorter solve on both sides).
 constexpr int kIcpStepGroups = VS_ICP_STEP_GROUPS;
