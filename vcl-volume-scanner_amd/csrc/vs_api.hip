@@ -26,7 +26,6 @@ void launch_track_setup_forced(const SessParams *P, int nsess, const double *T_i
 void launch_pose_derived(const SessParams *P, hipStream_t s);
 void launch_raycast_stats(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt,
                           unsigned long long *stats, hipStream_t s);
-void launch_fuse_ok(const SessParams *P, int nsess, hipStream_t s);
 }  // namespace vs
 
 using namespace vs;
@@ -782,9 +781,9 @@ void enqueue_track(const Batch &B, hipStream_t s) {
                 launch_icp_iter(B.dP, B.dGroup[l], B.nGroup[l], B.n, l, it, s);
         }
     if (one)
-        launch_icp_finish(B.dP, B.n, s);
+        launch_icp_finish(B.dP, B.n, B.bl.count, s);
     else
-        launch_track_finalize(B.dP, B.n, s);
+        launch_track_finalize(B.dP, B.n, B.bl.count, s);
 }
 
 // The per-frame launch sequence of a batch (so_Scan_Object order).
@@ -797,14 +796,13 @@ void enqueue_step(const Batch &B, hipStream_t s, Timer *timed) {
         launch_track_setup_active(B.dP, B.n, B.active, s);
     else
         launch_track_setup(B.dP, B.n, nullptr, s);
-    launch_bilateral(B.dP, B.dWork[0], B.nWork[0], s);
+    launch_bilateral(B.dP, B.dWork[0], B.nWork[0], 0, nullptr, s);
     mark(1);
-    for (int l = 1; l < B.levels; ++l) launch_pyr_down(B.dP, B.dWork[l], B.nWork[l], l, s);
+    for (int l = 1; l < B.levels; ++l) launch_pyr_down(B.dP, B.dWork[l], B.nWork[l], l, 0, s);
     mark(2);
     enqueue_track(B, s);
     mark(3);
-    launch_vis_clear(B.dP, B.n, B.bl, s);
-    launch_vis_mark(B.dP, B.dWork[0], B.nWork[0], B.n, B.max_words, B.bl, s);
+    launch_vis_mark(B.dP, B.dWork[0], B.nWork[0], B.n, B.max_words, B.bl, 0, s);
     mark(4);
     launch_integrate(B.dP, B.n, B.bl, B.tt, B.wt, integ_grid(B), B.sd_slices, s);
     mark(5);
@@ -1522,8 +1520,7 @@ vs_status vs_set_depth(vs_session *s, const uint16_t *depth_mm, int is_host, vs_
 vs_status vs_bilateral(vs_session *s, vs_stream stream) {
     if (!s) return fail(VS_EINVAL, "null session");
     hipStream_t h = pick(s, stream);
-    launch_fuse_ok(s->self.dP, 1, h);
-    launch_bilateral(s->self.dP, s->self.dWork[0], s->self.nWork[0], h);
+    launch_bilateral(s->self.dP, s->self.dWork[0], s->self.nWork[0], 1, nullptr, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }
@@ -1534,20 +1531,15 @@ vs_status vs_bilateral_filter_depth(vs_session *s, const void *depth_in, int in_
     hipStream_t h = pick(s, stream);
     vs_status r = copy_depth(s, depth_in, in_is_host, h);
     if (r != VS_OK) return r;
-    launch_fuse_ok(s->self.dP, 1, h);
-    launch_bilateral(s->self.dP, s->self.dWork[0], s->self.nWork[0], h);
+    launch_bilateral(s->self.dP, s->self.dWork[0], s->self.nWork[0], 1, depth_out_dev, h);
     HIP_TRY(hipGetLastError());
-    if (depth_out_dev)
-        HIP_TRY(hipMemcpyAsync(depth_out_dev, s->hp.filt[0], (size_t)s->d.width * s->d.height * 4,
-                               hipMemcpyDeviceToDevice, h));
     return VS_OK;
 }
 
 vs_status vs_pyramid(vs_session *s, vs_stream stream) {
     if (!s) return fail(VS_EINVAL, "null session");
     hipStream_t h = pick(s, stream);
-    launch_fuse_ok(s->self.dP, 1, h);
-    for (int l = 1; l < s->d.levels; ++l) launch_pyr_down(s->self.dP, s->self.dWork[l], s->self.nWork[l], l, h);
+    for (int l = 1; l < s->d.levels; ++l) launch_pyr_down(s->self.dP, s->self.dWork[l], s->self.nWork[l], l, 1, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }
@@ -1587,9 +1579,8 @@ vs_status vs_integrate(vs_session *s, vs_stream stream) {
     if (!s) return fail(VS_EINVAL, "null session");
     hipStream_t h = pick(s, stream);
     const Batch &B = s->self;
-    launch_fuse_ok(B.dP, 1, h);
-    launch_vis_clear(B.dP, 1, B.bl, h);
-    launch_vis_mark(B.dP, B.dWork[0], B.nWork[0], 1, B.max_words, B.bl, h);
+    launch_integrate_begin(B.dP, B.bl.count, h);
+    launch_vis_mark(B.dP, B.dWork[0], B.nWork[0], 1, B.max_words, B.bl, 1, h);
     launch_integrate(B.dP, B.n, B.bl, B.tt, B.wt, integ_grid(B), B.sd_slices, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
@@ -1604,24 +1595,18 @@ vs_status vs_integrate_depth(vs_session *s, const void *depth_dev, vs_stream str
 
 vs_status vs_render_maps(vs_session *s, int level, float *depth_dev, float *vtx_dev, float *nrm_dev,
                          uint8_t *img_dev, vs_stream stream) {
-    vs_status r = vs_raycast(s, level, stream);
-    if (r != VS_OK) return r;
-    const size_t npx = (size_t)(s->d.width >> level) * (s->d.height >> level);
-    if (depth_dev || vtx_dev || nrm_dev || img_dev)
-        launch_maps_out(s->self.dP, level, npx, depth_dev, vtx_dev, nrm_dev, img_dev, s->last);
+    if (!s) return fail(VS_EINVAL, "null session");
+    if (level < 0 || level >= s->d.levels) return fail(VS_EINVAL, "level %d", level);
+    const Batch &B = s->self;
+    const MapsOut out{depth_dev, vtx_dev, nrm_dev, img_dev};
+    launch_raycast(B.dP, B.dWork[level], B.nWork[level], level, B.tt, B.wt, B.addr,
+                   depth_dev || vtx_dev || nrm_dev || img_dev ? &out : nullptr, pick(s, stream));
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }
 
 vs_status vs_raycast(vs_session *s, int level, vs_stream stream) {
-    if (!s) return fail(VS_EINVAL, "null session");
-    if (level < 0 || level >= s->d.levels) return fail(VS_EINVAL, "level %d", level);
-    hipStream_t h = pick(s, stream);
-    const Batch &B = s->self;
-    launch_fuse_ok(B.dP, 1, h);
-    launch_raycast(B.dP, B.dWork[level], B.nWork[level], level, B.tt, B.wt, B.addr, h);
-    HIP_TRY(hipGetLastError());
-    return VS_OK;
+    return vs_render_maps(s, level, nullptr, nullptr, nullptr, nullptr, stream);
 }
 
 vs_status vs_fuse_frame(vs_session *s, const uint16_t *depth_mm, int is_host, vs_stream stream) {
@@ -2237,7 +2222,6 @@ vs_status vs_raycast_counts(vs_session *s, int level, unsigned long long counts[
     unsigned long long *d = (unsigned long long *)(s->mem + s->L.stats);
     HIP_TRY(hipMemset(d, 0, 64));
     const Batch &B = s->self;
-    launch_fuse_ok(B.dP, 1, s->stream);
     launch_raycast_stats(B.dP, B.dWork[level], B.nWork[level], level, B.tt, B.wt, d, s->stream);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(s->stream));

@@ -842,8 +842,24 @@ __device__ __forceinline__ void track_finalize(const SessParams &P, SessState *s
     if (status == 0) st->frames += 1;
     publish_host(P, st);
 }
-__global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess) {
+// What the step's integration counts from zero: the batch's brick list (by the
+// launch's first thread), a session's visible bricks and updated voxels, and
+// whether it gained a band superbrick (every kernel that reads that flag runs
+// after the integration that sets it and before the next reset).
+__device__ __forceinline__ void integrate_begin(SessState *st) {
+    st->vis_count = 0u;
+    st->upd_count = 0ull;
+    st->sdist_dirty = 0;
+}
+__global__ void k_integrate_begin(const SessParams *__restrict__ SP, unsigned *bricks) {
+    if (threadIdx.x != 0) return;
+    *bricks = 0u;
+    SP[0].st->active = 1;
+    integrate_begin(SP[0].st);
+}
+__global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess, unsigned *bricks) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) *bricks = 0u;
     if (s >= nsess) return;
     const SessParams &P = SP[s];
     SessState *st = P.st;
@@ -851,12 +867,14 @@ __global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess) {
         st->fuse_ok = 0;
         return;
     }
+    integrate_begin(st);
     track_finalize(P, st);
 }
 // The same after the one-launch iterations: one workgroup per session solves
 // the last one first.
-__global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *__restrict__ SP, int nsess) {
+__global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *__restrict__ SP, unsigned *bricks) {
     __shared__ StepShared sh;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *bricks = 0u;
     const SessParams &P = SP[blockIdx.x];
     SessState *st = P.st;
     if (!st->active) {
@@ -872,7 +890,10 @@ __global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *_
             st->solves = sh.solves;
         }
     }
-    if (threadIdx.x == 0) track_finalize(P, st);
+    if (threadIdx.x == 0) {
+        integrate_begin(st);
+        track_finalize(P, st);
+    }
 }
 
 // Pose set from the host: derived copies only.
@@ -905,18 +926,6 @@ __global__ __launch_bounds__(kTileThreads) void k_icp_system(const SessParams *_
     add_terms(ok, A, b, v);
     block_terms(v, red64);
     if (threadIdx.x < kIcpVals) out_part[(size_t)wi.tile * kIcpVals + threadIdx.x] = red64[threadIdx.x];
-}
-
-// Standalone integrate/raycast calls always run: mark the frame fusable.
-__global__ void k_fuse_ok(const SessParams *__restrict__ SP, int nsess) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < nsess) {
-        SP[s].st->fuse_ok = 1;
-        SP[s].st->active = 1;
-    }
-}
-void launch_fuse_ok(const SessParams *P, int nsess, hipStream_t s) {
-    hipLaunchKernelGGL(k_fuse_ok, dim3((nsess + 63) / 64), dim3(64), 0, s, P, nsess);
 }
 
 void launch_track_setup(const SessParams *P, int nsess, const double *T_init, hipStream_t s) {
@@ -988,11 +997,14 @@ void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level
         hipLaunchKernelGGL(k_icp_step<icp_group(2)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq);
 #endif
 }
-void launch_icp_finish(const SessParams *P, int nsess, hipStream_t s) {
-    hipLaunchKernelGGL(k_icp_finish, dim3(nsess), dim3(kStepThreads), 0, s, P, nsess);
+void launch_icp_finish(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s) {
+    hipLaunchKernelGGL(k_icp_finish, dim3(nsess), dim3(kStepThreads), 0, s, P, bricks);
 }
-void launch_track_finalize(const SessParams *P, int nsess, hipStream_t s) {
-    hipLaunchKernelGGL(k_track_finalize, dim3((nsess + 63) / 64), dim3(64), 0, s, P, nsess);
+void launch_track_finalize(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s) {
+    hipLaunchKernelGGL(k_track_finalize, dim3((nsess + 63) / 64), dim3(64), 0, s, P, nsess, bricks);
+}
+void launch_integrate_begin(const SessParams *P, unsigned *bricks, hipStream_t s) {
+    hipLaunchKernelGGL(k_integrate_begin, dim3(1), dim3(64), 0, s, P, bricks);
 }
 void launch_pose_derived(const SessParams *P, hipStream_t s) {
     hipLaunchKernelGGL(k_pose_derived, dim3(1), dim3(64), 0, s, P);

@@ -43,12 +43,13 @@ __device__ __forceinline__ void bil_window(const float (*tile)[TW], int cy, int 
 // the centre value (c + sum w (d - c) / sum w), which is the same weighted mean
 // with a smaller rounding error.
 __global__ __launch_bounds__(kTileThreads) void k_bilateral(const SessParams *__restrict__ SP,
-                                                            const WorkItem *__restrict__ work) {
+                                                            const WorkItem *__restrict__ work, int force,
+                                                            float *out) {
     __shared__ float tile[kTileH + 2 * kHalo][kTileW + 2 * kHalo];
     const WorkItem wi = work[blockIdx.x];
     const SessParams &P = SP[wi.sess];
     const LevelDesc &L = P.lev[0];
-    if (tile_out(L, wi.tile) || !P.st->active) return;
+    if (tile_out(L, wi.tile) || !(force || P.st->active)) return;
     const int W = L.W, H = L.H;
     const int x0 = (wi.tile % L.tiles_x) * kTileW, y0 = (wi.tile / L.tiles_x) * kTileH;
     const int R = P.bil_radius;
@@ -68,20 +69,24 @@ __global__ __launch_bounds__(kTileThreads) void k_bilateral(const SessParams *__
     bool zero = false;
     const float nk = P.bil_nk;
     const int cy = ly + kHalo, cx = lx + kHalo;
+    const auto store = [&](float v) {
+        stg(P.filt[0], (size_t)y * W + x, v);
+        if (out) stg(out, (size_t)y * W + x, v);
+    };
     // session creation accepts radii 1..3 only; each radius has its own
     // complete path to the store
     switch (R) {
     case 1:
         bil_window<1, TW>(tile, cy, cx, P.bil_w, c, nk, s, t, zero);
-        stg(P.filt[0], (size_t)y * W + x, zero ? 0.0f : c + t / s);
+        store(zero ? 0.0f : c + t / s);
         break;
     case 2:
         bil_window<2, TW>(tile, cy, cx, P.bil_w, c, nk, s, t, zero);
-        stg(P.filt[0], (size_t)y * W + x, zero ? 0.0f : c + t / s);
+        store(zero ? 0.0f : c + t / s);
         break;
     case 3:
         bil_window<3, TW>(tile, cy, cx, P.bil_w, c, nk, s, t, zero);
-        stg(P.filt[0], (size_t)y * W + x, zero ? 0.0f : c + t / s);
+        store(zero ? 0.0f : c + t / s);
         break;
     }
 }
@@ -92,11 +97,11 @@ __global__ __launch_bounds__(kTileThreads) void k_bilateral(const SessParams *__
 // (z_yooji_image_processor.cpp:368-407, 857-940, 567-596). Only the decimated
 // pixels are computed.
 __global__ __launch_bounds__(kTileThreads) void k_pyr_down(const SessParams *__restrict__ SP,
-                                                           const WorkItem *__restrict__ work, int l) {
+                                                           const WorkItem *__restrict__ work, int l, int force) {
     const WorkItem wi = work[blockIdx.x];
     const SessParams &P = SP[wi.sess];
     const LevelDesc &L = P.lev[l];
-    if (l >= P.levels || tile_out(L, wi.tile) || !P.st->active) return;
+    if (l >= P.levels || tile_out(L, wi.tile) || !(force || P.st->active)) return;
     const int Wi = P.lev[l - 1].W, Hi = P.lev[l - 1].H;
     const int x = (wi.tile % L.tiles_x) * kTileW + threadIdx.x % kTileW;
     const int y = (wi.tile / L.tiles_x) * kTileH + threadIdx.x / kTileW;
@@ -316,11 +321,11 @@ void launch_gather_depth(const SessParams *P, const DepthChunk &ch, hipStream_t 
     if (ch.n > 0) hipLaunchKernelGGL(k_gather_depth, dim3(64, ch.n), dim3(256), 0, s, P, ch);
 }
 
-void launch_bilateral(const SessParams *P, const WorkItem *work, int n, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_bilateral, dim3(n), dim3(kTileThreads), 0, s, P, work);
+void launch_bilateral(const SessParams *P, const WorkItem *work, int n, int force, float *out, hipStream_t s) {
+    if (n > 0) hipLaunchKernelGGL(k_bilateral, dim3(n), dim3(kTileThreads), 0, s, P, work, force, out);
 }
-void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int l, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_pyr_down, dim3(n), dim3(kTileThreads), 0, s, P, work, l);
+void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int l, int force, hipStream_t s) {
+    if (n > 0) hipLaunchKernelGGL(k_pyr_down, dim3(n), dim3(kTileThreads), 0, s, P, work, l, force);
 }
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int l, float *vtx, float *nrm, hipStream_t s) {
     if (n > 0)

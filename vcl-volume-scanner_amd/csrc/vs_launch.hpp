@@ -20,8 +20,11 @@ struct DepthChunk {  // passed by value: device frame pointers and the batch slo
 void launch_gather_depth(const SessParams *P, const DepthChunk &ch, hipStream_t s);
 // n 32-bit words at p set to v
 void launch_fill_u32(uint32_t *p, size_t n, uint32_t v, hipStream_t s);
-void launch_bilateral(const SessParams *P, const WorkItem *work, int n, hipStream_t s);
-void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int level, hipStream_t s);
+// force (here and below): run also for sessions whose state does not have a
+// frame in a step (the single operators)
+// out (nullable, single session): the filtered frame also goes there
+void launch_bilateral(const SessParams *P, const WorkItem *work, int n, int force, float *out, hipStream_t s);
+void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int level, int force, hipStream_t s);
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int level, float *vtx, float *nrm, hipStream_t s);
 // single session (P[0]), the reference loop's in-place order; bits: vn_words(W)
 // * H words of scratch
@@ -37,7 +40,9 @@ void launch_track_setup_active(const SessParams *P, int nsess, const int *active
 void launch_set_active(int *active, int nslots, const uint32_t bits[kMaxSlots / 32], hipStream_t s);
 void launch_icp_iter(const SessParams *P, const WorkItem *work, int n, int nsess, int level, int iter,
                      hipStream_t s);
-void launch_track_finalize(const SessParams *P, int nsess, hipStream_t s);
+// bricks: the step's brick counter; this launch and launch_icp_finish also
+// reset it and the sessions' integrate counters (integrate_begin)
+void launch_track_finalize(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s);
 // The one-launch form of an iteration, for launches of up to kIcpStepGroups
 // level-0 groups, a CU each for their 16-wave workgroups. Fused frame with
 // preview, two launches / one: 38 groups (320x240) 443 / 398 us, 150
@@ -48,7 +53,9 @@ constexpr int kIcpStepGroups = VS_ICP_STEP_GROUPS;
 // seq: 1, 2, ... over the launches of one track
 void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level, int iter, int seq, hipStream_t s);
 // the last iteration's solve, then launch_track_finalize's work
-void launch_icp_finish(const SessParams *P, int nsess, hipStream_t s);
+void launch_icp_finish(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s);
+// integrate_begin alone, for an integration without a track (single session)
+void launch_integrate_begin(const SessParams *P, unsigned *bricks, hipStream_t s);
 // one system, no solve: writes 29 doubles (+ optional mask) for diagnostics
 void launch_icp_system(const SessParams *P, const WorkItem *work, int n, int level, const float *T21,
                        double *out_part, uint8_t *mask, hipStream_t s);
@@ -61,11 +68,10 @@ struct BrickList {
     unsigned *count;    // device counter
     unsigned capacity;
 };
-void launch_vis_clear(const SessParams *P, int nsess, BrickList bl, hipStream_t s);
 // marks the visible bricks' bits, then compacts every session's bits into
 // the brick list (max_words: the longest bitmap of the nsess sessions)
 void launch_vis_mark(const SessParams *P, const WorkItem *work, int n, int nsess, uint32_t max_words, BrickList bl,
-                     hipStream_t s);
+                     int force, hipStream_t s);
 // sd_slices: the most superbricks along z of any session (distance field)
 void launch_integrate(const SessParams *P, int nsess, BrickList bl, int tsdf_type, int weight_type, int grid,
                       int sd_slices, hipStream_t s);
@@ -75,12 +81,14 @@ void launch_integrate(const SessParams *P, int nsess, BrickList bl, int tsdf_typ
 // records are at most 1 GB). The form for mixed and large grids reads the
 // superbrick size per session.
 enum VoxAddr { kAddrSmall = 0, kAddr32 = 1, kAddr64 = 2 };
+// Caller buffers of a single session's maps at one level (each nullable):
+// depth, vertex and normal (3 floats per pixel), image.
+struct MapsOut {
+    float *depth, *vtx, *nrm;
+    uint8_t *img;
+};
 void launch_raycast(const SessParams *P, const WorkItem *work, int n, int level, int tsdf_type, int weight_type,
-                    int addr, hipStream_t s);
-// a single session's model maps of `level` (npx pixels) into caller buffers
-// (each nullable): depth, vertex and normal (3 floats per pixel), image
-void launch_maps_out(const SessParams *P, int level, size_t npx, float *depth, float *vtx, float *nrm, uint8_t *img,
-                     hipStream_t s);
+                    int addr, const MapsOut *out, hipStream_t s);
 // Several pyramid levels in one launch: segment k of the grid is level
 // level[k]'s work list (passed by value).
 struct LevelWork {
@@ -88,6 +96,7 @@ struct LevelWork {
     int n[kMaxLevels];
     int level[kMaxLevels];
     int nseg;
+    int force;
     int blocks() const {
         int t = 0;
         for (int k = 0; k < nseg; ++k) t += n[k];

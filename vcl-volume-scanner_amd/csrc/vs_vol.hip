@@ -23,41 +23,23 @@ namespace vs {
 // ---------------------------------------------------------------------------
 // A13: visible bricks (g_fvsc_Find_Visible_Sub_Cubes, volume_integrator.cu:84-152)
 // ---------------------------------------------------------------------------
-// Clears the list counter and, for every session that fuses this frame, its
-// visible-brick flags.
-__global__ void k_vis_clear(const SessParams *__restrict__ SP, int nsess, BrickList bl) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *bl.count = 0u;
-    const int s = blockIdx.y;
-    if (s >= nsess) return;
-    const SessParams &P = SP[s];
-    if (!P.st->active) return;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        P.st->vis_count = 0u;
-        P.st->upd_count = 0ull;
-    }
-    if (!P.st->fuse_ok) return;
-    const uint32_t nb = (uint32_t)P.bdim[0] * P.bdim[1] * P.bdim[2];
-    const uint32_t n16 = (nb + 127) / 128 * 8;  // 16-byte words of the padded flags
-    for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < n16; w += gridDim.x * blockDim.x)
-        stg((vs_u4 *)P.vmask, w, vs_u4{0u, 0u, 0u, 0u});
-}
-
 // Flags the bricks hit by the samples p + n*mu*dir, n = -4..1, of every valid
 // pixel's ray: one byte per brick, set to 1 by plain stores (the reference's
 // bool mask), so the bricks that many pixels hit need neither atomics nor a
 // deduplication pass; a lane whose brick equals its left neighbour's for the
 // same sample leaves the store to that lane (runs of ~10 neighbouring pixels
 // share a brick). The brick list and the visible-brick bits are built from
-// the flags by k_vis_list. (A device-scope atomic per new brick on a bitmap,
+// the flags by k_vis_list, which leaves them cleared for the next frame. (A
+// device-scope atomic per new brick on a bitmap,
 // and a returning atomic on one list counter per image tile, had cost this
 // launch most of its time.)
 __global__ __launch_bounds__(kTileThreads) void k_vis_mark(const SessParams *__restrict__ SP,
-                                                           const WorkItem *__restrict__ work) {
+                                                           const WorkItem *__restrict__ work, int force) {
     const WorkItem wi = work[blockIdx.x];
     const SessParams &P = SP[wi.sess];
     SessState *st = P.st;
     const LevelDesc &L = P.lev[0];
-    if (!st->fuse_ok || tile_out(L, wi.tile)) return;
+    if (!(force || st->fuse_ok) || tile_out(L, wi.tile)) return;
     const int x = (wi.tile % L.tiles_x) * kTileW + threadIdx.x % kTileW;
     const int y = (wi.tile / L.tiles_x) * kTileH + threadIdx.x / kTileW;
     const float td = (x < L.W && y < L.H) ? raw_depth(P, (size_t)y * L.W + x) : 0.0f;
@@ -94,7 +76,8 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_mark(const SessParams *__r
 // Turns the sessions' visible-brick flags into the visible-brick bits and
 // the batch's brick list. Workgroup (c, s) takes bricks [c, c + 1) *
 // kVisListBricks of session s: each thread packs the flags of 128
-// consecutive bricks (eight 16-byte loads) into 4 bit words and stores them,
+// consecutive bricks (eight 16-byte loads) into 4 bit words and stores them
+// (clearing the flags it found set),
 // then the workgroup ranks the set bits (popcounts and a prefix sum),
 // reserves their range with one atomic on the list counter (8 workgroups for
 // a 512^3 session) and writes (session, brick) in brick order, each thread
@@ -102,22 +85,26 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_mark(const SessParams *__r
 constexpr int kVisListWordsPerThread = 4;
 constexpr uint32_t kVisListBricks = 32u * kVisListWordsPerThread * kTileThreads;
 
-__global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__restrict__ SP, BrickList bl) {
+__global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__restrict__ SP, BrickList bl, int force) {
     __shared__ unsigned wsum[kTileThreads / 64];
     __shared__ unsigned base;
     const int sess = blockIdx.y;
     const SessParams &P = SP[sess];
     SessState *st = P.st;
-    if (!ldg(&st->fuse_ok, 0)) return;
+    if (!(force || ldg(&st->fuse_ok, 0))) return;
     const uint32_t nb = (uint32_t)P.bdim[0] * P.bdim[1] * P.bdim[2], nw = (nb + 31) / 32;
     const uint32_t b0 = blockIdx.x * kVisListBricks + threadIdx.x * (32u * kVisListWordsPerThread);
     if (blockIdx.x * kVisListBricks >= nb) return;
     uint32_t w[kVisListWordsPerThread] = {0u, 0u, 0u, 0u};
     if (b0 < nb) {  // flags padded to 128 bricks: the 128 read here are in the buffer
-        const vs_u4 *f = (const vs_u4 *)(P.vmask + b0);
+        vs_u4 *f = (vs_u4 *)(P.vmask + b0);
+        vs_u4 fl[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) fl[q] = ldg(f, q);
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-            const vs_u4 v = ldg(f, q);
+            const vs_u4 v = fl[q];
+            if (v.x | v.y | v.z | v.w) stg(f, q, vs_u4{0u, 0u, 0u, 0u});
             const uint32_t e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -450,14 +437,14 @@ __global__ __launch_bounds__(kTileThreads) void k_integrate(const SessParams *__
 // does x and y in LDS and leaves one byte per superbrick in the session's
 // scratch; pass 2, one per (session, 2048 superbricks), does z from the
 // scratch and packs two cells per byte of the field (byte-aligned chunks, so
-// no two workgroups write one byte); pass 3 clears the rebuild flags, which
-// every workgroup of passes 1 and 2 has read by then.
+// no two workgroups write one byte). The rebuild flags are cleared before the
+// next integration (integrate_begin).
 // ---------------------------------------------------------------------------
 constexpr int kSdistThreads = 1024, kSdistChunk = 2 * kSdistThreads;
 
 __device__ __forceinline__ bool sdist_todo(const SessParams &P, int force) {
     const int n = P.sdim[0] * P.sdim[1] * P.sdim[2];
-    return n > 0 && (force || ldg(&P.st->sdist_dirty, 0));
+    return n > 0 && (force || (ldg(&P.st->active, 0) && ldg(&P.st->sdist_dirty, 0)));
 }
 
 // min of rd(c) and, over 0 < |t| < kDistMax with pos + t in [0, len), of
@@ -508,16 +495,10 @@ __global__ __launch_bounds__(kSdistThreads) void k_sdist_z(const SessParams *__r
     stg(P.sdist, (size_t)(c0 >> 1), out);
 }
 
-__global__ void k_sdist_done(const SessParams *__restrict__ SP, int nsess) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < nsess) stg(&SP[s].st->sdist_dirty, 0, 0);
-}
-
 void launch_sdist(const SessParams *P, int nsess, int sd_slices, int force, hipStream_t s) {
     if (nsess <= 0 || sd_slices <= 0) return;
     hipLaunchKernelGGL(k_sdist_xy, dim3(nsess, sd_slices), dim3(kSdistThreads), 0, s, P, force);
     hipLaunchKernelGGL(k_sdist_z, dim3(nsess, kDistCells / kSdistChunk), dim3(kSdistThreads), 0, s, P, force);
-    hipLaunchKernelGGL(k_sdist_done, dim3((nsess + 255) / 256), dim3(256), 0, s, P, nsess);
 }
 
 // ---------------------------------------------------------------------------
@@ -1241,7 +1222,7 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(LA
     const SessParams &P = SP[wi.sess];
     const SessState *st = P.st;
     const LevelDesc &L = P.lev[level];
-    if (!st->fuse_ok || level >= P.levels || tile_out(L, wi.tile)) return;
+    if (!(lw.force || st->fuse_ok) || level >= P.levels || tile_out(L, wi.tile)) return;
     const int ncell = P.sdim[0] * P.sdim[1] * P.sdim[2];
     // four 16-byte loads per thread, issued together (the field's buffer is
     // padded to 256 bytes)
@@ -1303,6 +1284,18 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(LA
     }
 }
 
+// Pixel t of a level's maps in the caller's buffers, in the layout of
+// rmi_Render_Maps_for_ICP's outputs (z_yooji_cuda_tsdf_renderer.cu:1642-1656,
+// g_rmi :1069-1209): depth = camera z of the hit or 0, vertex and normal 3
+// floats per pixel (-100 for a miss), normal image one byte per pixel.
+__device__ __forceinline__ void put_maps(const MapsOut &o, size_t t, float vx, float vy, float vz, float nx, float ny,
+                                         float nz, uint8_t img) {
+    if (o.depth) stg(o.depth, t, vx == -100.0f ? 0.0f : vz);
+    if (o.vtx) stg3((MapXYZ *)o.vtx, t, vx, vy, vz);
+    if (o.nrm) stg3((MapXYZ *)o.nrm, t, nx, ny, nz);
+    if (o.img) stg(o.img, t, img);
+}
+
 // WV: the waves per SIMD the register allocation aims for (4: the compiler's
 // own choice, ~126 VGPRs with all 64 stencil loads in flight; 5: 91, fewer
 // loads in flight); the same results for each, so the autotuner picks. (6
@@ -1310,16 +1303,19 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(LA
 // or kAddr64; with the former the stencil's loads take 32-bit offsets from the array bases (every session
 // of the launch has its voxel records below 4 GB): 62 VGPRs instead of 101 at
 // WV 4, the same results.
-template <class TV, class TW, bool STATS, int RB, int WV, int AD>
+// OUT: the maps also go to the caller's buffers `mo` (single session, one
+// level); a launch of its own for that copy had cost a 3-level render 4 us a
+// level.
+template <class TV, class TW, bool STATS, int RB, int WV, int AD, bool OUT>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(WV == 4 ? 1 : WV, WV == 4 ? 8 : WV)))
 void k_raycast_shade(
-    const SessParams *__restrict__ SP, LevelWork lw, unsigned long long *stats) {
+    const SessParams *__restrict__ SP, LevelWork lw, unsigned long long *stats, MapsOut mo) {
     int level;
     const WorkItem wi = level_item(lw, level);
     const SessParams &P = SP[wi.sess];
     const SessState *st = P.st;
     const LevelDesc &L = P.lev[level];
-    if (!st->fuse_ok || level >= P.levels || tile_out(L, wi.tile)) return;
+    if (!(lw.force || st->fuse_ok) || level >= P.levels || tile_out(L, wi.tile)) return;
     int px, py;
     ray_pixel<RB>(threadIdx.x, px, py);
     const int x = (wi.tile % L.tiles_x) * kTileW + px;
@@ -1329,7 +1325,10 @@ void k_raycast_shade(
     // the march's output (it always runs just before): a world hit point,
     // or -100 for a miss, which is final already
     const MapXYZ h = ld_mvtx(P.mvn[level], t);
-    if (h.x == -100.0f) return;
+    if (h.x == -100.0f) {
+        if (OUT) put_maps(mo, t, -100.0f, -100.0f, -100.0f, -100.0f, -100.0f, -100.0f, 0);
+        return;
+    }
     const Vol<TV, TW, AD> V{P, P.vox, nullptr};
     const f3 p = {h.x, h.y, h.z};
     if (STATS) {
@@ -1348,7 +1347,9 @@ void k_raycast_shade(
         st_mnrm(P.mvn[level], t, nc.x, nc.y, nc.z);
         // light (0,0,-1): n.l = 0*nx + 0*ny - nz (z_yooji_object_scanner.cpp:1313)
         const float sa = nc.x * 0.0f + nc.y * 0.0f + nc.z * -1.0f;
-        stg(P.mimg[level], t, (uint8_t)(fmaxf(0.0f, fminf(255.0f, (0.8f * sa + 0.2f) * 255.0f))));
+        const uint8_t shade = (uint8_t)(fmaxf(0.0f, fminf(255.0f, (0.8f * sa + 0.2f) * 255.0f)));
+        stg(P.mimg[level], t, shade);
+        if (OUT) put_maps(mo, t, pc.x, pc.y, pc.z, nc.x, nc.y, nc.z, shade);
         if (P.mtex[level]) {
             f3 pv;
             world_to_voxel(P, p, pv);
@@ -1359,6 +1360,7 @@ void k_raycast_shade(
         st_mvtx(P.mvn[level], t, -100.0f, -100.0f, -100.0f);
         st_mnrm(P.mvn[level], t, -100.0f, -100.0f, -100.0f);
         stg(P.mimg[level], t, (uint8_t)0);
+        if (OUT) put_maps(mo, t, -100.0f, -100.0f, -100.0f, -100.0f, -100.0f, -100.0f, 0);
         if (P.mtex[level]) write_texture(P, level, t, 0u);
     }
 }
@@ -1380,6 +1382,9 @@ __global__ void k_volume_init(const SessParams *__restrict__ SP, size_t nvox, ui
         stg(P.bband, w, 0u);
         if (w < (size_t)P.sband_words) stg(P.sband, w, 0u);
     }
+    const size_t nflag = ((size_t)P.bdim[0] * P.bdim[1] * P.bdim[2] + 127) / 128 * 32;  // 32-bit words of the padded flags
+    for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < nflag; w += (size_t)gridDim.x * blockDim.x)
+        stg((uint32_t *)P.vmask, w, 0u);
 }
 
 __global__ void k_sband_clear(const SessParams *__restrict__ SP) {
@@ -1559,15 +1564,12 @@ __global__ __launch_bounds__(kTileThreads) void k_occupancy(const SessParams *__
 // ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
-void launch_vis_clear(const SessParams *P, int nsess, BrickList bl, hipStream_t s) {
-    hipLaunchKernelGGL(k_vis_clear, dim3(8, nsess), dim3(256), 0, s, P, nsess, bl);
-}
 void launch_vis_mark(const SessParams *P, const WorkItem *work, int n, int nsess, uint32_t max_words, BrickList bl,
-                     hipStream_t s) {
+                     int force, hipStream_t s) {
     if (n <= 0 || nsess <= 0 || max_words == 0) return;
-    hipLaunchKernelGGL(k_vis_mark, dim3(n), dim3(kTileThreads), 0, s, P, work);
+    hipLaunchKernelGGL(k_vis_mark, dim3(n), dim3(kTileThreads), 0, s, P, work, force);
     const uint32_t per = kVisListBricks / 32u;  // bitmap words per k_vis_list workgroup
-    hipLaunchKernelGGL(k_vis_list, dim3((max_words + per - 1) / per, nsess), dim3(kTileThreads), 0, s, P, bl);
+    hipLaunchKernelGGL(k_vis_list, dim3((max_words + per - 1) / per, nsess), dim3(kTileThreads), 0, s, P, bl, force);
 }
 
 #define VS_DISPATCH(tt, wt, FN, ...)                                                \
@@ -1628,20 +1630,29 @@ static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long
 }
 template <class TV, class TW>
 static void shade_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int waves,
-                    int addr, hipStream_t s) {
+                    int addr, const MapsOut *out, hipStream_t s) {
     const int n = lw.blocks();
     if (n <= 0) return;
+    if (out) {
+        if (addr != kAddr64)
+            hipLaunchKernelGGL((k_raycast_shade<TV, TW, false, kRay8x8, 4, kAddr32, true>), dim3(n), dim3(kTileThreads),
+                               0, s, P, lw, stats, *out);
+        else
+            hipLaunchKernelGGL((k_raycast_shade<TV, TW, false, kRay8x8, 4, kAddr64, true>), dim3(n), dim3(kTileThreads),
+                               0, s, P, lw, stats, *out);
+        return;
+    }
 #define VS_SHADE_A(RB_, WV_, AD_)                                                                              \
-    hipLaunchKernelGGL((k_raycast_shade<TV, TW, false, RB_, WV_, AD_>), dim3(n), dim3(kTileThreads), 0, s, P, lw, \
-                       stats)
+    hipLaunchKernelGGL((k_raycast_shade<TV, TW, false, RB_, WV_, AD_, false>), dim3(n), dim3(kTileThreads), 0, s, \
+                       P, lw, stats, MapsOut{})
 #define VS_SHADE(RB_, WV_)                                     \
     do {                                                       \
         if (addr != kAddr64) VS_SHADE_A(RB_, WV_, kAddr32);    \
         else VS_SHADE_A(RB_, WV_, kAddr64);                    \
     } while (0)
     if (stats)
-        hipLaunchKernelGGL((k_raycast_shade<TV, TW, true, kRay32x2, 4, kAddr64>), dim3(n), dim3(kTileThreads), 0, s, P,
-                           lw, stats);
+        hipLaunchKernelGGL((k_raycast_shade<TV, TW, true, kRay32x2, 4, kAddr64, false>), dim3(n), dim3(kTileThreads), 0, s, P,
+                           lw, stats, MapsOut{});
     else if (rb == kRay8x8 && waves == 5)
         VS_SHADE(kRay8x8, 5);
     else if (rb == kRay8x8)
@@ -1670,7 +1681,7 @@ void launch_raycast_march(const SessParams *P, const LevelWork &lw, int tt, int 
 }
 void launch_raycast_shade(const SessParams *P, const LevelWork &lw, int tt, int wt, unsigned long long *stats,
                           int rb, int waves, int addr, hipStream_t s) {
-    VS_DISPATCH(tt, wt, shade_t, P, lw, stats, rb, waves, addr, s);
+    VS_DISPATCH(tt, wt, shade_t, P, lw, stats, rb, waves, addr, (const MapsOut *)nullptr, s);
 }
 static LevelWork one_level(const WorkItem *work, int n, int level) {
     LevelWork lw{};
@@ -1679,14 +1690,15 @@ static LevelWork one_level(const WorkItem *work, int n, int level) {
         lw.n[0] = n;
         lw.level[0] = level;
         lw.nseg = 1;
+        lw.force = 1;
     }
     return lw;
 }
 void launch_raycast(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt, int addr,
-                    hipStream_t s) {
+                    const MapsOut *out, hipStream_t s) {
     const LevelWork lw = one_level(work, n, level);
     launch_raycast_march(P, lw, tt, wt, nullptr, kRay8x8, addr, s);
-    launch_raycast_shade(P, lw, tt, wt, nullptr, kRay8x8, 4, addr, s);
+    VS_DISPATCH(tt, wt, shade_t, P, lw, nullptr, kRay8x8, 4, addr, out, s);
 }
 void launch_raycast_stats(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt,
                           unsigned long long *stats, hipStream_t s) {
@@ -1741,39 +1753,6 @@ static void carve_t(const SessParams *P, const uint8_t *valid, unsigned *carved,
 }
 void launch_carve(const SessParams *P, int tt, int wt, const uint8_t *valid, unsigned *carved, hipStream_t s) {
     VS_DISPATCH(tt, wt, carve_t, P, valid, carved, s);
-}
-
-// The session's model maps of `level` written into caller buffers (any may be
-// null), in the layout of rmi_Render_Maps_for_ICP's outputs
-// (z_yooji_cuda_tsdf_renderer.cu:1642-1656, g_rmi :1069-1209): depth = camera
-// z of the hit or 0, vertex and normal 3 floats per pixel (-100 for a miss),
-// normal image one byte per pixel. Grid-stride over the pixels.
-__global__ __launch_bounds__(256) void k_maps_out(const SessParams *__restrict__ SP, int level, float *depth,
-                                                  float *vtx, float *nrm, uint8_t *img) {
-    const SessParams &P = SP[0];
-    const size_t n = (size_t)P.lev[level].W * P.lev[level].H;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
-        const MapXYZ v = ld_mvtx(P.mvn[level], i);
-        if (depth) stg(depth, i, v.x == -100.0f ? 0.0f : v.z);
-        if (vtx) {
-            stg(vtx, 3 * i, v.x);
-            stg(vtx, 3 * i + 1, v.y);
-            stg(vtx, 3 * i + 2, v.z);
-        }
-        if (nrm) {
-            const MapXYZ q = ld_mnrm(P.mvn[level], i);
-            stg(nrm, 3 * i, q.x);
-            stg(nrm, 3 * i + 1, q.y);
-            stg(nrm, 3 * i + 2, q.z);
-        }
-        if (img) stg(img, i, ldg(P.mimg[level], i));
-    }
-}
-void launch_maps_out(const SessParams *P, int level, size_t npx, float *depth, float *vtx, float *nrm, uint8_t *img,
-                     hipStream_t s) {
-    const size_t nb = (npx + 255) / 256;
-    const int g = (int)(nb < 1024 ? nb : 1024);
-    if (g > 0) hipLaunchKernelGGL(k_maps_out, dim3(g), dim3(256), 0, s, P, level, depth, vtx, nrm, img);
 }
 
 }  // namespace vs
