@@ -73,7 +73,7 @@ struct LevelDesc {
 // form of an iteration (k_icp_step): two records used in turn, the later one
 // (by seq) is current. Its group partials, not yet solved when pending >= 0,
 // are in the half of icp_part with the record's index.
-struct IcpStep {
+struct alignas(16) IcpStep {
     double T_12[16];
     int seq;         // launch that wrote the record (0: track setup, -1: never)
     int pending;     // level of the unsolved partials, -1 none

@@ -596,15 +596,19 @@ struct StepShared {
 // Brings the loop up to date into sh (all threads); returns the record it
 // started from. seq: only records of earlier launches count.
 __device__ __forceinline__ int step_resume(const SessParams &P, const SessState *st, int seq, StepShared &sh) {
-    const int s0 = ldg(&st->step[0].seq, 0), s1 = ldg(&st->step[1].seq, 0);
-    const int cur = (s1 < seq && (s0 >= seq || s1 > s0)) ? 1 : 0;
-    const IcpStep *S = &st->step[cur];
-    const int pending = ldg(&S->pending, 0);
-    if (threadIdx.x < 16) sh.T12[threadIdx.x] = ldg(S->T_12, threadIdx.x);
+    // both records at once: seq, pending, failed, conv_level; solves
+    const vs_u4 a0 = ldg((const vs_u4 *)&st->step[0].seq, 0), a1 = ldg((const vs_u4 *)&st->step[1].seq, 0);
+    const int n0 = ldg(&st->step[0].solves, 0), n1 = ldg(&st->step[1].solves, 0);
+    const double t0 = ldg(st->step[0].T_12, threadIdx.x & 15), t1 = ldg(st->step[1].T_12, threadIdx.x & 15);
+    const int s0 = (int)a0.x, s1 = (int)a1.x;
+    const int cur = (int)(s1 < seq) & ((int)(s0 >= seq) | (int)(s1 > s0));
+    const vs_u4 S = cur ? a1 : a0;
+    const int pending = (int)S.y;
+    if (threadIdx.x < 16) sh.T12[threadIdx.x] = cur ? t1 : t0;
     if (threadIdx.x == 16) {
-        sh.failed = ldg(&S->failed, 0);
-        sh.conv_level = ldg(&S->conv_level, 0);
-        sh.solves = ldg(&S->solves, 0);
+        sh.failed = (int)S.z;
+        sh.conv_level = (int)S.w;
+        sh.solves = cur ? n1 : n0;
     }
     if (pending >= 0) {
         const LevelDesc &L = P.lev[pending];
@@ -714,18 +718,19 @@ __global__ __launch_bounds__(kStepThreads) void k_icp_step(const SessParams *__r
                                                            const WorkItem *__restrict__ work, int level, int iter,
                                                            int seq) {
     __shared__ StepShared sh;
-    const WorkItem wi = work[blockIdx.x];
+    const WorkItem wi = work ? work[blockIdx.x] : WorkItem{0, (int)blockIdx.x};
     const SessParams &P = SP[wi.sess];
     SessState *st = P.st;
-    if (level >= P.levels || !ldg(&st->do_track, 0)) return;
+    if (level >= P.levels) return;
     const LevelDesc &L = P.lev[level];
     const int t0 = wi.tile * G;
     if (t0 >= L.tiles_x * L.tiles_y) return;
+    const int track = ldg(&st->do_track, 0), single = ldg(&st->force_single, 0);
     WidePixels<G> px;
     px.load(P, level, t0);  // in flight during the solve
+    if (!track) return;
     const int out = step_resume(P, st, seq, sh) ^ 1;
-    const bool skip = sh.failed || sh.conv_level == level || iter >= P.iters[level] ||
-                      (ldg(&st->force_single, 0) && level != 0);
+    const bool skip = sh.failed || sh.conv_level == level || iter >= P.iters[level] || (single && level != 0);
     if (wi.tile == 0) {
         IcpStep *S = &st->step[out];
         if (threadIdx.x < 16) stg(S->T_12, threadIdx.x, sh.T12[threadIdx.x]);
