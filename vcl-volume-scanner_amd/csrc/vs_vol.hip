@@ -75,17 +75,17 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_mark(const SessParams *__r
 
 // Turns the sessions' visible-brick flags into the visible-brick bits and
 // the batch's brick list. Workgroup (c, s) takes bricks [c, c + 1) *
-// kVisListBricks of session s: each thread packs the flags of 128
-// consecutive bricks (eight 16-byte loads) into 4 bit words and stores them
+// kVisListBricks of session s: each thread packs the flags of 32 * WPT
+// consecutive bricks (16-byte loads) into WPT bit words and stores them
 // (clearing the flags it found set),
 // then the workgroup ranks the set bits (popcounts and a prefix sum),
-// reserves their range with one atomic on the list counter (8 workgroups for
+// reserves their range with one atomic on the list counter (8 workgroups of WPT 4 for
 // a 512^3 session) and writes (session, brick) in brick order, each thread
 // its own bricks.
-constexpr int kVisListWordsPerThread = 4;
-constexpr uint32_t kVisListBricks = 32u * kVisListWordsPerThread * kTileThreads;
+template <int WPT>
 
 __global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__restrict__ SP, BrickList bl, int force) {
+    constexpr uint32_t kVisListBricks = 32u * WPT * kTileThreads;
     __shared__ unsigned wsum[kTileThreads / 64];
     __shared__ unsigned base;
     const int sess = blockIdx.y;
@@ -93,16 +93,16 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__r
     SessState *st = P.st;
     if (!(force || ldg(&st->fuse_ok, 0))) return;
     const uint32_t nb = (uint32_t)P.bdim[0] * P.bdim[1] * P.bdim[2], nw = (nb + 31) / 32;
-    const uint32_t b0 = blockIdx.x * kVisListBricks + threadIdx.x * (32u * kVisListWordsPerThread);
+    const uint32_t b0 = blockIdx.x * kVisListBricks + threadIdx.x * (32u * WPT);
     if (blockIdx.x * kVisListBricks >= nb) return;
-    uint32_t w[kVisListWordsPerThread] = {0u, 0u, 0u, 0u};
+    uint32_t w[WPT] = {};
     if (b0 < nb) {  // flags padded to 128 bricks: the 128 read here are in the buffer
         vs_u4 *f = (vs_u4 *)(P.vmask + b0);
-        vs_u4 fl[8];
+        vs_u4 fl[2 * WPT];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) fl[q] = ldg(f, q);
+        for (int q = 0; q < 2 * WPT; ++q) fl[q] = ldg(f, q);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < 2 * WPT; ++q) {
             const vs_u4 v = fl[q];
             if (v.x | v.y | v.z | v.w) stg(f, q, vs_u4{0u, 0u, 0u, 0u});
             const uint32_t e[4] = {v.x, v.y, v.z, v.w};
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__r
     const uint32_t w0 = b0 / 32u;
     unsigned c = 0;
 #pragma unroll
-    for (int k = 0; k < kVisListWordsPerThread; ++k) {
+    for (int k = 0; k < WPT; ++k) {
         if (w0 + k < nw) stg(P.bvis, w0 + k, w[k]);
         c += (unsigned)__popc(w[k]);
     }
@@ -144,7 +144,7 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__r
     __syncthreads();
     unsigned pos = base + before + inc - c;
 #pragma unroll
-    for (int k = 0; k < kVisListWordsPerThread; ++k) {
+    for (int k = 0; k < WPT; ++k) {
         uint32_t bits = w[k];
         while (bits) {
             const int j = __ffs(bits) - 1;
@@ -260,8 +260,8 @@ __device__ __forceinline__ void st_rec4(void *base, size_t i, const typename Vox
     }
 }
 
-// The integrate walks the brick list in chunks of kIntegChunk consecutive
-// entries. The list comes from k_vis_mark in (session, image tile) order, so
+// The integrate walks the brick list in chunks of up to kIntegChunk
+// consecutive entries. The list comes from k_vis_mark in (session, image tile) order, so
 // a chunk's bricks mostly belong to one session and lie behind one small
 // patch of its depth frame. Workgroup g runs on XCD g % 8 (workgroups are
 // dealt to the eight XCDs in turn), and the workgroups of one XCD take the
@@ -285,8 +285,13 @@ constexpr int kXcds = 8;
 template <class TV, class TW>
 __global__ __launch_bounds__(kTileThreads) void k_integrate(const SessParams *__restrict__ SP, BrickList bl) {
     const unsigned n = min(*bl.count, bl.capacity);
-    const unsigned nch = (n + kIntegChunk - 1) / kIntegChunk;
     const unsigned G = gridDim.x;
+    // entries per chunk: whole chunks of 8 while every workgroup gets some (the
+    // 24-slot server's 8 steps 1219 us, 1255 with chunks of 2), pairs for a lone
+    // session's short list, whose 8-entry chunks had left most CUs idle
+    // (603x451 colour scan 461 -> 439 us, 320x240 356 -> 353)
+    const unsigned ch = n >= 2 * G ? (unsigned)kIntegChunk : n >= G ? 4u : 2u;
+    const unsigned nch = (n + ch - 1) / ch;
     const unsigned nx = (G % kXcds == 0) ? kXcds : 1u;
     const unsigned xcd = blockIdx.x % nx, R = G / nx, r = blockIdx.x / nx;
     const unsigned c_lo = (unsigned)((unsigned long long)nch * xcd / nx);
@@ -306,8 +311,8 @@ __global__ __launch_bounds__(kTileThreads) void k_integrate(const SessParams *__
     int run_sess = -1;
     unsigned long long run_upd = 0ull;
     for (unsigned j = c_lo + r; j < c_hi; j += R) {
-        const unsigned b0 = j * kIntegChunk;
-        const int nb = (int)min((unsigned)kIntegChunk, n - b0);
+        const unsigned b0 = j * ch;
+        const int nb = (int)min(ch, n - b0);
         for (int k = half; k < nb; k += 2) {
             const int2 it = bl.items[b0 + k];
             const SessParams &P = SP[it.x];
@@ -1568,8 +1573,14 @@ void launch_vis_mark(const SessParams *P, const WorkItem *work, int n, int nsess
                      int force, hipStream_t s) {
     if (n <= 0 || nsess <= 0 || max_words == 0) return;
     hipLaunchKernelGGL(k_vis_mark, dim3(n), dim3(kTileThreads), 0, s, P, work, force);
-    const uint32_t per = kVisListBricks / 32u;  // bitmap words per k_vis_list workgroup
-    hipLaunchKernelGGL(k_vis_list, dim3((max_words + per - 1) / per, nsess), dim3(kTileThreads), 0, s, P, bl, force);
+    // 32 bricks a thread while that keeps the launch small (a thread writes its
+    // bricks one after another, and one session's surface crosses few threads'
+    // ranges: 640x480 scan 423 -> 418 us), else 128 and a quarter of the atomics
+    const auto blocks = [&](uint32_t wpt) { return (max_words + wpt * kTileThreads - 1) / (wpt * kTileThreads); };
+    if (blocks(1) * (uint32_t)nsess <= 512u)
+        hipLaunchKernelGGL(k_vis_list<1>, dim3(blocks(1), nsess), dim3(kTileThreads), 0, s, P, bl, force);
+    else
+        hipLaunchKernelGGL(k_vis_list<4>, dim3(blocks(4), nsess), dim3(kTileThreads), 0, s, P, bl, force);
 }
 
 #define VS_DISPATCH(tt, wt, FN, ...)                                                \
