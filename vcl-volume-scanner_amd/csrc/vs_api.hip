@@ -23,7 +23,8 @@
 
 namespace vs {
 void launch_track_setup_forced(const SessParams *P, int nsess, const double *T_init, hipStream_t s);
-void launch_pose_derived(const SessParams *P, hipStream_t s);
+// T null: identity; frames (nullable): the frame count
+void launch_set_pose(const SessParams *P, const double *T, int reset, const int *frames, hipStream_t s);
 void launch_raycast_stats(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt,
                           unsigned long long *stats, hipStream_t s);
 }  // namespace vs
@@ -110,12 +111,23 @@ Layout make_layout(const vs_session_desc &d) {
     L.nswords = (L.nsuper + 31) / 32;
     const size_t sv = d.tsdf_type == VS_TSDF_F16 ? 2 : 4, sw = d.weight_type == VS_WEIGHT_U8 ? 1 : 4;
     L.state = take(sizeof(SessState));
+    // params, wtab and the work lists (the head of lists) are uploaded in one
+    // piece when the session is created
     L.params = take(sizeof(SessParams));
+    L.wtab = take((size_t)(d.vol_dim[0] + d.vol_dim[1] + d.vol_dim[2]) * 4);
+    for (int l = 0; l < kMaxLevels; ++l) L.tiles[l] = l < d.levels ? tiles_of(W >> l, H >> l) : 0;
+    {
+        size_t nt[kMaxLevels], ng[kMaxLevels];
+        for (int l = 0; l < kMaxLevels; ++l) {
+            nt[l] = (size_t)L.tiles[l];
+            ng[l] = (size_t)icp_groups(L.tiles[l], l);
+        }
+        L.lists = take(lists_bytes(nt, ng, L.nbricks));
+    }
     L.raw = take((size_t)W * H * (d.depth_units == VS_DEPTH_M_F32 ? 4 : 2));
     for (int l = 0; l < kMaxLevels; ++l) {
         const int Wl = W >> l, Hl = H >> l;
         const size_t n = (size_t)Wl * Hl;
-        L.tiles[l] = l < d.levels ? tiles_of(Wl, Hl) : 0;
         L.filt[l] = take(n * 4);
         L.mvn[l] = take((n + 1) * 2 * sizeof(MapXYZ));  // vertex + normal per pixel, one padding pixel
         L.mimg[l] = take(n);
@@ -136,17 +148,8 @@ Layout make_layout(const vs_session_desc &d) {
     L.icp_part = take((size_t)L.icp_half * 2 * 8);
     L.diag_part = take((size_t)L.tiles[0] * kIcpVals * 8);
     L.diag_mask = take((size_t)W * H);
-    {
-        size_t nt[kMaxLevels], ng[kMaxLevels];
-        for (int l = 0; l < kMaxLevels; ++l) {
-            nt[l] = (size_t)L.tiles[l];
-            ng[l] = (size_t)icp_groups(L.tiles[l], l);
-        }
-        L.lists = take(lists_bytes(nt, ng, L.nbricks));
-    }
     L.stats = take(64);
     L.keys = take((size_t)W * H * 4);  // depth reprojection z-buffer
-    L.wtab = take((size_t)(d.vol_dim[0] + d.vol_dim[1] + d.vol_dim[2]) * 4);
     if (d.integrate_mode == VS_INTEGRATE_COLOR) {
         L.vcol = take(L.nvox * 4);
         L.rgb = take((size_t)W * H * 3);
@@ -520,16 +523,20 @@ struct ListSet {
         HIP_TRY(hipMemset(B.bl.count, 0, 16));
         return settle(B, integ_max);
     }
-    // The same in stream order on h, from `stage` (pinned, head_bytes() long,
-    // not to be rewritten before the uploads have run).
-    vs_status place_async(Batch &B, char *mem, char *stage, hipStream_t h, int integ_max) const {
-        const size_t head = point(B, mem);
+    // The work lists of a batch that points at mem, at the same offsets of `host`
+    void copy_lists(const Batch &B, const char *mem, char *host) const {
         for (int l = 0; l < kMaxLevels; ++l) {
             if (!tile[l].empty())
-                std::memcpy(stage + ((char *)B.dWork[l] - mem), tile[l].data(), tile[l].size() * sizeof(WorkItem));
+                std::memcpy(host + ((char *)B.dWork[l] - mem), tile[l].data(), tile[l].size() * sizeof(WorkItem));
             if (!group[l].empty())
-                std::memcpy(stage + ((char *)B.dGroup[l] - mem), group[l].data(), group[l].size() * sizeof(WorkItem));
+                std::memcpy(host + ((char *)B.dGroup[l] - mem), group[l].data(), group[l].size() * sizeof(WorkItem));
         }
+    }
+    // The same as place in stream order on h, from `stage` (pinned, head_bytes()
+    // long, not to be rewritten before the uploads have run).
+    vs_status place_async(Batch &B, char *mem, char *stage, hipStream_t h, int integ_max) const {
+        const size_t head = point(B, mem);
+        copy_lists(B, mem, stage);
         std::memset(stage + head, 0, 16);
         HIP_TRY(hipMemcpyAsync(mem, stage, head, hipMemcpyHostToDevice, h));
         HIP_TRY(hipMemcpyAsync(B.bl.count, stage + head, 16, hipMemcpyHostToDevice, h));
@@ -1325,16 +1332,6 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
         P.wtab[0] = wt;
         P.wtab[1] = wt + d.vol_dim[0];
         P.wtab[2] = wt + d.vol_dim[0] + d.vol_dim[1];
-        // the same FP32 operations as the device would do (division, then
-        // addition, each rounded once; this file is built without contraction)
-        std::vector<float> h((size_t)d.vol_dim[0] + d.vol_dim[1] + d.vol_dim[2]);
-        size_t o = 0;
-        for (int a = 0; a < 3; ++a)
-            for (int i = 0; i < d.vol_dim[a]; ++i) {
-                volatile float q = ((float)i + 0.5f) / P.vox_inv;
-                h[o++] = q + P.origin[a];
-            }
-        HIP_TRY(hipMemcpy(wt, h.data(), h.size() * 4, hipMemcpyHostToDevice));
     }
     P.st = (SessState *)(m + L.state);
     P.host = s->host;
@@ -1354,26 +1351,30 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
     B.tt = d.tsdf_type;
     B.wt = d.weight_type;
     B.dP = (SessParams *)(m + L.params);
+    B.members = {s.get()};
     {
+        // parameters, voxel-centre coordinates and work lists in one upload
         ListSet ls;
         ls.add(0, s.get());
-        vs_status r = ls.place(B, m + L.lists, 2048);
+        const size_t head = ls.point(B, m + L.lists);
+        vs_status r = ls.settle(B, 2048);
         if (r != VS_OK) return r;
+        std::vector<char> up(L.lists + head - L.params);
+        std::memcpy(up.data(), &P, sizeof(P));
+        // the same FP32 operations as the device would do (division, then
+        // addition, each rounded once; this file is built without contraction)
+        float *wt = (float *)(up.data() + (L.wtab - L.params));
+        for (int a = 0; a < 3; ++a)
+            for (int i = 0; i < d.vol_dim[a]; ++i) {
+                volatile float q = ((float)i + 0.5f) / P.vox_inv;
+                *wt++ = q + P.origin[a];
+            }
+        ls.copy_lists(B, m + L.lists, up.data() + (L.lists - L.params));
+        HIP_TRY(hipMemcpy(m + L.params, up.data(), up.size(), hipMemcpyHostToDevice));
     }
-    B.members = {s.get()};
-    HIP_TRY(hipMemcpy(B.dP, &P, sizeof(P), hipMemcpyHostToDevice));
-    // state: pose, counters; volume F = 1, W = 0 (vs_session_reset); empty
-    // pyramid and images, model maps at the -100 sentinel; all on the
-    // session's stream (one wait at the end of set-up)
-    HIP_TRY(hipMemsetAsync(m + L.state, 0, sizeof(SessState), s->stream));
-    const uint32_t kMiss = 0xC2C80000u;  // -100.0f
-    for (int l = 0; l < kMaxLevels; ++l) {
-        const size_t n = (size_t)(d.width >> l) * (d.height >> l);
-        HIP_TRY(hipMemsetAsync(m + L.filt[l], 0, n * 4, s->stream));
-        HIP_TRY(hipMemsetAsync(m + L.mimg[l], 0, n, s->stream));
-        if (P.mtex[l]) HIP_TRY(hipMemsetAsync(P.mtex[l], 0, n * 3, s->stream));
-        launch_fill_u32((uint32_t *)(m + L.mvn[l]), (n + 1) * 6, kMiss, s->stream);
-    }
+    // empty pyramid and images, model maps at the sentinel; then state and
+    // volume (vs_session_reset), all on the session's stream
+    launch_session_init(B.dP, (size_t)d.width * d.height, s->stream);
     HIP_TRY(hipGetLastError());
     vs_session *raw = s.release();
     ctx->sessions.push_back(raw);
@@ -1382,7 +1383,6 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
         vs_session_destroy(raw);
         return r;
     }
-    HIP_TRY(hipStreamSynchronize(raw->stream));
     *out = raw;
     return VS_OK;
 }
@@ -1449,13 +1449,8 @@ vs_status vs_session_destroy(vs_session *s) {
 vs_status vs_session_reset(vs_session *s, const double T_gc0[16], vs_stream stream) {
     if (!s) return fail(VS_EINVAL, "null session");
     hipStream_t h = pick(s, stream);
-    launch_volume_init(s->self.dP, s->L.nvox, s->d.tsdf_type, s->d.weight_type, s->L.nwords, s->L.sdim[2], h);
-    SessState init{};
-    for (int k = 0; k < 16; ++k) init.T_gc[k] = T_gc0 ? T_gc0[k] : ((k % 5) == 0 ? 1.0 : 0.0);
-    init.conv_level = -1;
-    init.active = 1;
-    HIP_TRY(hipMemcpyAsync(s->st, &init, sizeof(init), hipMemcpyHostToDevice, h));
-    launch_pose_derived(s->self.dP, h);
+    launch_volume_init(s->self.dP, s->L.nvox, s->d.tsdf_type, s->d.weight_type, s->L.nwords, h);
+    launch_set_pose(s->self.dP, T_gc0, 1, nullptr, h);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(h));
     return VS_OK;
@@ -1734,9 +1729,7 @@ vs_status vs_get_pose(vs_session *s, double T_gc[16]) {
 vs_status vs_set_pose(vs_session *s, const double T_gc[16], vs_stream stream) {
     if (!s || !T_gc) return fail(VS_EINVAL, "null argument");
     hipStream_t h = pick(s, stream);
-    HIP_TRY(hipStreamSynchronize(h));
-    HIP_TRY(hipMemcpy(s->st->T_gc, T_gc, 16 * sizeof(double), hipMemcpyHostToDevice));
-    launch_pose_derived(s->self.dP, h);
+    launch_set_pose(s->self.dP, T_gc, 0, nullptr, h);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(h));
     return VS_OK;
@@ -1866,8 +1859,8 @@ static vs_status occupied_bricks(vs_session *s, std::vector<uint32_t> &out) {
     std::vector<uint32_t> bits(s->L.nwords);
     HIP_TRY(hipMemcpy(bits.data(), s->hp.bocc, bits.size() * 4, hipMemcpyDeviceToHost));
     out.clear();
-    for (uint32_t b = 0; b < s->L.nbricks; ++b)
-        if ((bits[b >> 5] >> (b & 31)) & 1u) out.push_back(b);
+    for (uint32_t w = 0; w < s->L.nwords; ++w)
+        for (uint32_t v = bits[w]; v; v &= v - 1) out.push_back(w * 32 + (uint32_t)__builtin_ctz(v));
     return VS_OK;
 }
 
@@ -1898,8 +1891,7 @@ vs_status vs_session_snapshot(vs_session *s, void *buf, size_t capacity, size_t 
     *bytes = need;
     if (!buf || capacity < need) return buf ? fail(VS_EINVAL, "snapshot needs %zu bytes, buffer has %zu", need, capacity)
                                             : VS_OK;
-    SessState st;
-    HIP_TRY(hipMemcpy(&st, s->st, sizeof(st), hipMemcpyDeviceToHost));
+    const HostState &st = *s->host;
     vs_snapshot_header h;
     std::memset(&h, 0, sizeof(h));
     std::memcpy(h.magic, "VSCANSNP", 8);
@@ -1971,19 +1963,19 @@ vs_status restore_session(vs_ctx *ctx, const void *buf, size_t bytes, bool poole
     const size_t packed = n * (size_t)kBrickVox * (h.value_bytes + h.weight_bytes + h.color_bytes);
     hipError_t e = hipSuccess;
     if (n) {
+        // indices and bricks in one upload, placed so that the bricks are aligned
+        const size_t lead = align_up(n * 4);
         char *dev = nullptr;
-        e = pooled ? hipMallocAsync((void **)&dev, align_up(n * 4) + packed, s->stream)
-                   : hipMalloc((void **)&dev, align_up(n * 4) + packed);
+        e = pooled ? hipMallocAsync((void **)&dev, lead + packed, s->stream) : hipMalloc((void **)&dev, lead + packed);
         if (e == hipSuccess && pooled) e = hipStreamSynchronize(s->stream);
         if (e == hipSuccess) {
-            const char *in = (const char *)buf + sizeof(h);
-            e = hipMemcpy(dev, in, n * 4, hipMemcpyHostToDevice);
-            if (e == hipSuccess) e = hipMemcpy(dev + align_up(n * 4), in + n * 4, packed, hipMemcpyHostToDevice);
+            const uint32_t *idx = (const uint32_t *)(dev + lead - n * 4);
+            e = hipMemcpy((void *)idx, (const char *)buf + sizeof(h), n * 4 + packed, hipMemcpyHostToDevice);
             if (e == hipSuccess) {
-                launch_brick_pack(s->self.dP, (const uint32_t *)dev, (unsigned)n, (int)h.value_bytes,
-                                  (int)h.weight_bytes, (int)h.color_bytes, (uint8_t *)dev + align_up(n * 4), 1,
-                                  s->stream);
-                launch_occupancy_rebuild(s->self.dP, s->L.nbricks, s->d.tsdf_type, s->d.weight_type, s->L.sdim[2], s->stream);
+                launch_brick_pack(s->self.dP, idx, (unsigned)n, (int)h.value_bytes, (int)h.weight_bytes,
+                                  (int)h.color_bytes, (uint8_t *)dev + lead, 1, s->stream);
+                launch_occupancy_rebuild(s->self.dP, idx, (uint32_t)n, s->d.tsdf_type, s->d.weight_type,
+                                         s->L.sdim[2], s->stream);
                 e = hipStreamSynchronize(s->stream);
             }
             if (pooled) {
@@ -1993,17 +1985,23 @@ vs_status restore_session(vs_ctx *ctx, const void *buf, size_t bytes, bool poole
             }
         }
     }
-    if (e == hipSuccess) {
-        const int32_t frames = h.frames;
-        e = hipMemcpy((char *)s->st + offsetof(SessState, frames), &frames, sizeof(frames), hipMemcpyHostToDevice);
-        launch_pose_derived(s->self.dP, s->stream);  // the pose as it is, and the host's record with the count
-    }
+    launch_set_pose(s->self.dP, h.T_gc, 0, &h.frames, s->stream);
+    if (e == hipSuccess) e = hipGetLastError();
     if (e != hipSuccess) {
         vs_session_destroy(s);
         return fail(VS_EHIP, "restore: %s", hipGetErrorString(e));
     }
-    // the model maps the next frame tracks against: render them at the saved pose
-    for (int l = 0; l < s->d.levels && r == VS_OK; ++l) r = vs_raycast(s, l, nullptr);
+    // the model maps the next frame tracks against: render them at the saved
+    // pose, all levels in one launch (a launch lasts as long as its longest ray)
+    {
+        const Batch &B = s->self;
+        LevelWork lw = level_work(B.dWork, B.nWork, B.levels);
+        lw.force = 1;
+        launch_raycast_march(B.dP, lw, B.tt, B.wt, nullptr, kRay8x8, B.addr, s->stream);
+        launch_raycast_shade(B.dP, lw, B.tt, B.wt, nullptr, kRay8x8, 4, B.addr, s->stream);
+        s->last = s->stream;
+        if (hipGetLastError() != hipSuccess) r = fail(VS_EHIP, "restore: the render could not be launched");
+    }
     if (r == VS_OK) r = sync_last(s);
     if (r != VS_OK) {
         vs_session_destroy(s);
@@ -2080,7 +2078,7 @@ vs_status vs_volume_upload(vs_session *s, const float *tsdf, const float *weight
     if (e == hipSuccess) e = hipMemcpy(tmp + N, weight, N * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
         launch_volume_from_linear(s->self.dP, N, s->d.tsdf_type, s->d.weight_type, tmp, tmp + N, s->stream);
-        launch_occupancy_rebuild(s->self.dP, s->L.nbricks, s->d.tsdf_type, s->d.weight_type, s->L.sdim[2], s->stream);
+        launch_occupancy_rebuild(s->self.dP, nullptr, s->L.nbricks, s->d.tsdf_type, s->d.weight_type, s->L.sdim[2], s->stream);
         e = hipStreamSynchronize(s->stream);
     }
     hipFree(tmp);

@@ -901,12 +901,25 @@ __global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *_
     }
 }
 
-// Pose set from the host: derived copies only.
-__global__ void k_pose_derived(const SessParams *__restrict__ SP) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        set_pose_derived(SP[0], SP[0].st);
-        publish_host(SP[0], SP[0].st);
+// Pose set from the host, with its derived copies; reset: every other field of
+// the state as for a new session first; set_frames: the frame count too.
+__global__ __launch_bounds__(64) void k_set_pose(const SessParams *__restrict__ SP, Mat16d T, int reset, int set_frames,
+                                                 int frames) {
+    SessState *st = SP[0].st;
+    if (reset) {
+        static_assert(sizeof(SessState) % 4 == 0, "cleared by words");
+        for (unsigned i = threadIdx.x; i < sizeof(SessState) / 4; i += 64) stg((uint32_t *)st, i, 0u);
     }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int k = 0; k < 16; ++k) st->T_gc[k] = T.m[k];
+    if (reset) {
+        st->conv_level = -1;
+        st->active = 1;
+    }
+    if (set_frames) st->frames = frames;
+    set_pose_derived(SP[0], st);
+    publish_host(SP[0], st);
 }
 
 // Normal equations of one iteration without a solve (diagnostics/parity).
@@ -1011,8 +1024,10 @@ void launch_track_finalize(const SessParams *P, int nsess, unsigned *bricks, hip
 void launch_integrate_begin(const SessParams *P, unsigned *bricks, hipStream_t s) {
     hipLaunchKernelGGL(k_integrate_begin, dim3(1), dim3(64), 0, s, P, bricks);
 }
-void launch_pose_derived(const SessParams *P, hipStream_t s) {
-    hipLaunchKernelGGL(k_pose_derived, dim3(1), dim3(64), 0, s, P);
+void launch_set_pose(const SessParams *P, const double *T, int reset, const int *frames, hipStream_t s) {
+    Mat16d m;
+    for (int k = 0; k < 16; ++k) m.m[k] = T ? T[k] : ((k % 5) == 0 ? 1.0 : 0.0);
+    hipLaunchKernelGGL(k_set_pose, dim3(1), dim3(64), 0, s, P, m, reset, frames != nullptr, frames ? *frames : 0);
 }
 // Sum of one ICP system's tile partials in tile order: thread k adds term k
 // of tiles 0, 1, ..., nt-1 in FP64, the order of vs_icp_system's host loop,

@@ -306,15 +306,26 @@ __global__ __launch_bounds__(256) void k_gather_depth(const SessParams *__restri
     }
 }
 
-// n 32-bit words at p set to v (session set-up: map sentinels).
-__global__ void k_fill_u32(uint32_t *__restrict__ p, size_t n, uint32_t v) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        stg(p, i, v);
+// Image buffers of a new session: empty pyramid, images and textures, model
+// maps at the -100 sentinel, in one launch (a fill per buffer had cost an open
+// ~12 launches). Every buffer is 256-byte aligned and padded.
+__global__ __launch_bounds__(256) void k_session_init(const SessParams *__restrict__ SP) {
+    const SessParams &P = SP[0];
+    const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+    const auto fill = [&](void *p, size_t bytes, uint32_t v) {
+        for (size_t i = i0; i < (bytes + 15) / 16; i += step) stg((vs_u4 *)p, i, vs_u4{v, v, v, v});
+    };
+    for (int l = 0; l < kMaxLevels; ++l) {
+        const size_t n = (size_t)P.lev[l].W * P.lev[l].H;
+        fill(P.filt[l], n * 4, 0u);
+        fill(P.mvn[l], (n + 1) * 2 * sizeof(MapXYZ), 0xC2C80000u);  // -100.0f
+        fill(P.mimg[l], n, 0u);
+        if (P.mtex[l]) fill(P.mtex[l], n * 3, 0u);
+    }
 }
-void launch_fill_u32(uint32_t *p, size_t n, uint32_t v, hipStream_t s) {
-    if (n == 0) return;
-    const size_t blocks = std::min<size_t>((n + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, s, p, n, v);
+void launch_session_init(const SessParams *P, size_t npx, hipStream_t s) {
+    const size_t blocks = std::min<size_t>((npx + 255) / 256, 2048);
+    hipLaunchKernelGGL(k_session_init, dim3((unsigned)blocks), dim3(256), 0, s, P);
 }
 
 void launch_gather_depth(const SessParams *P, const DepthChunk &ch, hipStream_t s) {

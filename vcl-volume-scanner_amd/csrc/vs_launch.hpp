@@ -18,8 +18,8 @@ struct DepthChunk {  // passed by value: device frame pointers and the batch slo
     int n;
 };
 void launch_gather_depth(const SessParams *P, const DepthChunk &ch, hipStream_t s);
-// n 32-bit words at p set to v
-void launch_fill_u32(uint32_t *p, size_t n, uint32_t v, hipStream_t s);
+// image buffers of a new session (P[0]; npx level-0 pixels)
+void launch_session_init(const SessParams *P, size_t npx, hipStream_t s);
 // force (here and below): run also for sessions whose state does not have a
 // frame in a step (the single operators)
 // out (nullable, single session): the filtered frame also goes there
@@ -117,13 +117,15 @@ void launch_raycast_shade(const SessParams *P, const LevelWork &lw, int tsdf_typ
                           unsigned long long *stats, int ray_block, int waves, int addr, hipStream_t s);
 // volume maintenance (single session, P points at its parameters)
 void launch_volume_init(const SessParams *P, size_t nvox, int tsdf_type, int weight_type, uint32_t nwords,
-                        int sd_slices, hipStream_t s);
+                        hipStream_t s);
 void launch_volume_to_linear(const SessParams *P, size_t nvox, int tsdf_type, int weight_type, float *F, float *Wt,
                              hipStream_t s);
 void launch_volume_from_linear(const SessParams *P, size_t nvox, int tsdf_type, int weight_type, const float *F,
                                const float *Wt, hipStream_t s);
-void launch_occupancy_rebuild(const SessParams *P, uint32_t nbricks, int tsdf_type, int weight_type, int sd_slices,
-                              hipStream_t s);
+// idx (nullable): only these nbricks bricks, of a volume whose other bricks are
+// as launch_volume_init leaves them
+void launch_occupancy_rebuild(const SessParams *P, const uint32_t *idx, uint32_t nbricks, int tsdf_type,
+                              int weight_type, int sd_slices, hipStream_t s);
 void launch_color_to_linear(const SessParams *P, size_t nvox, uint8_t *rgb, hipStream_t s);
 // input pre-steps (vs_pre.hip); is_float selects float metres, else uint16 mm
 void launch_depth_reproject(int is_float, const void *src, int sw, int sh, const float Ks[4], const float Kd[4],

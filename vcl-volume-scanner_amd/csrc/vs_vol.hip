@@ -1387,6 +1387,11 @@ __global__ void k_volume_init(const SessParams *__restrict__ SP, size_t nvox, ui
         stg(P.bband, w, 0u);
         if (w < (size_t)P.sband_words) stg(P.sband, w, 0u);
     }
+    // no band superbrick: every distance at the cap
+    const size_t nsd = ((size_t)P.sdim[0] * P.sdim[1] * P.sdim[2] + 7) / 8;
+    static_assert(kDistMax == 15, "four set bits a superbrick");
+    for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < nsd; w += (size_t)gridDim.x * blockDim.x)
+        stg((uint32_t *)P.sdist, w, 0xFFFFFFFFu);
     const size_t nflag = ((size_t)P.bdim[0] * P.bdim[1] * P.bdim[2] + 127) / 128 * 32;  // 32-bit words of the padded flags
     for (size_t w = (size_t)blockIdx.x * blockDim.x + threadIdx.x; w < nflag; w += (size_t)gridDim.x * blockDim.x)
         stg((uint32_t *)P.vmask, w, 0u);
@@ -1535,11 +1540,13 @@ __global__ void k_volume_from_linear(const SessParams *__restrict__ SP, size_t n
     }
 }
 // bocc and the band bits from the volume (after an upload or a restore): one
-// workgroup per brick; sband is cleared first
+// workgroup per brick (of idx, when given); sband is cleared first
 template <class TV, class TW>
-__global__ __launch_bounds__(kTileThreads) void k_occupancy(const SessParams *__restrict__ SP, uint32_t nbricks) {
+__global__ __launch_bounds__(kTileThreads) void k_occupancy(const SessParams *__restrict__ SP,
+                                                            const uint32_t *__restrict__ idx, uint32_t nbricks) {
     const SessParams &P = SP[0];
-    for (uint32_t b = blockIdx.x; b < nbricks; b += gridDim.x) {
+    for (uint32_t i0 = blockIdx.x; i0 < nbricks; i0 += gridDim.x) {
+        const uint32_t b = idx ? idx[i0] : i0;
         bool any = false, band = false;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -1726,10 +1733,8 @@ template <class TV, class TW>
 static void init_t(const SessParams *P, size_t nvox, uint32_t nwords, hipStream_t s) {
     hipLaunchKernelGGL((k_volume_init<TV, TW>), dim3(grid_for(nvox)), dim3(256), 0, s, P, nvox, nwords);
 }
-void launch_volume_init(const SessParams *P, size_t nvox, int tt, int wt, uint32_t nwords, int sd_slices,
-                        hipStream_t s) {
+void launch_volume_init(const SessParams *P, size_t nvox, int tt, int wt, uint32_t nwords, hipStream_t s) {
     VS_DISPATCH(tt, wt, init_t, P, nvox, nwords, s);
-    launch_sdist(P, 1, sd_slices, 1, s);
 }
 template <class TV, class TW>
 static void to_lin_t(const SessParams *P, size_t nvox, float *F, float *Wt, hipStream_t s) {
@@ -1747,14 +1752,15 @@ void launch_volume_from_linear(const SessParams *P, size_t nvox, int tt, int wt,
     VS_DISPATCH(tt, wt, from_lin_t, P, nvox, F, Wt, s);
 }
 template <class TV, class TW>
-static void occupancy_t(const SessParams *P, uint32_t nbricks, int g, hipStream_t s) {
-    hipLaunchKernelGGL((k_occupancy<TV, TW>), dim3(g), dim3(kTileThreads), 0, s, P, nbricks);
+static void occupancy_t(const SessParams *P, const uint32_t *idx, uint32_t nbricks, int g, hipStream_t s) {
+    hipLaunchKernelGGL((k_occupancy<TV, TW>), dim3(g), dim3(kTileThreads), 0, s, P, idx, nbricks);
 }
-void launch_occupancy_rebuild(const SessParams *P, uint32_t nbricks, int tt, int wt, int sd_slices, hipStream_t s) {
+void launch_occupancy_rebuild(const SessParams *P, const uint32_t *idx, uint32_t nbricks, int tt, int wt,
+                              int sd_slices, hipStream_t s) {
     int g = (int)(nbricks > 16384 ? 16384 : nbricks);
     if (g <= 0) return;
     hipLaunchKernelGGL(k_sband_clear, dim3(16), dim3(256), 0, s, P);
-    VS_DISPATCH(tt, wt, occupancy_t, P, nbricks, g, s);
+    VS_DISPATCH(tt, wt, occupancy_t, P, idx, nbricks, g, s);
     launch_sdist(P, 1, sd_slices, 1, s);
 }
 
