@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstddef>
@@ -13,6 +14,7 @@
 #include <exception>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -365,9 +367,111 @@ struct HostStates {
     }
 };
 
+// Large downloads to ordinary (pageable) host memory. The runtime's own copy
+// moves them through one thread, at 16 GB/s into touched memory and less into
+// fresh arrays, whose pages that thread also faults in. Here four threads take
+// the pieces in turn, each with two page-locked pieces of its own: one is
+// filled by DMA while the other is copied out. (A 256^3 volume's 134 MB of
+// values and weights: 8.1 -> 4.0 ms into touched memory, 15.2 -> 11.1 into
+// fresh arrays; a second stream makes it 6.4, pieces of 1 MB 4.9, eight lanes
+// change nothing.) The lanes (16 MB page-locked, one stream) are made by the
+// first large download and kept until the context ends; downloads of one
+// context take turns.
+constexpr int kLanes = 4;
+constexpr size_t kPiece = (size_t)2 << 20;
+constexpr size_t kStagedDownload = (size_t)16 << 20;  // smaller ones: the runtime's copy (no threads to start)
+struct Download {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+struct Downloader {
+    std::mutex m;
+    hipStream_t s = nullptr;
+    char *pinned = nullptr;  // two pieces per lane
+    hipEvent_t ev[kLanes][2] = {};
+    hipError_t init() {
+        hipError_t e = hipSuccess;
+        if (!s) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+        for (auto &l : ev)
+            for (auto &x : l)
+                if (e == hipSuccess && !x) e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
+        if (e == hipSuccess && !pinned) e = hipHostMalloc((void **)&pinned, kLanes * 2 * kPiece, hipHostMallocDefault);
+        return e;
+    }
+    // The device data is complete (the caller has waited for it).
+    hipError_t run(int device, const std::vector<Download> &list) {
+        struct Part {
+            char *dst;
+            const char *src;
+            size_t bytes;
+        };
+        std::vector<Part> parts;
+        size_t total = 0;
+        for (const Download &d : list) {
+            total += d.bytes;
+            for (size_t o = 0; o < d.bytes; o += kPiece)
+                parts.push_back({(char *)d.dst + o, (const char *)d.src + o, std::min(kPiece, d.bytes - o)});
+        }
+        std::lock_guard<std::mutex> hold(m);
+        if (total < kStagedDownload || init() != hipSuccess) {
+            for (const Download &d : list) {
+                const hipError_t e = hipMemcpy(d.dst, d.src, d.bytes, hipMemcpyDeviceToHost);
+                if (e != hipSuccess) return e;
+            }
+            return hipSuccess;
+        }
+        std::atomic<int> err{hipSuccess};
+        const auto work = [&](int w) {
+            char *buf = pinned + (size_t)w * 2 * kPiece;
+            hipError_t e = hipSetDevice(device);
+            const auto fetch = [&](size_t k, int h) {
+                if (e == hipSuccess)
+                    e = hipMemcpyAsync(buf + h * kPiece, parts[k].src, parts[k].bytes, hipMemcpyDeviceToHost, s);
+                if (e == hipSuccess) e = hipEventRecord(ev[w][h], s);
+            };
+            int h = 0;
+            if ((size_t)w < parts.size()) fetch(w, 0);
+            for (size_t k = w; k < parts.size() && e == hipSuccess; k += kLanes, h ^= 1) {
+                if (k + kLanes < parts.size()) fetch(k + kLanes, h ^ 1);
+                if (e == hipSuccess) e = hipEventSynchronize(ev[w][h]);
+                if (e == hipSuccess) std::memcpy(parts[k].dst, buf + h * kPiece, parts[k].bytes);
+            }
+            if (e != hipSuccess) err = e;
+        };
+        // lanes whose thread cannot be started are this thread's
+        std::vector<std::thread> pool;
+        std::vector<int> mine{0};
+        for (int w = 1; w < kLanes; ++w) {
+            try {
+                pool.emplace_back(work, w);
+            } catch (const std::exception &) {
+                mine.push_back(w);
+            }
+        }
+        for (int w : mine) work(w);
+        for (auto &t : pool) t.join();
+        if (err.load() != hipSuccess) (void)hipStreamSynchronize(s);
+        return (hipError_t)err.load();
+    }
+    void release() {
+        if (s) hipStreamSynchronize(s);
+        for (auto &l : ev)
+            for (auto &x : l) {
+                if (x) hipEventDestroy(x);
+                x = nullptr;
+            }
+        if (pinned) hipHostFree(pinned);
+        if (s) hipStreamDestroy(s);
+        pinned = nullptr;
+        s = nullptr;
+    }
+};
+
 struct vs_ctx {
     int device = 0;
     HostStates hosts;
+    Downloader down;
     double *scratch = nullptr;  // this device's copy of `scratch` (vs_icp_system_noalloc)
     std::map<std::vector<vs_session *>, std::unique_ptr<Batch>> batches;
     std::vector<vs_session *> sessions;
@@ -1193,6 +1297,7 @@ vs_status vs_ctx_destroy(vs_ctx *ctx) {
     ctx->timer.destroy();
     (void)hipDeviceSynchronize();
     ctx->hosts.release();
+    ctx->down.release();
     delete ctx;
     return VS_OK;
 }
@@ -1812,7 +1917,7 @@ vs_status vs_volume_download_color(vs_session *s, uint8_t *rgb_planar) {
     if (e != hipSuccess) return fail(VS_ENOMEM, "download buffer: %s", hipGetErrorString(e));
     launch_color_to_linear(s->self.dP, n, d, s->stream);
     e = hipStreamSynchronize(s->stream);
-    if (e == hipSuccess) e = hipMemcpy(rgb_planar, d, n * 3, hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = s->ctx->down.run(s->ctx->device, {{rgb_planar, d, n * 3}});
     hipFree(d);
     if (e != hipSuccess) return fail(VS_EHIP, "colour download: %s", hipGetErrorString(e));
     return VS_OK;
@@ -1918,7 +2023,8 @@ vs_status vs_session_snapshot(vs_session *s, void *buf, size_t capacity, size_t 
                               (uint8_t *)dev + align_up(n * 4), 0, s->stream);
             e = hipStreamSynchronize(s->stream);
         }
-        if (e == hipSuccess) e = hipMemcpy(out + sizeof(h) + n * 4, dev + align_up(n * 4), packed, hipMemcpyDeviceToHost);
+        if (e == hipSuccess)
+            e = s->ctx->down.run(s->ctx->device, {{out + sizeof(h) + n * 4, dev + align_up(n * 4), packed}});
         hipFree(dev);
         if (e != hipSuccess) return fail(VS_EHIP, "snapshot: %s", hipGetErrorString(e));
     }
@@ -2054,8 +2160,10 @@ vs_status vs_volume_download(vs_session *s, float *tsdf, float *weight, uint8_t 
         HIP_TRY(hipMalloc((void **)&tmp, 2 * N * sizeof(float)));
         launch_volume_to_linear(s->self.dP, N, s->d.tsdf_type, s->d.weight_type, tmp, tmp + N, s->stream);
         hipError_t e = hipStreamSynchronize(s->stream);
-        if (e == hipSuccess && tsdf) e = hipMemcpy(tsdf, tmp, N * 4, hipMemcpyDeviceToHost);
-        if (e == hipSuccess && weight) e = hipMemcpy(weight, tmp + N, N * 4, hipMemcpyDeviceToHost);
+        std::vector<Download> out;
+        if (tsdf) out.push_back({tsdf, tmp, N * 4});
+        if (weight) out.push_back({weight, tmp + N, N * 4});
+        if (e == hipSuccess) e = s->ctx->down.run(s->ctx->device, out);
         hipFree(tmp);
         if (e != hipSuccess) return fail(VS_EHIP, "volume download: %s", hipGetErrorString(e));
     }
