@@ -1479,7 +1479,7 @@ vs_status create_session(vs_ctx *ctx, const vs_session_desc *desc, const double 
     }
     // empty pyramid and images, model maps at the sentinel; then state and
     // volume (vs_session_reset), all on the session's stream
-    launch_session_init(B.dP, (size_t)d.width * d.height, s->stream);
+    launch_session_init(B.dP, (size_t)d.width * d.height, (uint32_t *)(m + L.keys), s->stream);
     HIP_TRY(hipGetLastError());
     vs_session *raw = s.release();
     ctx->sessions.push_back(raw);

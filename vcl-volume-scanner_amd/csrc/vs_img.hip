@@ -307,14 +307,15 @@ __global__ __launch_bounds__(256) void k_gather_depth(const SessParams *__restri
 }
 
 // Image buffers of a new session: empty pyramid, images and textures, model
-// maps at the -100 sentinel, in one launch (a fill per buffer had cost an open
+// maps at the -100 sentinel, the reprojection's keys empty, in one launch (a fill per buffer had cost an open
 // ~12 launches). Every buffer is 256-byte aligned and padded.
-__global__ __launch_bounds__(256) void k_session_init(const SessParams *__restrict__ SP) {
+__global__ __launch_bounds__(256) void k_session_init(const SessParams *__restrict__ SP, uint32_t *keys) {
     const SessParams &P = SP[0];
     const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
     const auto fill = [&](void *p, size_t bytes, uint32_t v) {
         for (size_t i = i0; i < (bytes + 15) / 16; i += step) stg((vs_u4 *)p, i, vs_u4{v, v, v, v});
     };
+    fill(keys, (size_t)P.lev[0].W * P.lev[0].H * 4, 0xFFFFFFFFu);
     for (int l = 0; l < kMaxLevels; ++l) {
         const size_t n = (size_t)P.lev[l].W * P.lev[l].H;
         fill(P.filt[l], n * 4, 0u);
@@ -323,9 +324,9 @@ __global__ __launch_bounds__(256) void k_session_init(const SessParams *__restri
         if (P.mtex[l]) fill(P.mtex[l], n * 3, 0u);
     }
 }
-void launch_session_init(const SessParams *P, size_t npx, hipStream_t s) {
+void launch_session_init(const SessParams *P, size_t npx, uint32_t *keys, hipStream_t s) {
     const size_t blocks = std::min<size_t>((npx + 255) / 256, 2048);
-    hipLaunchKernelGGL(k_session_init, dim3((unsigned)blocks), dim3(256), 0, s, P);
+    hipLaunchKernelGGL(k_session_init, dim3((unsigned)blocks), dim3(256), 0, s, P, keys);
 }
 
 void launch_gather_depth(const SessParams *P, const DepthChunk &ch, hipStream_t s) {

@@ -18,8 +18,8 @@ struct DepthChunk {  // passed by value: device frame pointers and the batch slo
     int n;
 };
 void launch_gather_depth(const SessParams *P, const DepthChunk &ch, hipStream_t s);
-// image buffers of a new session (P[0]; npx level-0 pixels)
-void launch_session_init(const SessParams *P, size_t npx, hipStream_t s);
+// image buffers of a new session (P[0]; npx level-0 pixels; keys: launch_depth_reproject's)
+void launch_session_init(const SessParams *P, size_t npx, uint32_t *keys, hipStream_t s);
 // force (here and below): run also for sessions whose state does not have a
 // frame in a step (the single operators)
 // out (nullable, single session): the filtered frame also goes there
@@ -127,7 +127,8 @@ void launch_volume_from_linear(const SessParams *P, size_t nvox, int tsdf_type, 
 void launch_occupancy_rebuild(const SessParams *P, const uint32_t *idx, uint32_t nbricks, int tsdf_type,
                               int weight_type, int sd_slices, hipStream_t s);
 void launch_color_to_linear(const SessParams *P, size_t nvox, uint8_t *rgb, hipStream_t s);
-// input pre-steps (vs_pre.hip); is_float selects float metres, else uint16 mm
+// input pre-steps (vs_pre.hip); is_float selects float metres, else uint16 mm;
+// key: dw * dh words, all ones before and after a call
 void launch_depth_reproject(int is_float, const void *src, int sw, int sh, const float Ks[4], const float Kd[4],
                             const float T[16], uint32_t *key, void *dst, int dw, int dh, hipStream_t s);
 void launch_depth_crop(const SessParams *P, int is_float, void *depth, int w, int h, const float K[4],

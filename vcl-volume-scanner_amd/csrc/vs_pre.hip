@@ -24,28 +24,79 @@ __device__ __forceinline__ float depth_value<float>(float v) { return v; }
 __device__ __forceinline__ uint32_t depth_key(uint16_t v) { return v; }
 __device__ __forceinline__ uint32_t depth_key(float v) { return __float_as_uint(v); }
 
+// One workgroup per 64x16 source tile, four rows a wave. The tile's pixels
+// land in a small window of the destination (its source scale plus the
+// parallax of its depths), so their minima are taken in LDS first and only one
+// atomic per destination pixel and tile goes to memory: those atomics, not the
+// arithmetic, bound the launch (1920x1080 into 1280x720: one per source pixel
+// 32 us, per tile and destination pixel 11). A tile whose window is larger than kWinW x kWinH goes to
+// memory directly.
+constexpr int kRepW = 64, kRepH = 16, kRepRows = 4;  // 256 threads
+constexpr int kWinW = 96, kWinH = 32;
 template <class T>
-__global__ void k_depth_reproject(const T *__restrict__ src, int sw, int sh, Mat16f Ks4, Mat16f Tds, uint32_t *key,
-                                  int dw, int dh) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= sw * sh) return;
-    const T raw = src[i];
-    const float td = depth_value<T>(raw);
-    if (!(td > 0.0f)) return;
+__global__ __launch_bounds__(256) void k_depth_reproject(const T *__restrict__ src, int sw, int sh, Mat16f Ks4,
+                                                         Mat16f Tds, uint32_t *key, int dw, int dh) {
+    __shared__ uint32_t win[kWinW * kWinH];
+    __shared__ int box[4][4];  // per wave: min x, min y, -max x, -max y
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int x0 = blockIdx.x * kRepW + lane, y0 = blockIdx.y * kRepH + wave * kRepRows;
     const float *Ks = Ks4.m, *Kd = Ks4.m + 4, *M = Tds.m;
-    const float x = (float)(i % sw), y = (float)(i / sw);
-    const f3 p = {td * (x - Ks[2]) / Ks[0], td * (y - Ks[3]) / Ks[1], td};
-    const f3 q = transform(M, p);
-    const float u = Kd[0] * q.x / q.z + Kd[2], v = Kd[1] * q.y / q.z + Kd[3];
-    int tx, ty;
-    if (!roundf_ref(u, tx) || !roundf_ref(v, ty)) return;
-    if (tx < 0 || tx > dw - 1 || ty < 0 || ty > dh - 1) return;
-    atomicMin(key + (size_t)ty * dw + tx, depth_key(raw));
-}
-
-__global__ void k_depth_key_fill(uint32_t *key, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        key[i] = 0xFFFFFFFFu;
+    T raw[kRepRows];
+    int tx[kRepRows], ty[kRepRows];
+#pragma unroll
+    for (int r = 0; r < kRepRows; ++r) {
+        const int y = y0 + r;
+        raw[r] = x0 < sw && y < sh ? ldg(src, (size_t)y * sw + x0) : T(0);
+    }
+    int b[4] = {0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF, 0x7FFFFFFF};
+#pragma unroll
+    for (int r = 0; r < kRepRows; ++r) {
+        const float td = depth_value<T>(raw[r]);
+        tx[r] = -1;
+        if (td > 0.0f) {
+            const float x = (float)x0, y = (float)(y0 + r);
+            const f3 p = {td * (x - Ks[2]) / Ks[0], td * (y - Ks[3]) / Ks[1], td};
+            const f3 q = transform(M, p);
+            const float u = Kd[0] * q.x / q.z + Kd[2], v = Kd[1] * q.y / q.z + Kd[3];
+            int ix, iy;
+            if (roundf_ref(u, ix) && roundf_ref(v, iy) && ix >= 0 && ix <= dw - 1 && iy >= 0 && iy <= dh - 1) {
+                tx[r] = ix;
+                ty[r] = iy;
+                b[0] = min(b[0], ix);
+                b[1] = min(b[1], iy);
+                b[2] = min(b[2], -ix);
+                b[3] = min(b[3], -iy);
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) b[k] = min(b[k], __shfl_xor(b[k], off, 64));
+        if (lane == 0) box[wave][k] = b[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) b[k] = min(min(box[0][k], box[1][k]), min(box[2][k], box[3][k]));
+    if (b[0] == 0x7FFFFFFF) return;  // no pixel of the tile lands
+    const int w = -b[2] - b[0] + 1, h = -b[3] - b[1] + 1;
+    if (w > kWinW || h > kWinH) {
+#pragma unroll
+        for (int r = 0; r < kRepRows; ++r)
+            if (tx[r] >= 0) atomicMin(key + (size_t)ty[r] * dw + tx[r], depth_key(raw[r]));
+        return;
+    }
+    for (int i = threadIdx.x; i < kWinW * h; i += 256) win[i] = 0xFFFFFFFFu;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kRepRows; ++r)
+        if (tx[r] >= 0) atomicMin(&win[(ty[r] - b[1]) * kWinW + tx[r] - b[0]], depth_key(raw[r]));
+    __syncthreads();
+    for (int y = wave; y < h; y += 4)
+        for (int x = lane; x < w; x += 64) {
+            const uint32_t k = win[y * kWinW + x];
+            if (k != 0xFFFFFFFFu) atomicMin(key + (size_t)(b[1] + y) * dw + b[0] + x, k);
+        }
 }
 
 __device__ __forceinline__ void key_to_depth(uint32_t k, uint16_t &out) { out = k == 0xFFFFFFFFu ? 0 : (uint16_t)k; }
@@ -53,9 +104,14 @@ __device__ __forceinline__ void key_to_depth(uint32_t k, float &out) {
     out = k == 0xFFFFFFFFu ? 0.0f : __uint_as_float(k);
 }
 template <class T>
-__global__ void k_depth_key_finish(const uint32_t *key, T *dst, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        key_to_depth(key[i], dst[i]);
+__global__ void k_depth_key_finish(uint32_t *key, T *dst, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x) {
+        const uint32_t k = ldg(key, i);
+        T v;
+        key_to_depth(k, v);
+        stg(dst, i, v);
+        if (k != 0xFFFFFFFFu) stg(key, i, 0xFFFFFFFFu);  // empty for the next frame
+    }
 }
 
 template <class T>
@@ -67,11 +123,11 @@ static void reproject_t(const void *src, int sw, int sh, const float Ks[4], cons
         k.m[4 + i] = Kd[i];
     }
     for (int i = 0; i < 16; ++i) m.m[i] = M[i];
-    const size_t nd = (size_t)dw * dh, ns = (size_t)sw * sh;
-    hipLaunchKernelGGL(k_depth_key_fill, dim3(1024), dim3(256), 0, s, key, nd);
-    hipLaunchKernelGGL(k_depth_reproject<T>, dim3((unsigned)((ns + 255) / 256)), dim3(256), 0, s, (const T *)src, sw,
-                       sh, k, m, key, dw, dh);
-    hipLaunchKernelGGL(k_depth_key_finish<T>, dim3(1024), dim3(256), 0, s, key, (T *)dst, nd);
+    const size_t nd = (size_t)dw * dh;
+    hipLaunchKernelGGL(k_depth_reproject<T>, dim3((unsigned)((sw + kRepW - 1) / kRepW), (unsigned)((sh + kRepH - 1) / kRepH)),
+                       dim3(256), 0, s, (const T *)src, sw, sh, k, m, key, dw, dh);
+    hipLaunchKernelGGL(k_depth_key_finish<T>, dim3((unsigned)std::min<size_t>((nd + 255) / 256, 4096)), dim3(256), 0, s,
+                       key, (T *)dst, nd);
 }
 void launch_depth_reproject(int is_float, const void *src, int sw, int sh, const float Ks[4], const float Kd[4],
                             const float T[16], uint32_t *key, void *dst, int dw, int dh, hipStream_t s) {
