@@ -288,6 +288,7 @@ struct HostStage {
 struct Batch {
     int n = 0, tt = 0, wt = 0, levels = 0;
     int max_iters[kMaxLevels] = {0, 0, 0};
+    bool pyr_pair = false;     // no member has exactly two levels
     int sd_slices = 1;         // most superbricks along z of a session (distance field passes)
     SessParams *dP = nullptr;  // device array
     WorkItem *dWork[kMaxLevels] = {nullptr, nullptr, nullptr};   // (slot, tile)
@@ -556,6 +557,7 @@ struct ListSet {
     size_t max_array = 0;  // largest voxel-record array of a member (bytes)
     int max_shift = 0, sd_slices = 0;  // largest superbrick, most superbricks along z
     int levels = 0, max_iters[kMaxLevels] = {0, 0, 0};
+    bool two_levels = false;
     int count = 0, max_w = 0, max_h = 0, max_dim = 0;
     void add(int slot, const vs_session *s) {
         ++count;
@@ -568,6 +570,7 @@ struct ListSet {
         max_h = std::max(max_h, s->d.height);
         for (int k = 0; k < 3; ++k) max_dim = std::max(max_dim, s->d.vol_dim[k]);
         levels = std::max(levels, s->d.levels);
+        two_levels |= s->d.levels == 2;
         for (int l = 0; l < kMaxLevels; ++l) {
             max_iters[l] = std::max(max_iters[l], s->hp.iters[l]);
             for (int t = 0; t < s->L.tiles[l]; ++t) tile[l].push_back({slot, t});
@@ -649,6 +652,7 @@ struct ListSet {
     // Iteration bounds, integrate grid and size class of the batch.
     vs_status settle(Batch &B, int integ_max) const {
         B.levels = levels;
+        B.pyr_pair = !two_levels;
         B.sd_slices = sd_slices;
         for (int l = 0; l < kMaxLevels; ++l) B.max_iters[l] = max_iters[l];
         B.bricks = bricks;
@@ -910,7 +914,7 @@ void enqueue_step(const Batch &B, hipStream_t s, Timer *timed) {
         launch_track_setup(B.dP, B.n, nullptr, s);
     launch_bilateral(B.dP, B.dWork[0], B.nWork[0], 0, nullptr, s);
     mark(1);
-    for (int l = 1; l < B.levels; ++l) launch_pyr_down(B.dP, B.dWork[l], B.nWork[l], l, 0, s);
+    launch_pyramid(B.dP, B.dWork, B.nWork, B.levels, B.pyr_pair, 0, s);
     mark(2);
     enqueue_track(B, s);
     mark(3);
@@ -1640,7 +1644,8 @@ vs_status vs_bilateral_filter_depth(vs_session *s, const void *depth_in, int in_
 vs_status vs_pyramid(vs_session *s, vs_stream stream) {
     if (!s) return fail(VS_EINVAL, "null session");
     hipStream_t h = pick(s, stream);
-    for (int l = 1; l < s->d.levels; ++l) launch_pyr_down(s->self.dP, s->self.dWork[l], s->self.nWork[l], l, 1, h);
+    const Batch &B = s->self;
+    launch_pyramid(B.dP, B.dWork, B.nWork, B.levels, B.pyr_pair, 1, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }

@@ -122,6 +122,78 @@ __global__ __launch_bounds__(kTileThreads) void k_pyr_down(const SessParams *__r
     stg(P.filt[l], (size_t)y * L.W + x, v);
 }
 
+// Levels 1 and 2 in one launch: a workgroup computes the level-1 pixels around
+// its 32x8 level-2 tile in LDS (the row sums of the blur first, each used by up
+// to three level-1 rows), writes the 64x16 of them that are its own, and
+// decimates them once more. Values as k_pyr_down's, operation for operation.
+// The halo repeats a quarter of level 1; a launch and its gap go (640x480 scan
+// 419 -> 416 us; with 4 waves a tile, walking its rows one after another, 419).
+constexpr int kP1W = 2 * kTileW + 3, kP1H = 2 * kTileH + 3;  // level-1 region: 67 x 19
+constexpr int kP0H = 2 * kP1H + 3;                           // level-0 rows of the row sums: 41
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_pyr_down2(const SessParams *__restrict__ SP,
+                                                            const WorkItem *__restrict__ work, int force) {
+    __shared__ float rows[kP0H][kP1W], l1[kP1H][kP1W];
+    const WorkItem wi = work[blockIdx.x];
+    const SessParams &P = SP[wi.sess];
+    const LevelDesc &L = P.lev[2];
+    if (P.levels < 3 || tile_out(L, wi.tile) || !(force || P.st->active)) return;
+    const int W0 = P.lev[0].W, H0 = P.lev[0].H, W1 = P.lev[1].W, H1 = P.lev[1].H;
+    const int tx = wi.tile % L.tiles_x, ty = wi.tile / L.tiles_x;
+    const int x1 = 2 * tx * kTileW - 1, y1 = 2 * ty * kTileH - 1;  // level-1 region's corner
+    const int y0 = 2 * y1 - 1;                                     // first level-0 row: 2 y1 + 1 - 2
+    const float *in = P.filt[0];
+#pragma unroll
+    for (int k0 = 0; k0 < kP0H * kP1W; k0 += THREADS) {
+        const int k = k0 + threadIdx.x;
+        if (k >= kP0H * kP1W) break;
+        const int r = k / kP1W, c = k - r * kP1W;
+        const int i = 2 * (x1 + c) + 1, y = y0 + r;
+        float h = 0.0f;
+        if (i >= 2 && i <= W0 - 3 && y >= 0 && y < H0) {
+            const size_t row = (size_t)y * W0;
+            h = 1.0f * ldg(in, row + i - 2) + 1.0f * ldg(in, row + i + 2) + 4.0f * ldg(in, row + i - 1) +
+                4.0f * ldg(in, row + i + 1) + 6.0f * ldg(in, row + i);
+        }
+        rows[r][c] = h;
+    }
+    __syncthreads();
+    // the last tile of a row or column also owns the odd column or row of level 1
+    const int xe = tx == L.tiles_x - 1 ? W1 : min(W1, 2 * (tx + 1) * kTileW);
+    const int ye = ty == L.tiles_y - 1 ? H1 : min(H1, 2 * (ty + 1) * kTileH);
+#pragma unroll
+    for (int k0 = 0; k0 < kP1H * kP1W; k0 += THREADS) {
+        const int k = k0 + threadIdx.x;
+        if (k >= kP1H * kP1W) break;
+        const int r = k / kP1W, c = k - r * kP1W;
+        const int x = x1 + c, y = y1 + r, i = 2 * x + 1, j = 2 * y + 1;
+        float v = 0.0f;
+        if (i >= 2 && i <= W0 - 3 && j >= 2 && j <= H0 - 3) {
+            const float *h = &rows[2 * r][c];  // level-0 row j - 2
+            v = (1.0f * h[0] + 1.0f * h[4 * kP1W] + 4.0f * h[kP1W] + 4.0f * h[3 * kP1W] + 6.0f * h[2 * kP1W]) /
+                (16.0f * 16.0f);
+        }
+        l1[r][c] = v;
+        if (r >= 1 && c >= 1 && x < xe && y < ye) stg(P.filt[1], (size_t)y * W1 + x, v);
+    }
+    __syncthreads();
+    const int lx = threadIdx.x % kTileW, ly = threadIdx.x / kTileW;
+    const int x = tx * kTileW + lx, y = ty * kTileH + ly;
+    if (ly >= kTileH || x >= L.W || y >= L.H) return;
+    const int i = 2 * x + 1, j = 2 * y + 1;
+    float v = 0.0f;
+    if (i >= 2 && i <= W1 - 3 && j >= 2 && j <= H1 - 3) {
+        float h[5];
+#pragma unroll
+        for (int r = 0; r < 5; ++r) {
+            const float *q = l1[2 * ly + r] + 2 * lx;  // level-1 row j + r - 2, columns i - 2 .. i + 2
+            h[r] = 1.0f * q[0] + 1.0f * q[4] + 4.0f * q[1] + 4.0f * q[3] + 6.0f * q[2];
+        }
+        v = (1.0f * h[0] + 1.0f * h[4] + 4.0f * h[1] + 4.0f * h[3] + 6.0f * h[2]) / (16.0f * 16.0f);
+    }
+    stg(P.filt[2], (size_t)y * L.W + x, v);
+}
+
 // Vertex and normal maps of pyramid level l (AoS float3, -100 invalid).
 // Reference: cpm_Compute_Point_Map / enm_Estimate_Normal_Map
 // (z_yooji_image_processor.cpp:119-227): n = normalize(dz/dx, dz/dy, -1) from
@@ -336,8 +408,19 @@ void launch_gather_depth(const SessParams *P, const DepthChunk &ch, hipStream_t 
 void launch_bilateral(const SessParams *P, const WorkItem *work, int n, int force, float *out, hipStream_t s) {
     if (n > 0) hipLaunchKernelGGL(k_bilateral, dim3(n), dim3(kTileThreads), 0, s, P, work, force, out);
 }
-void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int l, int force, hipStream_t s) {
-    if (n > 0) hipLaunchKernelGGL(k_pyr_down, dim3(n), dim3(kTileThreads), 0, s, P, work, l, force);
+void launch_pyramid(const SessParams *P, const WorkItem *const work[kMaxLevels], const int n[kMaxLevels], int levels,
+                    bool pair, int force, hipStream_t s) {
+    if (levels == 3 && pair) {
+        if (n[2] <= 0) return;
+        // 16 waves a tile while that leaves a CU for nearly every one of them
+        if (n[2] <= 1024)
+            hipLaunchKernelGGL(k_pyr_down2<1024>, dim3(n[2]), dim3(1024), 0, s, P, work[2], force);
+        else
+            hipLaunchKernelGGL(k_pyr_down2<kTileThreads>, dim3(n[2]), dim3(kTileThreads), 0, s, P, work[2], force);
+        return;
+    }
+    for (int l = 1; l < levels; ++l)
+        if (n[l] > 0) hipLaunchKernelGGL(k_pyr_down, dim3(n[l]), dim3(kTileThreads), 0, s, P, work[l], l, force);
 }
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int l, float *vtx, float *nrm, hipStream_t s) {
     if (n > 0)

@@ -24,7 +24,9 @@ void launch_session_init(const SessParams *P, size_t npx, uint32_t *keys, hipStr
 // frame in a step (the single operators)
 // out (nullable, single session): the filtered frame also goes there
 void launch_bilateral(const SessParams *P, const WorkItem *work, int n, int force, float *out, hipStream_t s);
-void launch_pyr_down(const SessParams *P, const WorkItem *work, int n, int level, int force, hipStream_t s);
+// levels 1 .. levels - 1 from level 0; pair: no session has exactly two levels
+void launch_pyramid(const SessParams *P, const WorkItem *const work[kMaxLevels], const int n[kMaxLevels], int levels,
+                    bool pair, int force, hipStream_t s);
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int level, float *vtx, float *nrm, hipStream_t s);
 // single session (P[0]), the reference loop's in-place order; bits: vn_words(W)
 // * H words of scratch
