@@ -888,16 +888,18 @@ hipStream_t pick(vs_session *s, vs_stream st) {
 void enqueue_track(const Batch &B, hipStream_t s) {
     const bool one = B.nGroup[0] <= kIcpStepGroups;  // one launch per iteration
     const bool lone = B.n == 1 && !B.active;             // its groups are 0, 1, ...
-    int seq = 0;
+    int seq = 0, prev = -1;
     for (int l = B.levels - 1; l >= 0; --l)
         for (int it = 0; it < B.max_iters[l]; ++it) {
-            if (one)
-                launch_icp_step(B.dP, lone ? nullptr : B.dGroup[l], B.nGroup[l], l, it, ++seq, s);
-            else
+            if (one) {
+                launch_icp_step(B.dP, lone ? nullptr : B.dGroup[l], B.nGroup[l], l, it, ++seq, prev, s);
+                prev = l;
+            } else {
                 launch_icp_iter(B.dP, B.dGroup[l], B.nGroup[l], B.n, l, it, s);
+            }
         }
     if (one)
-        launch_icp_finish(B.dP, B.n, B.bl.count, s);
+        launch_icp_finish(B.dP, B.n, B.bl.count, seq + 1, prev, s);
     else
         launch_track_finalize(B.dP, B.n, B.bl.count, s);
 }

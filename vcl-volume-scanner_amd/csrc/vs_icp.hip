@@ -46,85 +46,6 @@ __device__ void rigid_inverse(const double *T, double *Ti) {
     o[15] = 1.0;
     for (int k = 0; k < 16; ++k) Ti[k] = o[k];
 }
-// SE(3) exponential of x = [w; v] (the twist update of
-// z_uitme_Update_Incremental_Tracking_with_Matrix_Exponential, pose_tracker.cu:50-149),
-// with a series branch for small |w| (the reference divides by |w|).
-__device__ void expmap(const double *x, double *T) {
-    const double w0 = x[0], w1 = x[1], w2 = x[2];
-    const double th2 = w0 * w0 + w1 * w1 + w2 * w2, th = sqrt(th2);
-    double A, B, C;
-    if (th < 1e-4) {
-        A = 1.0 - th2 / 6.0 + th2 * th2 / 120.0;
-        B = 0.5 - th2 / 24.0 + th2 * th2 / 720.0;
-        C = 1.0 / 6.0 - th2 / 120.0 + th2 * th2 / 5040.0;
-    } else {
-        A = sin(th) / th;
-        B = (1.0 - cos(th)) / th2;
-        C = (th - sin(th)) / (th2 * th);
-    }
-    const double W[9] = {0, -w2, w1, w2, 0, -w0, -w1, w0, 0};
-    double W2[9];
-    for (int r = 0; r < 3; ++r)
-        for (int c = 0; c < 3; ++c) W2[r * 3 + c] = W[r * 3] * W[c] + W[r * 3 + 1] * W[3 + c] + W[r * 3 + 2] * W[6 + c];
-    for (int r = 0; r < 3; ++r) {
-        double t = 0.0;
-        for (int c = 0; c < 3; ++c) {
-            const double I = (r == c) ? 1.0 : 0.0;
-            T[r * 4 + c] = I + A * W[r * 3 + c] + B * W2[r * 3 + c];
-            t += (I + B * W[r * 3 + c] + C * W2[r * 3 + c]) * x[3 + c];
-        }
-        T[r * 4 + 3] = t;
-    }
-    T[12] = T[13] = T[14] = 0.0;
-    T[15] = 1.0;
-}
-// Cholesky and triangular solves with the reference's pivot rule
-// (d_lld_LL_Decomposition / d_sls_Solve_Linear_System_using_LLD,
-// _yooji_cuda_math.h:489-592): entries below a pivot < 1e-8 are zeroed and the
-// solve fails (status 4) if any pivot is below 1e-8 (or not a number). With
-// rel > 0 it also fails (status 8) when a squared pivot L_jj^2 is below
-// rel * A_jj: column j of J is then nearly a combination of the columns
-// before it (a plane leaves 3 of the 6 motions unconstrained), a near-rank
-// deficiency the absolute test cannot see at FP32 scales. The ratio is
-// invariant to the units of the rotation and translation columns.
-// Column by column, each below-diagonal entry and substitution step scaled by
-// the column's reciprocal pivot (6 FP64 divisions instead of 33 on the
-// solve's one-lane chain; the same sums in the same order).
-// Returns 0 on success.
-__device__ int cholesky_solve(const double *A, const double *b, double rel, double *x) {
-    double L[36], inv[6];
-    for (int k = 0; k < 36; ++k) L[k] = 0.0;
-    for (int j = 0; j < 6; ++j) {
-        double s = 0.0;
-        for (int k = 0; k < j; ++k) s += L[j * 6 + k] * L[j * 6 + k];
-        L[j * 6 + j] = sqrt(A[j * 6 + j] - s);
-        inv[j] = 1.0 / L[j * 6 + j];
-        const bool piv = fabs(L[j * 6 + j]) >= 1e-8;
-        for (int i = j + 1; i < 6; ++i) {
-            double t = 0.0;
-            for (int k = 0; k < j; ++k) t += L[i * 6 + k] * L[j * 6 + k];
-            L[i * 6 + j] = piv ? (A[i * 6 + j] - t) * inv[j] : 0.0;
-        }
-    }
-    for (int i = 0; i < 6; ++i)
-        if (!(fabs(L[i * 6 + i]) >= 1e-8)) return 4;
-    if (rel > 0.0)
-        for (int i = 0; i < 6; ++i)
-            if (L[i * 6 + i] * L[i * 6 + i] < rel * A[i * 6 + i]) return 8;
-    double y[6];
-    for (int i = 0; i < 6; ++i) {
-        double s = 0.0;
-        for (int k = 0; k < i; ++k) s += L[i * 6 + k] * y[k];
-        y[i] = (b[i] - s) * inv[i];
-    }
-    for (int i = 5; i >= 0; --i) {
-        double s = 0.0;
-        for (int k = i + 1; k < 6; ++k) s += L[k * 6 + i] * x[k];
-        x[i] = (y[i] - s) * inv[i];
-    }
-    return 0;
-}
-
 __device__ void publish_T21(SessState *st) {
     rigid_inverse(st->T_12, st->T_21);
     for (int k = 0; k < 16; ++k) st->T_21_f[k] = (float)st->T_21[k];
@@ -457,88 +378,228 @@ __global__ __launch_bounds__(kTileThreads) void k_icp_iter(const SessParams *__r
 
 // The 29 totals of ng group partials in FP64, in a fixed order that depends
 // on the group count alone: chunk c adds groups c, c + 64, ..., then the 64
-// chunk sums of a term are added as a tree of halves. A thread takes a (chunk,
-// term) pair, so neighbouring threads read neighbouring terms and a load
-// covers whole lines. (One wave with a group per lane, its sums exchanged
-// between the lanes in the same tree, read 64 lines per load.) Result in tot
-// (LDS), visible to the first wave only.
-constexpr int kSumChunks = 64;
+// chunk sums of a term are added as a tree of halves. A thread takes chunks c
+// and c + 32 of a term, the tree's first pair, so neighbouring threads read
+// neighbouring terms and a load covers whole lines. In two halves, so that a
+// kernel can have the first loads in flight together with the state it needs
+// before it knows whether there is anything to sum.
+constexpr int kSumChunks = 64, kSumPairs = kSumChunks / 2;
 template <int THREADS>
-__device__ __forceinline__ void sum_partials(const double *part, int ng, double (*chunk)[kIcpVals], double *tot) {
-    constexpr int U = 3, kPairs = kSumChunks * kIcpVals;
-    const int t = threadIdx.x;
+struct PartialSums {
+    static constexpr int N = (kSumPairs * kIcpVals + THREADS - 1) / THREADS;  // pairs per thread
+    static constexpr int U = N == 1 ? 5 : 3;                                  // groups per chunk and round
+    double v[N][2][U];
+    // groups g0 + c, g0 + c + 64, ... of the thread's chunks (0 beyond the
+    // last group: a running sum that began at 0.0 is never -0.0, so adding it
+    // changes nothing)
+    __device__ __forceinline__ void load(const double *part, int ng, int g0) {
 #pragma unroll
-    for (int p0 = 0; p0 < kPairs; p0 += THREADS) {
-        const int p = p0 + t, c = p / kIcpVals, k = p - c * kIcpVals;
-        if (p < kPairs) {
-            double s = 0.0;
-            for (int g = c; g < ng; g += U * kSumChunks) {
-                double v[U];
+        for (int n = 0; n < N; ++n) {
+            const int p = n * THREADS + (int)threadIdx.x, c = p / kIcpVals, k = p - c * kIcpVals;
 #pragma unroll
-                for (int u = 0; u < U; ++u) v[u] = ldg(part, (size_t)min(g + u * kSumChunks, ng - 1) * kIcpVals + k);
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int u = 0; u < U; ++u) s = g + u * kSumChunks < ng ? s + v[u] : s;
-            }
-            chunk[c][k] = s;
+                for (int u = 0; u < U; ++u) {
+                    const int g = g0 + c + h * kSumPairs + u * kSumChunks;
+                    v[n][h][u] = 0.0;
+                    if (p < kSumPairs * kIcpVals && g < ng) v[n][h][u] = ldg(part, (size_t)g * kIcpVals + k);
+                }
         }
     }
-    __syncthreads();
-    // two threads per term, each half of the first level's pairs
-    if (t < 2 * 32) {
-        const int k = t & 31, side = t >> 5;
-        if (k < kIcpVals) {
-            double v[16];
+    // after load(part, ng, 0); tot (LDS) is visible to the first wave only
+    __device__ __forceinline__ void finish(const double *part, int ng, double (*pair)[kIcpVals], double *tot) {
+        double s[N][2];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int c = q + 16 * side;
-                v[q] = chunk[c][k] + chunk[c + 32][k];
+        for (int n = 0; n < N; ++n)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                s[n][h] = 0.0;
+#pragma unroll
+                for (int u = 0; u < U; ++u) s[n][h] += v[n][h][u];
             }
+        for (int g0 = U * kSumChunks; g0 < ng; g0 += U * kSumChunks) {
+            load(part, ng, g0);
 #pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] += __shfl_xor(v[q], 32, 64);
+            for (int n = 0; n < N; ++n)
 #pragma unroll
-            for (int h = 8; h >= 1; h >>= 1)
+                for (int h = 0; h < 2; ++h)
 #pragma unroll
-                for (int q = 0; q < h; ++q) v[q] += v[q + h];
-            if (side == 0) tot[k] = v[0];
+                    for (int u = 0; u < U; ++u) s[n][h] += v[n][h][u];
         }
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            const int p = n * THREADS + (int)threadIdx.x, c = p / kIcpVals, k = p - c * kIcpVals;
+            if (p < kSumPairs * kIcpVals) pair[c][k] = s[n][0] + s[n][1];
+        }
+        __syncthreads();
+        // two threads per term, each half of the next level's pairs
+        const int t = threadIdx.x;
+        if (t < 2 * 32) {
+            const int k = t & 31, side = t >> 5;
+            if (k < kIcpVals) {
+                double w[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    const int c = q + 8 * side;
+                    w[q] = pair[c][k] + pair[c + 16][k];
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q) w[q] += __shfl_xor(w[q], 32, 64);
+#pragma unroll
+                for (int h = 4; h >= 1; h >>= 1)
+#pragma unroll
+                    for (int q = 0; q < h; ++q) w[q] += w[q + h];
+                if (side == 0) tot[k] = w[0];
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
     }
-    __builtin_amdgcn_wave_barrier();
-}
+};
 
-// One solve and SE(3) update from the 29 totals (one thread). Returns 0 when
-// T12 was updated, 1 when the step was below the convergence bound, else the
-// failure's status in `failed`.
+// Value of a double in a given lane (all lanes active), and in lane Q of each
+// quad of lanes.
+__device__ __forceinline__ double lane_of(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+template <int Q>
+__device__ __forceinline__ double quad_of(double v) {
+    constexpr int ctrl = Q * 0x55;
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xf, 0xf, true));
+}
+// position of entry (p, q), p <= q, of a 6x6 upper triangle stored by rows
+__device__ __forceinline__ constexpr int tri6(int p, int q) { return p * (11 - p) / 2 + q; }
+
+// One solve and SE(3) update from the 29 totals (LDS), by one wave; all of its
+// lanes are active. The outcome is the same in every lane, t12 is entry
+// lane % 16 of the updated increment.
 struct SolveResult {
     bool updated, converged;
     int failed;
+    double t12;
 };
-__device__ __forceinline__ SolveResult solve_totals(const SessParams &P, const double *tot, double T12[16]) {
-    SolveResult r{false, false, 0};
-    double ATA[36], ATb[6], x6[6];
-    int k = 0;
-    for (int i = 0; i < 6; ++i)
-        for (int j = i; j < 6; ++j) {
-            ATA[i * 6 + j] = ATA[j * 6 + i] = tot[k++];
-        }
-    for (int i = 0; i < 6; ++i) ATb[i] = tot[k++];
+// Cholesky and triangular solves with the reference's pivot rule
+// (d_lld_LL_Decomposition / d_sls_Solve_Linear_System_using_LLD,
+// _yooji_cuda_math.h:489-592): entries below a pivot < 1e-8 are zeroed and the
+// solve fails (status 4) if any pivot is below 1e-8 (or not a number). With
+// rel > 0 it also fails (status 8) when a squared pivot L_jj^2 is below
+// rel * A_jj: column j of J is then nearly a combination of the columns
+// before it (a plane leaves 3 of the 6 motions unconstrained), a near-rank
+// deficiency the absolute test cannot see at FP32 scales. The ratio is
+// invariant to the units of the rotation and translation columns. Each
+// below-diagonal entry and substitution step is scaled by the column's
+// reciprocal pivot (6 FP64 divisions instead of 33).
+// The update T12 <- exp(x) T12 takes x = [w; v] as a twist
+// (z_uitme_Update_Incremental_Tracking_with_Matrix_Exponential,
+// pose_tracker.cu:50-149), with a series branch for small |w| (the reference
+// divides by |w|).
+// Lane i holds row i of the factor and lane 4r + c entry (r, c) of the 4x4
+// matrices; every operation and its order are those of one lane doing it all,
+// which took 7000 cycles of a workgroup's 27000 in an iteration (640x480,
+// level 0), many of them the issue of independent FP64 operations; it is 5500
+// now, and an iteration 23500 with StepLoads (fused frame with preview: 412 ->
+// 408 us, 320x240 358 -> 354, 64 sessions 6.52 -> 6.45 ms).
+__device__ __forceinline__ SolveResult solve_wave(const SessParams &P, const double *tot, const double *T12) {
+    const int lane = threadIdx.x & 63;
+    SolveResult r{false, false, 0, 0.0};
     const double cnt = tot[21 + 6];
     if (P.icp_min_valid > 0 && cnt < (double)P.icp_min_valid) {
         r.failed = 7;
         return r;
     }
-    r.failed = cholesky_solve(ATA, ATb, (double)P.icp_rel_pivot, x6);
+    const int i = min(lane, 5), er = (lane >> 2) & 3, ec = lane & 3;
+    double a[6], l[6], t12c[4];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) a[j] = tot[tri6(min(i, j), max(i, j))];
+    const double b = tot[21 + i];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) t12c[k] = T12[k * 4 + ec];
+    double U[6][6], D[6], inv[6];  // the factor and its diagonal's reciprocals, in every lane
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < j; ++k) {
+            U[j][k] = lane_of(l[k], j);
+            t += l[k] * U[j][k];
+        }
+        const double d = a[j] - t;
+        D[j] = sqrt(lane_of(d, j));
+        inv[j] = 1.0 / D[j];
+        l[j] = fabs(D[j]) >= 1e-8 ? d * inv[j] : 0.0;
+    }
+    bool pivots = true, guard = false;
+    const double rel = (double)P.icp_rel_pivot;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+        pivots &= fabs(D[j]) >= 1e-8;
+        guard |= D[j] * D[j] < rel * tot[tri6(j, j)];
+    }
+    r.failed = !pivots ? 4 : (rel > 0.0 && guard) ? 8 : 0;
     if (r.failed != 0) return r;
+    double y[6], x[6], s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        y[k] = lane_of((b - s) * inv[k], k);
+        s += l[k] * y[k];
+    }
+#pragma unroll
+    for (int j = 5; j >= 0; --j) {
+        double q = 0.0;
+#pragma unroll
+        for (int k = j + 1; k < 6; ++k) q += U[k][j] * x[k];
+        x[j] = (y[j] - q) * inv[j];
+    }
     double ninf = 0.0;
-    for (int i = 0; i < 6; ++i) ninf = fmax(ninf, fabs(x6[i]));
+#pragma unroll
+    for (int k = 0; k < 6; ++k) ninf = fmax(ninf, fabs(x[k]));
     if (ninf < 5.0e-7) {
         r.converged = true;
         return r;
     }
-    double E[16];
-    expmap(x6, E);
-    matmul4d(E, T12, T12);
+    const double w0 = x[0], w1 = x[1], w2 = x[2];
+    const double th2 = w0 * w0 + w1 * w1 + w2 * w2, th = sqrt(th2);
+    double A, B, C;
+    if (th < 1e-4) {
+        A = 1.0 - th2 / 6.0 + th2 * th2 / 120.0;
+        B = 0.5 - th2 / 24.0 + th2 * th2 / 720.0;
+        C = 1.0 / 6.0 - th2 / 120.0 + th2 * th2 / 5040.0;
+    } else {
+        A = sin(th) / th;
+        B = (1.0 - cos(th)) / th2;
+        C = (th - sin(th)) / (th2 * th);
+    }
+    // W = [0 -w2 w1; w2 0 -w0; -w1 w0 0]: row er, column ec, and their product
+    const double Wr0 = er == 1 ? w2 : er == 2 ? -w1 : 0.0, Wr1 = er == 0 ? -w2 : er == 2 ? w0 : 0.0,
+                 Wr2 = er == 0 ? w1 : er == 1 ? -w0 : 0.0;
+    const double W0c = ec == 1 ? -w2 : ec == 2 ? w1 : 0.0, W1c = ec == 0 ? w2 : ec == 2 ? -w0 : 0.0,
+                 W2c = ec == 0 ? -w1 : ec == 1 ? w0 : 0.0;
+    const double W = ec == 0 ? Wr0 : ec == 1 ? Wr1 : Wr2, xv = ec == 0 ? x[3] : ec == 1 ? x[4] : x[5];
+    const double WW = Wr0 * W0c + Wr1 * W1c + Wr2 * W2c, I = er == ec ? 1.0 : 0.0;
+    const double rot = I + A * W + B * WW, vx = (I + B * W + C * WW) * xv;
+    double tr = 0.0;
+    tr += quad_of<0>(vx);
+    tr += quad_of<1>(vx);
+    tr += quad_of<2>(vx);
+    const double E = er == 3 ? (ec == 3 ? 1.0 : 0.0) : (ec == 3 ? tr : rot);
+    double m = 0.0;
+    m = fma(quad_of<0>(E), t12c[0], m);
+    m = fma(quad_of<1>(E), t12c[1], m);
+    m = fma(quad_of<2>(E), t12c[2], m);
+    m = fma(quad_of<3>(E), t12c[3], m);
+    r.t12 = m;
     r.updated = true;
     return r;
+}
+// Entry lane % 16 of the inverse of a rigid transform in LDS (rigid_inverse's
+// operations).
+__device__ __forceinline__ double rigid_inverse_lane(const double *T) {
+    const int er = (threadIdx.x >> 2) & 3, ec = threadIdx.x & 3;
+    const double rot = er < 3 && ec < 3 ? T[ec * 4 + er] : (er == ec ? 1.0 : 0.0);
+    const int c = min(er, 2);
+    const double t = -(T[c] * T[3] + T[4 + c] * T[7] + T[8 + c] * T[11]);
+    return er < 3 && ec == 3 ? t : rot;
 }
 
 // Second half of the two-launch form: one workgroup per session sums the
@@ -547,33 +608,35 @@ __device__ __forceinline__ SolveResult solve_totals(const SessParams &P, const d
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void k_icp_solve(const SessParams *__restrict__ SP, int nsess, int level,
                                                             int iter) {
-    __shared__ double chunk[kSumChunks][kIcpVals], tot[kIcpVals];
+    __shared__ double pair[kSumPairs][kIcpVals], tot[kIcpVals], T12[16];
     const int s = blockIdx.x;
     if (s >= nsess) return;
     const SessParams &P = SP[s];
     SessState *st = P.st;
-    if (level >= P.levels || icp_skip(P, st, level, iter)) return;
-    const LevelDesc &L = P.lev[level];
-    sum_partials<THREADS>(P.icp_part, icp_groups(L.tiles_x * L.tiles_y, level), chunk, tot);
-    if (threadIdx.x != 0) return;
-    // state through global-qualified accesses (a chain of generic accesses
-    // in one thread waits on both the vector-memory and the scalar counters)
-    double T12[16];
-    for (int i = 0; i < 16; ++i) T12[i] = ldg(st->T_12, i);
-    stg(&st->solves, 0, ldg(&st->solves, 0) + 1);
-    const SolveResult r = solve_totals(P, tot, T12);
-    if (r.failed) {
-        stg(&st->icp_failed, 0, r.failed);
-    } else if (r.converged) {
-        stg(&st->conv_level, 0, level);
-    } else {
-        double T21[16];
-        rigid_inverse(T12, T21);
-        for (int i = 0; i < 16; ++i) {
-            stg(st->T_12, i, T12[i]);
-            stg(st->T_21, i, T21[i]);
-            stg(st->T_21_f, i, (float)T21[i]);
-        }
+    if (level >= P.levels) return;
+    const int ng = icp_groups(P.lev[level].tiles_x * P.lev[level].tiles_y, level);
+    PartialSums<THREADS> sums;
+    sums.load(P.icp_part, ng, 0);  // in flight during the tests
+    const double t12 = ldg(st->T_12, threadIdx.x & 15);
+    const int solves = ldg(&st->solves, 0);
+    if (icp_skip(P, st, level, iter)) return;
+    if (threadIdx.x < 16) T12[threadIdx.x] = t12;
+    sums.finish(P.icp_part, ng, pair, tot);
+    if (threadIdx.x >= 64) return;
+    const SolveResult r = solve_wave(P, tot, T12);
+    if (threadIdx.x == 0) {
+        stg(&st->solves, 0, solves + 1);
+        if (r.failed) stg(&st->icp_failed, 0, r.failed);
+        else if (r.converged) stg(&st->conv_level, 0, level);
+    }
+    if (!r.updated) return;
+    if (threadIdx.x < 16) T12[threadIdx.x] = r.t12;
+    __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses are in order
+    const double t21 = rigid_inverse_lane(T12);
+    if (threadIdx.x < 16) {
+        stg(st->T_12, threadIdx.x, r.t12);
+        stg(st->T_21, threadIdx.x, t21);
+        stg(st->T_21_f, threadIdx.x, (float)t21);
     }
 }
 
@@ -588,49 +651,70 @@ __global__ __launch_bounds__(THREADS) void k_icp_solve(const SessParams *__restr
 // workgroups do not read.
 constexpr int kStepThreads = 1024;
 struct StepShared {
-    double chunk[kSumChunks][kIcpVals], tot[kIcpVals];
+    double pair[kSumPairs][kIcpVals], tot[kIcpVals];
     double T12[16];
     float T21f[16];
     int failed, conv_level, solves;
 };
+// What a launch needs before it can go on, all loads in flight together: both
+// records, the tracker's flags, and the partials it expects to find pending,
+// those of the launch before (level prev, -1: none) in the half that alternates
+// with seq. (Flags, then records, then partials, each waited for: a workgroup
+// began its solve after 7000 cycles of its 27000.)
+struct StepLoads {
+    vs_u4 a0, a1;  // seq, pending, failed, conv_level
+    int n0, n1;    // solves
+    double t0, t1;
+    int track, single;
+    PartialSums<kStepThreads> sums;
+    // part, ng: the expected partials (ng 0: none)
+    __device__ __forceinline__ void load(const SessState *st, const double *part, int ng) {
+        a0 = ldg((const vs_u4 *)&st->step[0].seq, 0);
+        a1 = ldg((const vs_u4 *)&st->step[1].seq, 0);
+        n0 = ldg(&st->step[0].solves, 0);
+        n1 = ldg(&st->step[1].solves, 0);
+        t0 = ldg(st->step[0].T_12, threadIdx.x & 15);
+        t1 = ldg(st->step[1].T_12, threadIdx.x & 15);
+        track = ldg(&st->do_track, 0);
+        single = ldg(&st->force_single, 0);
+        sums.load(part, ng, 0);
+    }
+};
 // Brings the loop up to date into sh (all threads); returns the record it
 // started from. seq: only records of earlier launches count.
-__device__ __forceinline__ int step_resume(const SessParams &P, const SessState *st, int seq, StepShared &sh) {
-    // both records at once: seq, pending, failed, conv_level; solves
-    const vs_u4 a0 = ldg((const vs_u4 *)&st->step[0].seq, 0), a1 = ldg((const vs_u4 *)&st->step[1].seq, 0);
-    const int n0 = ldg(&st->step[0].solves, 0), n1 = ldg(&st->step[1].solves, 0);
-    const double t0 = ldg(st->step[0].T_12, threadIdx.x & 15), t1 = ldg(st->step[1].T_12, threadIdx.x & 15);
-    const int s0 = (int)a0.x, s1 = (int)a1.x;
+__device__ __forceinline__ int step_resume(const SessParams &P, StepLoads &ld, int seq, int prev, StepShared &sh) {
+    const int s0 = (int)ld.a0.x, s1 = (int)ld.a1.x;
     const int cur = (int)(s1 < seq) & ((int)(s0 >= seq) | (int)(s1 > s0));
-    const vs_u4 S = cur ? a1 : a0;
+    const vs_u4 S = cur ? ld.a1 : ld.a0;
     const int pending = (int)S.y;
-    if (threadIdx.x < 16) sh.T12[threadIdx.x] = cur ? t1 : t0;
+    if (threadIdx.x < 16) sh.T12[threadIdx.x] = cur ? ld.t1 : ld.t0;
     if (threadIdx.x == 16) {
         sh.failed = (int)S.z;
         sh.conv_level = (int)S.w;
-        sh.solves = cur ? n1 : n0;
+        sh.solves = cur ? ld.n1 : ld.n0;
     }
     if (pending >= 0) {
-        const LevelDesc &L = P.lev[pending];
-        sum_partials<kStepThreads>(P.icp_part + (size_t)cur * P.icp_half, icp_groups(L.tiles_x * L.tiles_y, pending),
-                                   sh.chunk, sh.tot);
+        const double *part = P.icp_part + (size_t)cur * P.icp_half;
+        const int ng = icp_groups(P.lev[pending].tiles_x * P.lev[pending].tiles_y, pending);
+        // not where they were expected: a session with fewer levels than the batch
+        if (pending != prev || cur != ((seq - 1) & 1)) ld.sums.load(part, ng, 0);
+        ld.sums.finish(part, ng, sh.pair, sh.tot);
     } else {
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        double T12[16];
-        for (int i = 0; i < 16; ++i) T12[i] = sh.T12[i];
+    if (threadIdx.x < 64) {
         if (pending >= 0) {
-            const SolveResult r = solve_totals(P, sh.tot, T12);
-            sh.solves += 1;
-            if (r.failed) sh.failed = r.failed;
-            else if (r.converged) sh.conv_level = pending;
-            else
-                for (int i = 0; i < 16; ++i) sh.T12[i] = T12[i];
+            const SolveResult r = solve_wave(P, sh.tot, sh.T12);
+            if (threadIdx.x == 0) {
+                sh.solves += 1;
+                if (r.failed) sh.failed = r.failed;
+                else if (r.converged) sh.conv_level = pending;
+            }
+            if (r.updated && threadIdx.x < 16) sh.T12[threadIdx.x] = r.t12;
         }
-        double T21[16];
-        rigid_inverse(T12, T21);
-        for (int i = 0; i < 16; ++i) sh.T21f[i] = (float)T21[i];
+        __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses are in order
+        const double t21 = rigid_inverse_lane(sh.T12);
+        if (threadIdx.x < 16) sh.T21f[threadIdx.x] = (float)t21;
     }
     __syncthreads();
     return cur;
@@ -650,8 +734,7 @@ struct WidePixels {
     static constexpr int N = G / 4;  // tiles per wave
     int xs[N], ys[N];
     float td[N];
-    __device__ __forceinline__ void load(const SessParams &P, int level, int t0) {
-        const LevelDesc &L = P.lev[level];
+    __device__ __forceinline__ void load(const LevelDesc &L, const float *filt, int t0) {
         const int ntiles = L.tiles_x * L.tiles_y;
         const int wave = threadIdx.x >> 6, tt = (wave & 3) * 64 + (threadIdx.x & 63);  // thread of the tile
 #pragma unroll
@@ -660,14 +743,14 @@ struct WidePixels {
             xs[j] = (tile % L.tiles_x) * kTileW + tt % kTileW;
             ys[j] = (tile / L.tiles_x) * kTileH + tt / kTileW;
             const bool in = tile < ntiles && xs[j] < L.W && ys[j] < L.H;
-            const float d = ldg(P.filt[level], in ? (size_t)ys[j] * L.W + xs[j] : (size_t)0);
+            const float d = ldg(filt, in ? (size_t)ys[j] * L.W + xs[j] : (size_t)0);
             td[j] = in ? d : 0.0f;
         }
     }
 };
 template <int G>
 __device__ __forceinline__ void group_sums_wide(const SessParams &P, int level, const WidePixels<G> &px,
-                                                const float *T21s, double *out) {
+                                                const float *T21s, double *out, int ti, int tj) {
     constexpr int N = WidePixels<G>::N;
     __shared__ __align__(16) float feat[4][G][64][8];
     __shared__ float gw[4][8][8];
@@ -704,33 +787,39 @@ __device__ __forceinline__ void group_sums_wide(const SessParams &P, int level, 
     }
     __syncthreads();
     if (threadIdx.x < kIcpVals) {
-        int i, j;
-        term_ij(threadIdx.x, i, j);
         double s = 0.0;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) s += (double)gw[w][i][j];
+        for (int w = 0; w < 4; ++w) s += (double)gw[w][ti][tj];
         stg(out, threadIdx.x, s);
     }
 }
 
+// prev: level of launch seq - 1 (-1: none)
 template <int G>
 __global__ __launch_bounds__(kStepThreads) void k_icp_step(const SessParams *__restrict__ SP,
                                                            const WorkItem *__restrict__ work, int level, int iter,
-                                                           int seq) {
+                                                           int seq, int prev) {
     __shared__ StepShared sh;
     const WorkItem wi = work ? work[blockIdx.x] : WorkItem{0, (int)blockIdx.x};
-    const SessParams &P = SP[wi.sess];
+    const SessParams &P = SP[__builtin_amdgcn_readfirstlane(wi.sess)];
+    // read now, with the sizes tested below, not in a round of its own after them
     SessState *st = P.st;
-    if (level >= P.levels) return;
+    double *part = P.icp_part;
+    const float *filt = P.filt[level];
+    int half = P.icp_half, nprev = prev < 0 ? 0 : P.lev[prev].tiles_x * P.lev[prev].tiles_y;
+    asm volatile("" : "+s"(st), "+s"(part), "+s"(filt), "+s"(half), "+s"(nprev));
     const LevelDesc &L = P.lev[level];
     const int t0 = wi.tile * G;
-    if (t0 >= L.tiles_x * L.tiles_y) return;
-    const int track = ldg(&st->do_track, 0), single = ldg(&st->force_single, 0);
+    if ((int)(level >= P.levels) | (int)(t0 >= L.tiles_x * L.tiles_y)) return;
+    StepLoads ld;
+    ld.load(st, part + (size_t)((seq - 1) & 1) * half, icp_groups(nprev, prev));
     WidePixels<G> px;
-    px.load(P, level, t0);  // in flight during the solve
-    if (!track) return;
-    const int out = step_resume(P, st, seq, sh) ^ 1;
-    const bool skip = sh.failed || sh.conv_level == level || iter >= P.iters[level] || (single && level != 0);
+    px.load(L, filt, t0);  // in flight during the solve
+    int ti, tj;
+    term_ij(threadIdx.x < kIcpVals ? threadIdx.x : 0, ti, tj);
+    if (!ld.track) return;
+    const int out = step_resume(P, ld, seq, prev, sh) ^ 1;
+    const bool skip = sh.failed || sh.conv_level == level || iter >= P.iters[level] || (ld.single && level != 0);
     if (wi.tile == 0) {
         IcpStep *S = &st->step[out];
         if (threadIdx.x < 16) stg(S->T_12, threadIdx.x, sh.T12[threadIdx.x]);
@@ -743,7 +832,7 @@ __global__ __launch_bounds__(kStepThreads) void k_icp_step(const SessParams *__r
         }
     }
     if (skip) return;
-    group_sums_wide<G>(P, level, px, sh.T21f, P.icp_part + (size_t)out * P.icp_half + (size_t)wi.tile * kIcpVals);
+    group_sums_wide<G>(P, level, px, sh.T21f, P.icp_part + (size_t)out * P.icp_half + (size_t)wi.tile * kIcpVals, ti, tj);
 }
 #endif
 
@@ -877,7 +966,8 @@ __global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess, u
 }
 // The same after the one-launch iterations: one workgroup per session solves
 // the last one first.
-__global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *__restrict__ SP, unsigned *bricks) {
+__global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *__restrict__ SP, unsigned *bricks,
+                                                             int seq, int prev) {
     __shared__ StepShared sh;
     if (blockIdx.x == 0 && threadIdx.x == 0) *bricks = 0u;
     const SessParams &P = SP[blockIdx.x];
@@ -886,8 +976,11 @@ __global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *_
         if (threadIdx.x == 0) st->fuse_ok = 0;
         return;
     }
-    if (st->do_track) {
-        step_resume(P, st, 0x7FFFFFFF, sh);
+    StepLoads ld;
+    ld.load(st, P.icp_part + (size_t)((seq - 1) & 1) * P.icp_half,
+            prev < 0 ? 0 : icp_groups(P.lev[prev].tiles_x * P.lev[prev].tiles_y, prev));
+    if (ld.track) {
+        step_resume(P, ld, seq, prev, sh);
         if (threadIdx.x == 0) {
             for (int i = 0; i < 16; ++i) st->T_12[i] = sh.T12[i];
             st->icp_failed = sh.failed;
@@ -1004,19 +1097,23 @@ void launch_icp_iter(const SessParams *P, const WorkItem *work, int n, int nsess
     else
         hipLaunchKernelGGL(k_icp_solve<kTileThreads>, dim3(nsess), dim3(kTileThreads), 0, s, P, nsess, level, iter);
 }
-void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level, int iter, int seq, hipStream_t s) {
+void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level, int iter, int seq, int prev,
+                     hipStream_t s) {
     if (n <= 0) return;
 #if VS_ICP_MFMA
     if (level == 0)
-        hipLaunchKernelGGL(k_icp_step<icp_group(0)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq);
+        hipLaunchKernelGGL(k_icp_step<icp_group(0)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq,
+                           prev);
     else if (level == 1)
-        hipLaunchKernelGGL(k_icp_step<icp_group(1)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq);
+        hipLaunchKernelGGL(k_icp_step<icp_group(1)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq,
+                           prev);
     else
-        hipLaunchKernelGGL(k_icp_step<icp_group(2)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq);
+        hipLaunchKernelGGL(k_icp_step<icp_group(2)>, dim3(n), dim3(kStepThreads), 0, s, P, work, level, iter, seq,
+                           prev);
 #endif
 }
-void launch_icp_finish(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s) {
-    hipLaunchKernelGGL(k_icp_finish, dim3(nsess), dim3(kStepThreads), 0, s, P, bricks);
+void launch_icp_finish(const SessParams *P, int nsess, unsigned *bricks, int seq, int prev, hipStream_t s) {
+    hipLaunchKernelGGL(k_icp_finish, dim3(nsess), dim3(kStepThreads), 0, s, P, bricks, seq, prev);
 }
 void launch_track_finalize(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s) {
     hipLaunchKernelGGL(k_track_finalize, dim3((nsess + 63) / 64), dim3(64), 0, s, P, nsess, bricks);

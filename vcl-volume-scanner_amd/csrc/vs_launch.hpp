@@ -52,10 +52,12 @@ void launch_track_finalize(const SessParams *P, int nsess, unsigned *bricks, hip
 // (1280x960) 1125 / 1246 and a 24-slot server's 2291 1295 / 1359 (these two
 // with a shorter solve on both sides).
 constexpr int kIcpStepGroups = VS_ICP_STEP_GROUPS;
-// seq: 1, 2, ... over the launches of one track; work null: a single session's groups 0..n-1
-void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level, int iter, int seq, hipStream_t s);
+// seq: 1, 2, ... over the launches of one track; prev: the level of launch seq - 1
+// (-1: none); work null: a single session's groups 0..n-1
+void launch_icp_step(const SessParams *P, const WorkItem *work, int n, int level, int iter, int seq, int prev,
+                     hipStream_t s);
 // the last iteration's solve, then launch_track_finalize's work
-void launch_icp_finish(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s);
+void launch_icp_finish(const SessParams *P, int nsess, unsigned *bricks, int seq, int prev, hipStream_t s);
 // integrate_begin alone, for an integration without a track (single session)
 void launch_integrate_begin(const SessParams *P, unsigned *bricks, hipStream_t s);
 // one system, no solve: writes 29 doubles (+ optional mask) for diagnostics
