@@ -15,6 +15,8 @@
 // decrease, so the bit is set once and kept) and the band bits `bband` /
 // `sband` (bricks / superbricks that may hold a voxel of weight > 0 and a value
 // other than 1.0; set when an update writes such a value, and kept).
+#include <type_traits>
+
 #include "vs_device.hpp"
 #include "vs_launch.hpp"
 
@@ -527,12 +529,25 @@ __device__ __forceinline__ bool below3(int x, int y, int z, int nx, int ny, int 
     return (int)((unsigned)x < (unsigned)nx) & (int)((unsigned)y < (unsigned)ny) & (int)((unsigned)z < (unsigned)nz);
 }
 
+// ROUNDF of a finite coordinate (v - 0.5 below zero, else v + 0.5, truncated)
+// without a select.
+__device__ __forceinline__ int round_half(float v) { return (int)(v + copysignf(0.5f, v)); }
+
 // A voxel outside the grid on an axis along which the ray moves away or not
 // at all.
 __device__ __forceinline__ bool leaves3(int x, int y, int z, int nx, int ny, int nz, f3 rd) {
     return (int)(x < 0 && !(rd.x > 0.0f)) | (int)(x >= nx && !(rd.x < 0.0f)) | (int)(y < 0 && !(rd.y > 0.0f)) |
            (int)(y >= ny && !(rd.y < 0.0f)) | (int)(z < 0 && !(rd.z > 0.0f)) | (int)(z >= nz && !(rd.z < 0.0f));
 }
+
+// A region whose voxels all read 1.0: the cell of 2^sh voxels an edge with
+// lower corner lo, and r such cells around it on every side (parts of it
+// outside the grid read 1.0 as well).
+struct FreeBox {
+    int3 lo;
+    int sh, r;
+};
+constexpr int kNoBox = -1, kBeforeGrid = -2;  // r: no region; outside the grid, moving towards it
 
 // AD (VoxAddr): 32- or 64-bit record offsets, superbrick size known or read
 // from the session.
@@ -602,6 +617,35 @@ struct Vol {
         out = ok ? R::val(r) : 1.0f;
         return ok;
     }
+    // Byte offsets of the 2x2x2 stencil's records at (ox, oy, oz) as sums of
+    // one part per axis: (x >> 3) * 512 + (x & 7) = x + 63 * (x & ~7) along x,
+    // a row of bd0 bricks per 8 along y, bd01 bricks per 8 along z (24-bit
+    // products: < 2^24 bricks), so a corner costs one three-operand addition.
+    struct Corners {
+        typedef typename std::conditional<O32, unsigned, size_t>::type Off;
+        unsigned X[2], Y[2];
+        Off Z[2];
+        __device__ __forceinline__ Corners(int ox, int oy, int oz, unsigned bd0, unsigned bd01) {
+            constexpr unsigned B = sizeof(typename VoxRec<TV, TW>::T);
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const unsigned x = (unsigned)(ox + a), y = (unsigned)(oy + a), z = (unsigned)(oz + a);
+                X[a] = __umul24(x & ~7u, 63u * B) + x * B;
+                Y[a] = __umul24(y >> 3, bd0 * (kBrickVox * B)) + ((y * (8u * B)) & (56u * B));
+                Z[a] = (Off)__umul24(z >> 3, bd01) * (kBrickVox * B) + ((z * (64u * B)) & (448u * B));
+            }
+        }
+        // corner k: bit 0 x, bit 1 y, bit 2 z
+        __device__ __forceinline__ Off at(int k) const { return (Off)(X[k & 1] + Y[(k >> 1) & 1]) + Z[k >> 2]; }
+    };
+    __device__ __forceinline__ typename VoxRec<TV, TW>::T rec_at(typename Corners::Off byte) const {
+        return *(const VS_GLOBAL typename VoxRec<TV, TW>::T *)((const VS_GLOBAL char *)vx + byte);
+    }
+    // the cell of 2^sh voxels an edge around voxel (x, y, z), and r more
+    static __device__ __forceinline__ FreeBox box_at(int x, int y, int z, int sh, int r) {
+        const int m = (int)(~0u << sh);
+        return {make_int3(x & m, y & m, z & m), sh, r};
+    }
     // the record of voxel b * 512 + l
     __device__ __forceinline__ typename VoxRec<TV, TW>::T rec_bl(unsigned b, unsigned l) const {
         return O32 ? ld_rec32<TV, TW>(vx, (b << 9) | l) : ld_rec<TV, TW>(vx, (size_t)b * kBrickVox + l);
@@ -620,23 +664,19 @@ struct Vol {
     // lies outside the grid on an axis along which the ray moves away or not
     // at all: every later position of a ray that keeps stepping forward is
     // then outside as well. For 0 it also reports what the lookup learnt
-    // about the neighbourhood: size > 0 when every voxel of the box
-    // [lo, lo + size)^3 (a superbrick or brick without band bit) reads 1.0,
-    // size = -1 when the position is outside the grid (moving towards it),
-    // size = 0 otherwise.
-    __device__ __forceinline__ int nearest(f3 v, f3 rd, float &out, int3 &lo, int &size) const {
+    // about the neighbourhood: the box of voxels that read 1.0 (superbricks
+    // without a band brick, or a brick without band bit), kBeforeGrid or kNoBox.
+    __device__ __forceinline__ int nearest(f3 v, f3 rd, float &out, FreeBox &box) const {
         out = 1.0f;
-        size = 0;
+        box.r = kNoBox;
         // the tests of the three axes are combined with & rather than &&:
         // one exec-mask branch instead of a nest of six, each with its own
         // mask bookkeeping (the march loop's instruction issue is its bound)
         if (!finite3(v)) return 0;
-        const int x = v.x < 0.0f ? (int)(v.x - 0.5f) : (int)(v.x + 0.5f);  // ROUNDF
-        const int y = v.y < 0.0f ? (int)(v.y - 0.5f) : (int)(v.y + 0.5f);
-        const int z = v.z < 0.0f ? (int)(v.z - 0.5f) : (int)(v.z + 0.5f);
+        const int x = round_half(v.x), y = round_half(v.y), z = round_half(v.z);
         if (!below3(x, y, z, P.vdim[0], P.vdim[1], P.vdim[2])) {
             if (leaves3(x, y, z, P.vdim[0], P.vdim[1], P.vdim[2], rd)) return -1;
-            size = -1;
+            box.r = kBeforeGrid;
             return 0;
         }
         if (!band(x, y, z)) {
@@ -644,9 +684,7 @@ struct Vol {
             // superbrick); d > 0: the (2d-1)^3 superbricks centred here,
             // which hold no band brick
             const int d = dist();
-            const int sh = d == 0 ? 3 : super_log2(), r = max(d - 1, 0), unit = 1 << sh;
-            lo = make_int3(((x >> sh) - r) * unit, ((y >> sh) - r) * unit, ((z >> sh) - r) * unit);
-            size = (2 * r + 1) * unit;
+            box = box_at(x, y, z, d == 0 ? 3 : super_log2(), max(d - 1, 0));
             return 0;
         }
         return load_bl((unsigned)cb(), (unsigned)(((z & 7) << 6) | ((y & 7) << 3) | (x & 7)), out) ? 1 : 0;
@@ -708,28 +746,15 @@ struct Vol {
         // 0 <= o and o + 1 < vdim on every axis
         if (!below3(ox, oy, oz, P.vdim[0] - 1, P.vdim[1] - 1, P.vdim[2] - 1)) return false;
         const float rx = v.x - (float)ox, ry = v.y - (float)oy, rz = v.z - (float)oz;
-        // vox_index of the 8 corners from per-axis parts: brick index
-        // bz*bdim1*bdim0 + by*bdim0 + bx (24-bit products: < 2^24 bricks)
-        // and in-brick offset lz*64 + ly*8 + lx of the two coordinates on
-        // each axis
-        const unsigned bd0 = (unsigned)P.bdim[0], bd01 = (unsigned)(P.bdim[0] * P.bdim[1]);
-        unsigned Bx[2], By[2], Bz[2], Lx[2], Ly[2], Lz[2];
-#pragma unroll
-        for (int a = 0; a < 2; ++a) {
-            Bx[a] = (unsigned)(ox + a) >> 3;
-            By[a] = __umul24((unsigned)(oy + a) >> 3, bd0);
-            Bz[a] = __umul24((unsigned)(oz + a) >> 3, bd01);
-            Lx[a] = (unsigned)(ox + a) & 7u;
-            Ly[a] = ((unsigned)(oy + a) & 7u) << 3;
-            Lz[a] = ((unsigned)(oz + a) & 7u) << 6;
-        }
+        const Corners c(ox, oy, oz, (unsigned)P.bdim[0], (unsigned)(P.bdim[0] * P.bdim[1]));
         float f[8];
         bool ok = true;
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const unsigned b = Bz[k >> 2] + By[(k >> 1) & 1] + Bx[k & 1];
-            const unsigned l = Lz[k >> 2] | Ly[(k >> 1) & 1] | Lx[k & 1];
-            ok &= load_bl(b, l, f[k]);
+            typedef VoxRec<TV, TW> R;
+            const typename R::T r = rec_at(c.at(k));
+            ok &= R::has_w(r);
+            f[k] = R::val(r);
         }
         if (!ok) return false;
         const float fi = (1.0f - ry) * ((1.0f - rx) * f[0] + rx * f[1]) + ry * ((1.0f - rx) * f[2] + rx * f[3]);
@@ -761,20 +786,26 @@ struct RayConst {
 constexpr int kSkipMax = 64;
 constexpr float kSkipMargin = 0.25f;
 
-// rounded position inside [lo, lo + size)^3 clipped to the grid:
-// v in [lo - 0.5, hi + 0.5) on each axis
-__device__ __forceinline__ int steps_in_box(f3 v, f3 d, int3 lo, int size, int nx, int ny, int nz) {
-    float k = (float)kSkipMax;
-    const float vv[3] = {v.x, v.y, v.z}, dd[3] = {d.x, d.y, d.z};
-    const int ll[3] = {lo.x, lo.y, lo.z}, vdim[3] = {nx, ny, nz};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        const float hi = (float)min(ll[a] + size - 1, vdim[a] - 1);
-        const float bound = dd[a] > 0.0f ? hi + 0.5f - kSkipMargin : (float)ll[a] - 0.5f + kSkipMargin;
-        const float t = (bound - vv[a]) * __builtin_amdgcn_rcpf(dd[a]);
-        k = dd[a] != 0.0f ? fminf(k, t) : k;
-    }
-    return k >= 1.0f ? (int)k : 0;
+// Rounded position inside the box: |v - m| < (r + 1/2) * 2^sh on each axis,
+// m the cell's middle. The box need not be clipped to the grid: a ray inside
+// the grid leaves it for good, and the iteration after the skip ends it as the
+// miss that it is. With t = (reach - sign(d) (v - m)) / |d| an axis costs 7
+// operations; an axis the ray does not move along gives NaN or infinity, which
+// the minimum passes over. (Bounds picked by the direction's sign and clipped
+// to the grid, and the trilinear corners as brick and in-brick offsets, had
+// been 100 of ~400 vector operations of a loop iteration: 64-session step 6.62
+// -> 6.32 ms, 1280x960 scan into 1024^3 1166 -> 1127 us, 640x480 scan 413 ->
+// 403, 264x200x312 render 100 -> 95.)
+__device__ __forceinline__ int steps_in_box(f3 v, f3 d, const FreeBox &box) {
+    const float unit = (float)(1 << box.sh), mid = 0.5f * unit - 0.5f;
+    const float reach = (float)box.r * unit + (0.5f * unit - kSkipMargin);
+    const auto steps = [&](float a, float da, int lo) {
+        const float rc = __builtin_amdgcn_rcpf(da);
+        return fmaf(-((a - (float)lo) - mid), rc, reach * fabsf(rc));
+    };
+    const float k = fminf(fminf(steps(v.x, d.x, box.lo.x), steps(v.y, d.y, box.lo.y)),
+                          fminf(steps(v.z, d.z, box.lo.z), (float)kSkipMax));
+    return max((int)k, 0);
 }
 
 // rounded position outside the grid: it stays outside while any axis does
@@ -894,17 +925,15 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW, AD> &V, const RayCons
         // A ray that has left the grid for good can only end as a miss
         // (every later tap reads 1.0 and the step stays positive); the
         // instrumented form keeps marching to count the reference's taps.
-        int3 lo;
-        int size;
-        if (V.nearest(vox, rd, tsdf, lo, size) < 0 && !STATS) return false;
-        if (!STATS && size != 0) {
+        FreeBox box;
+        if (V.nearest(vox, rd, tsdf, box) < 0 && !STATS) return false;
+        if (!STATS && box.r != kNoBox) {
             // 1.0 here and in the region around: skip the steps that stay
             // inside it (tsdf is 1.0, so the next step is the same S each time)
             const float S = coarse ? C.step_scale : fmaxf(C.step_scale * tsdf, 1.0f);
             const f3 d = scale(S, rd);
             const int *n = V.P.vdim;
-            const int k = size > 0 ? steps_in_box(vox, d, lo, size, n[0], n[1], n[2])
-                                   : steps_outside(vox, d, n[0], n[1], n[2]);
+            const int k = box.r >= 0 ? steps_in_box(vox, d, box) : steps_outside(vox, d, n[0], n[1], n[2]);
             skip_steps(vox, total, iter, d, S, k);
             if ((int)(iter > C.max_iter) | (int)(total > C.total_max)) return false;
             continue;
@@ -944,8 +973,7 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW, AD> &V, const RayCons
 // branches, and up to three dependent rounds of loads. Here the sizes stay in
 // vector registers, the tests are flags, and one round loads the band word,
 // the nearest record and the eight trilinear corners together (the corners of
-// a stencil that leaves the grid read the nearest record and count as
-// failed). Decisions and values are cast_ray's: the same FP32 operations on
+// a stencil that leaves the grid read the origin's and count as failed). Decisions and values are cast_ray's: the same FP32 operations on
 // the same operands.
 template <class TV, class TW, int AD>
 __device__ __forceinline__ bool cast_ray_latency(const Vol<TV, TW, AD> &V, const RayConst &C, const float *Tcg,
@@ -994,9 +1022,7 @@ __device__ __forceinline__ bool cast_ray_latency(const Vol<TV, TW, AD> &V, const
         total += step;
         const bool fin = finite3(vox);
         const f3 v = {fin ? vox.x : 0.0f, fin ? vox.y : 0.0f, fin ? vox.z : 0.0f};
-        const int x = v.x < 0.0f ? (int)(v.x - 0.5f) : (int)(v.x + 0.5f);  // ROUNDF
-        const int y = v.y < 0.0f ? (int)(v.y - 0.5f) : (int)(v.y + 0.5f);
-        const int z = v.z < 0.0f ? (int)(v.z - 0.5f) : (int)(v.z + 0.5f);
+        const int x = round_half(v.x), y = round_half(v.y), z = round_half(v.z);
         const bool in = (int)fin & (int)below3(x, y, z, nx, ny, nz);
         miss = (int)miss | (int)(iter > C.max_iter) | (int)(total > C.total_max) |
                ((int)fin & (int)!in & (int)leaves3(x, y, z, nx, ny, nz, rd));
@@ -1009,25 +1035,13 @@ __device__ __forceinline__ bool cast_ray_latency(const Vol<TV, TW, AD> &V, const
             const unsigned l = (unsigned)(((z & 7) << 6) | ((y & 7) << 3) | (x & 7));
             const int ox = (int)v.x, oy = (int)v.y, oz = (int)v.z;
             const bool inner = below3(ox, oy, oz, nx - 1, ny - 1, nz - 1);
-            unsigned Bx[2], By[2], Bz[2], Lx[2], Ly[2], Lz[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) {
-                Bx[a] = (unsigned)(ox + a) >> 3;
-                By[a] = __umul24((unsigned)(oy + a) >> 3, bd0);
-                Bz[a] = __umul24((unsigned)(oz + a) >> 3, bd01);
-                Lx[a] = (unsigned)(ox + a) & 7u;
-                Ly[a] = ((unsigned)(oy + a) & 7u) << 3;
-                Lz[a] = ((unsigned)(oz + a) & 7u) << 6;
-            }
+            // a stencil that leaves the grid reads the one at the origin
+            const typename Vol<TV, TW, AD>::Corners c(inner ? ox : 0, inner ? oy : 0, inner ? oz : 0, bd0, bd01);
             const uint32_t word = ldg(bband, b >> 5);
             const typename R::T rn = V.rec_bl(b, l);
             typename R::T rc[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const unsigned cb = Bz[k >> 2] + By[(k >> 1) & 1] + Bx[k & 1];
-                const unsigned cl = Lz[k >> 2] | Ly[(k >> 1) & 1] | Lx[k & 1];
-                rc[k] = V.rec_bl(inner ? cb : b, inner ? cl : l);
-            }
+            for (int k = 0; k < 8; ++k) rc[k] = V.rec_at(c.at(k));
             band = (word >> (b & 31)) & 1u;
             const float tn = R::has_w(rn) ? R::val(rn) : 1.0f;
             near = (int)band & (int)(fabsf(tn) < 1.0f);
@@ -1051,9 +1065,7 @@ __device__ __forceinline__ bool cast_ray_latency(const Vol<TV, TW, AD> &V, const
             const f3 dv = scale(S, rd);
             int k;
             if (in) {
-                const int sh = d == 0 ? 3 : ss, r = max(d - 1, 0), unit = 1 << sh;
-                const int3 lo = make_int3(((x >> sh) - r) * unit, ((y >> sh) - r) * unit, ((z >> sh) - r) * unit);
-                k = steps_in_box(vox, dv, lo, (2 * r + 1) * unit, nx, ny, nz);
+                k = steps_in_box(vox, dv, V.box_at(x, y, z, d == 0 ? 3 : ss, max(d - 1, 0)));
             } else {
                 k = steps_outside(vox, dv, nx, ny, nz);
             }
