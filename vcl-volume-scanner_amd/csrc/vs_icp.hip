@@ -116,9 +116,12 @@ __device__ __forceinline__ IcpPre icp_pre(const SessParams &P, int l, int x, int
     const LevelDesc &L = P.lev[l];
     const int W = L.W, H = L.H;
     IcpPre r;
-    r.p = transform(T21, back_project((float)x, (float)y, L.K, td1));
+    // back_project and project by shared divisors (640x480 level 0: the pixels
+    // are 8000 of an iteration's 23500 cycles, vector issue)
+    r.p = transform(T21, f3{quotient(td1 * ((float)x - L.K[2]), divisor(L.K[0])),
+                            quotient(td1 * ((float)y - L.K[3]), divisor(L.K[1])), td1});
     float u, v;
-    project(r.p, L.K, u, v);
+    project_finite(r.p, L.K, u, v);
     const bool inside = u >= 0.0f && u <= float(W - 1) && v >= 0.0f && v <= float(H - 1);
     r.ok = !(td1 < 1.0e-6f) && inside;
     const float uc = inside ? u : 0.0f, vc = inside ? v : 0.0f;
@@ -138,7 +141,10 @@ __device__ __forceinline__ bool icp_post(const SessParams &P, const IcpPre &r, f
     const float dx = v0.x - p.x, dy = v0.y - p.y, dz = v0.z - p.z;
     ok &= !(dx * dx + dy * dy + dz * dz > P.icp_dist2);
     ok &= bilerp(normal_quad(r.r0, r.r1), r.rx, r.ry, n);
-    n = normalised(n);
+    {
+        const Divisor len = divisor(sqrtf(dot(n, n)));
+        n = scale(quotient(1.0f, len), n);
+    }
     A[0] = ok ? p.z * n.y + (-p.y) * n.z : 0.0f;
     A[1] = ok ? (-p.z) * n.x + p.x * n.z : 0.0f;
     A[2] = ok ? p.y * n.x + (-p.x) * n.y : 0.0f;

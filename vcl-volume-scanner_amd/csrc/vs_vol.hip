@@ -201,7 +201,7 @@ __device__ __forceinline__ bool integrate_voxel_color(const SessParams &P, const
     const LevelDesc &L = P.lev[0];
     const f3 p = transform(T, g);
     float u, v;
-    project(p, L.K, u, v);
+    project_finite(p, L.K, u, v);
     int x, y;
     if (!rint_ref(u, x) || !rint_ref(v, y)) return false;
     if (x < 0 || x > L.W - 1 || y < 0 || y > L.H - 1) return false;
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(kTileThreads) void k_integrate(const SessParams *__
                 for (int q = 0; q < 4; ++q) {
                     const f3 p = transform(T, {gxs[q], gy, gz});
                     float u, v;
-                    project(p, L.K, u, v);
+                    project_finite(p, L.K, u, v);
                     // the pixel tests combined with & (no nest of branches); the
                     // depth is read at pixel 0 for a voxel outside the image
                     const bool fin = (int)(fabsf(u) < 2147483520.0f) & (int)(fabsf(v) < 2147483520.0f);
