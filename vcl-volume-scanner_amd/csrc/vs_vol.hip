@@ -1621,14 +1621,21 @@ void launch_integrate(const SessParams *P, int nsess, BrickList bl, int tt, int 
     launch_sdist(P, nsess, sd_slices, 0, s);
 }
 
-// Launches of up to this many workgroups (the 8 per CU that are resident at
-// once on 256 CUs) take the latency form of the march. Fused frame with a
-// 1200-workgroup preview: 1575 workgroups at 640x480 / 256^3, 532 us in the
-// wide form, 509 in the latency form; 1443 at 603x451 in colour, 615 / 550;
-// three levels of 1260, 300 and 75 workgroups (264x200x312), 155 / 117. Above
-// it the waves' own number hides their latency: 6300 and 4800 workgroups at
-// 1280x960 / 1024^3, 1177 / 1225.
-constexpr int kLatencyGroups = 2048;
+// Launches of up to this many workgroups take the latency form of the march.
+// 2048, the 8 per CU that are resident at once on 256 CUs, for any grid (fused
+// frame with a 1200-workgroup preview: 1575 workgroups at 640x480 / 256^3, 427
+// us in the wide form and 402 in the latency form; 1443 at 603x451 in colour,
+// 503 / 431; three levels of 1260, 300 and 75, 116 / 102). Above it the waves'
+// own number hides their latency, and what counts is each form's work per ray:
+// grids of small superbricks, whose boxes are short, gain from the latency
+// form's fewer branches (6300 workgroups at 1280x960 / 512^3 with 4-byte records
+// 1069 / 992, 3 sessions of 640x480 / 256^3 764 / 703, 16 of 384^3 2039 / 1960,
+// a server's 24168 1112 / 1076; 8-byte records 4700 workgroups 556 / 532, 6300
+// 756 / 751, 12600 equal; 4-byte 33075 equal), larger grids lose (6300 at
+// 1280x960 / 1024^3 1036 / 1074).
+__host__ constexpr int latency_groups(int addr, int rec_bytes) {
+    return addr != kAddrSmall ? 2048 : rec_bytes == 4 ? 32768 : 8192;
+}
 template <class TV, class TW>
 static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int addr,
                     hipStream_t s) {
@@ -1646,7 +1653,7 @@ static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long
     } while (0)
     if (stats)
         hipLaunchKernelGGL((k_raycast<TV, TW, true, kRay8x8, kAddr64, false>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats);
-    else if (n <= kLatencyGroups) {
+    else if (n <= latency_groups(addr, (int)sizeof(typename VoxRec<TV, TW>::T))) {
         if (addr != kAddr64) VS_MARCH_L(kAddr32);
         else VS_MARCH_L(kAddr64);
     } else if (rb == kRay16x4)
