@@ -885,7 +885,9 @@ hipStream_t pick(vs_session *s, vs_stream st) {
 }
 
 // The Gauss-Newton iterations of a batch, coarse to fine, and the pose update.
-void enqueue_track(const Batch &B, hipStream_t s) {
+// integrates: the step goes on to an integration (its counters start from zero).
+void enqueue_track(const Batch &B, bool integrates, hipStream_t s) {
+    unsigned *bricks = integrates ? B.bl.count : nullptr;
     const bool one = B.nGroup[0] <= kIcpStepGroups;  // one launch per iteration
     const bool lone = B.n == 1 && !B.active;             // its groups are 0, 1, ...
     int seq = 0, prev = -1;
@@ -899,9 +901,9 @@ void enqueue_track(const Batch &B, hipStream_t s) {
             }
         }
     if (one)
-        launch_icp_finish(B.dP, B.n, B.bl.count, seq + 1, prev, s);
+        launch_icp_finish(B.dP, B.n, bricks, seq + 1, prev, s);
     else
-        launch_track_finalize(B.dP, B.n, B.bl.count, s);
+        launch_track_finalize(B.dP, B.n, bricks, s);
 }
 
 // The per-frame launch sequence of a batch (so_Scan_Object order).
@@ -918,7 +920,7 @@ void enqueue_step(const Batch &B, hipStream_t s, Timer *timed) {
     mark(1);
     launch_pyramid(B.dP, B.dWork, B.nWork, B.levels, B.pyr_pair, 0, s);
     mark(2);
-    enqueue_track(B, s);
+    enqueue_track(B, true, s);
     mark(3);
     launch_vis_mark(B.dP, B.dWork[0], B.nWork[0], B.n, B.max_words, B.bl, 0, s);
     mark(4);
@@ -1678,7 +1680,7 @@ vs_status vs_track(vs_session *s, const double *T_01_init, vs_stream stream) {
     hipStream_t h = pick(s, stream);
     const Batch &B = s->self;
     launch_track_setup_forced(B.dP, 1, T_01_init, h);
-    enqueue_track(B, h);
+    enqueue_track(B, false, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }

@@ -945,7 +945,9 @@ __device__ __forceinline__ void track_finalize(const SessParams &P, SessState *s
 // What the step's integration counts from zero: the batch's brick list (by the
 // launch's first thread), a session's visible bricks and updated voxels, and
 // whether it gained a band superbrick (every kernel that reads that flag runs
-// after the integration that sets it and before the next reset).
+// after the integration that sets it and before the next reset). A track of
+// its own (bricks null) has no integration behind it and leaves them alone:
+// the counts are the last integration's until the next one.
 __device__ __forceinline__ void integrate_begin(SessState *st) {
     st->vis_count = 0u;
     st->upd_count = 0ull;
@@ -959,7 +961,7 @@ __global__ void k_integrate_begin(const SessParams *__restrict__ SP, unsigned *b
 }
 __global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess, unsigned *bricks) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s == 0) *bricks = 0u;
+    if (s == 0 && bricks) *bricks = 0u;
     if (s >= nsess) return;
     const SessParams &P = SP[s];
     SessState *st = P.st;
@@ -967,7 +969,7 @@ __global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess, u
         st->fuse_ok = 0;
         return;
     }
-    integrate_begin(st);
+    if (bricks) integrate_begin(st);
     track_finalize(P, st);
 }
 // The same after the one-launch iterations: one workgroup per session solves
@@ -975,7 +977,7 @@ __global__ void k_track_finalize(const SessParams *__restrict__ SP, int nsess, u
 __global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *__restrict__ SP, unsigned *bricks,
                                                              int seq, int prev) {
     __shared__ StepShared sh;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *bricks = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0 && bricks) *bricks = 0u;
     const SessParams &P = SP[blockIdx.x];
     SessState *st = P.st;
     if (!st->active) {
@@ -995,7 +997,7 @@ __global__ __launch_bounds__(kStepThreads) void k_icp_finish(const SessParams *_
         }
     }
     if (threadIdx.x == 0) {
-        integrate_begin(st);
+        if (bricks) integrate_begin(st);
         track_finalize(P, st);
     }
 }

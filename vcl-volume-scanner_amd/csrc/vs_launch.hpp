@@ -42,8 +42,9 @@ void launch_track_setup_active(const SessParams *P, int nsess, const int *active
 void launch_set_active(int *active, int nslots, const uint32_t bits[kMaxSlots / 32], hipStream_t s);
 void launch_icp_iter(const SessParams *P, const WorkItem *work, int n, int nsess, int level, int iter,
                      hipStream_t s);
-// bricks: the step's brick counter; this launch and launch_icp_finish also
-// reset it and the sessions' integrate counters (integrate_begin)
+// bricks: the step's brick counter, which this launch and launch_icp_finish
+// then reset with the sessions' integrate counters (integrate_begin); null: no
+// integration follows, the counters stay
 void launch_track_finalize(const SessParams *P, int nsess, unsigned *bricks, hipStream_t s);
 // The one-launch form of an iteration, for launches of up to kIcpStepGroups
 // level-0 groups, a CU each for their 16-wave workgroups. Fused frame with
