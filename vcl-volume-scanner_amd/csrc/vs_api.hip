@@ -71,7 +71,6 @@ struct Layout {
     size_t state, raw, filt[kMaxLevels], mvn[kMaxLevels], mimg[kMaxLevels];
     size_t vox, bvis, vmask, bocc, bband, sband, sdist, sdtmp, icp_part, diag_part, diag_mask, lists, params, stats, keys;
     size_t vcol, rgb, mtex[kMaxLevels];  // colour sessions only (0 otherwise)
-    size_t vnbits[kMaxLevels];            // in-place normal maps: one bit per pixel (vn_words)
     size_t wtab;                          // voxel-centre world coordinates, x then y then z
     size_t total;
     size_t nvox;
@@ -133,7 +132,6 @@ Layout make_layout(const vs_session_desc &d) {
         L.filt[l] = take(n * 4);
         L.mvn[l] = take((n + 1) * 2 * sizeof(MapXYZ));  // vertex + normal per pixel, one padding pixel
         L.mimg[l] = take(n);
-        L.vnbits[l] = take((size_t)vn_words(Wl) * Hl * 8);
     }
     // value and weight of a voxel in one record (4 bytes for FP16 + u8, 8
     // otherwise)
@@ -1669,8 +1667,7 @@ vs_status vs_vertex_normal_maps_inplace(vs_session *s, int level, float *vtx_dev
     if (level < 0 || level >= s->d.levels) return fail(VS_EINVAL, "level %d", level);
     hipStream_t h = pick(s, stream);
     const LevelDesc &ld = s->hp.lev[level];
-    launch_vnmap_inplace(s->self.dP, s->self.dWork[level], s->self.nWork[level], level, ld.W, ld.H,
-                         (unsigned long long *)(s->mem + s->L.vnbits[level]), vtx_dev, nrm_dev, h);
+    launch_vnmap_inplace(s->self.dP, level, ld.W, ld.H, vtx_dev, nrm_dev, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }

@@ -234,13 +234,21 @@ __device__ __forceinline__ VnPixel vn_pixel(const float *D, const float *K, int 
     }
     return r;
 }
-// Without `inv`: every pixel evaluated on the input vertex map (the
-// order-independent form). With it (the reference loop's in-place order,
-// below): one bit per pixel, rows of `nw` 64-bit words, set where the loop
-// invalidates the vertex.
+// Pixel t of the caller's maps: the vertex unless it is gone, the normal if
+// there is one.
+__device__ __forceinline__ void put_vn(const VnPixel &r, bool gone, float *vtx, float *nrm, size_t t) {
+    const bool v = r.valid && !gone;
+    stg(vtx, 3 * t + 0, v ? r.c.x : -100.f);
+    stg(vtx, 3 * t + 1, v ? r.c.y : -100.f);
+    stg(vtx, 3 * t + 2, v ? r.c.z : -100.f);
+    stg(nrm, 3 * t + 0, r.normal ? r.n.x : -100.f);
+    stg(nrm, 3 * t + 1, r.normal ? r.n.y : -100.f);
+    stg(nrm, 3 * t + 2, r.normal ? r.n.z : -100.f);
+}
+// Every pixel evaluated on the input vertex map (the order-independent form).
 __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__restrict__ SP,
                                                         const WorkItem *__restrict__ work, int l, float *vtx,
-                                                        float *nrm, const unsigned long long *inv, int nw) {
+                                                        float *nrm) {
     const WorkItem wi = work[blockIdx.x];
     const SessParams &P = SP[wi.sess];
     const LevelDesc &L = P.lev[l];
@@ -248,23 +256,8 @@ __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__rest
     const int x = (wi.tile % L.tiles_x) * kTileW + threadIdx.x % kTileW;
     const int y = (wi.tile / L.tiles_x) * kTileH + threadIdx.x / kTileW;
     if (x >= W || y >= H) return;
-    VnPixel r = vn_pixel(P.filt[l], L.K, W, H, x, y);
-    bool gone = r.grazing;
-    if (inv) {
-        auto bit = [&](int xx, int yy) -> bool {
-            return xx >= 0 && yy >= 0 && ((ldg(inv, (size_t)yy * nw + (xx >> 6)) >> (xx & 63)) & 1ull);
-        };
-        gone = bit(x, y);
-        r.normal &= !(bit(x - 1, y) || bit(x, y - 1));
-    }
-    const bool v = r.valid && !gone;
-    const size_t t = (size_t)y * W + x;
-    stg(vtx, 3 * t + 0, v ? r.c.x : -100.f);
-    stg(vtx, 3 * t + 1, v ? r.c.y : -100.f);
-    stg(vtx, 3 * t + 2, v ? r.c.z : -100.f);
-    stg(nrm, 3 * t + 0, r.normal ? r.n.x : -100.f);
-    stg(nrm, 3 * t + 1, r.normal ? r.n.y : -100.f);
-    stg(nrm, 3 * t + 2, r.normal ? r.n.z : -100.f);
+    const VnPixel r = vn_pixel(P.filt[l], L.K, W, H, x, y);
+    put_vn(r, r.grazing, vtx, nrm, (size_t)y * W + x);
 }
 
 // The reference CPU loop's in-place order (enm_Estimate_Normal_Map,
@@ -282,10 +275,27 @@ __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__rest
 // resolving each row's runs one at a time in one lane it had taken 3.2 ms a
 // level: frame preparation and the maps of three levels of a 640x480 frame,
 // alone, 9.31 -> 0.19 ms.)
+//
+// The bits live in the caller's vertex map until the last launch writes it, so
+// calls on several streams share nothing: row y's 12 W bytes begin with its
+// bits of c (vn_words(W) words of 64 pixels, bit 0 the leftmost), followed by
+// the ordered bits of row y - 1. The last launch's workgroup for a row finds
+// both in the row that it alone overwrites, and takes the recurrence's step for
+// its row once more. (Bits in a scratch of the session's were 1 us of 54 faster
+// for the 640x480 frame's preparation, and made calls for one session and level
+// on two streams race.) A map is aligned to 4 bytes, hence the half words.
+__device__ __forceinline__ uint32_t *vn_row(float *vtx, int W, int y) { return (uint32_t *)vtx + (size_t)y * 3 * W; }
+__device__ __forceinline__ unsigned long long ld_word(const uint32_t *row, int k) {
+    return (unsigned long long)ldg(row, 2 * k) | (unsigned long long)ldg(row, 2 * k + 1) << 32;
+}
+__device__ __forceinline__ void st_word(uint32_t *row, int k, unsigned long long v) {
+    stg(row, 2 * k, (uint32_t)v);
+    stg(row, 2 * k + 1, (uint32_t)(v >> 32));
+}
 
 // One wave per 64 pixels of a row: word k of row y = bits of c.
-__global__ __launch_bounds__(kTileThreads) void k_vn_graze(const SessParams *__restrict__ SP, int l,
-                                                           unsigned long long *bits, int nw) {
+__global__ __launch_bounds__(kTileThreads) void k_vn_graze(const SessParams *__restrict__ SP, int l, float *vtx,
+                                                           int nw) {
     const SessParams &P = SP[0];
     const LevelDesc &L = P.lev[l];
     const int item = blockIdx.x * (kTileThreads / 64) + (threadIdx.x >> 6);
@@ -294,19 +304,49 @@ __global__ __launch_bounds__(kTileThreads) void k_vn_graze(const SessParams *__r
     const int x = k * 64 + (threadIdx.x & 63);
     const bool c = x < L.W && vn_pixel(P.filt[l], L.K, L.W, L.H, x, y).grazing;
     const unsigned long long m = __ballot(c);
-    if ((threadIdx.x & 63) == 0) stg(bits, (size_t)item, m);
+    if ((threadIdx.x & 63) == 0) st_word(vn_row(vtx, L.W, y), k, m);
 }
 
-// The recurrence, in place on the bits of c: one wave, lane k holds words
-// k * N .. k * N + N - 1 of a row. Along a row, a run of r = c & ~inv(row
-// above) is invalidated at every other pixel from its first: adding the first
-// bits of the runs that start at even columns to r (one addition over the
-// whole row) clears exactly those runs, which tells the runs' parities apart.
-// The addition's carries cross lanes by the generate / propagate masks of the
-// wave. Bound: a chain of ~25 dependent instructions per row; the rows' bits
-// are loaded kAhead rows ahead of their use.
+// One step of the recurrence by one wave, lane k holding words k * N .. k * N +
+// N - 1 of a row: up, the ordered bits of the row above, becomes this row's.
+// Along a row, a run of r = c & ~inv(row above) is invalidated at every other
+// pixel from its first: adding the first bits of the runs that start at even
+// columns to r (one addition over the whole row) clears exactly those runs,
+// which tells the runs' parities apart. The addition's carries cross lanes by
+// the generate / propagate masks of the wave.
 template <int N>
-__global__ __launch_bounds__(64) void k_vn_order(unsigned long long *bits, int nw, int H) {
+__device__ __forceinline__ void vn_order_row(const unsigned long long *c, unsigned long long *up, int lane) {
+    unsigned long long r[N], sum[N];
+#pragma unroll
+    for (int q = 0; q < N; ++q) r[q] = c[q] & ~up[q];
+    // last bit of the previous lane's words
+    unsigned prev = __shfl_up((unsigned)(r[N - 1] >> 63), 1, 64);
+    if (lane == 0) prev = 0u;
+    bool carry = false, prop = true;
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        const unsigned long long first = r[q] & ~((r[q] << 1) | prev);
+        const unsigned long long s = r[q] + (first & 0x5555555555555555ull);
+        sum[q] = s + (carry ? 1ull : 0ull);
+        carry = s < r[q] || sum[q] < s;
+        prop &= sum[q] == ~0ull;
+        prev = (unsigned)(r[q] >> 63);
+    }
+    const unsigned long long G = __ballot(carry), Pr = __ballot(prop);
+    bool in = ((((G << 1) + Pr) ^ Pr) >> lane) & 1ull;  // carry into this lane's first word
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        sum[q] += in ? 1ull : 0ull;
+        in = in && sum[q] == 0ull;
+        up[q] = r[q] & ((~sum[q] & 0x5555555555555555ull) | (sum[q] & 0xAAAAAAAAAAAAAAAAull));
+    }
+}
+
+// The recurrence over all rows by one wave: the ordered bits of the row above
+// into each row. Bound: a chain of ~25 dependent instructions per row; the
+// rows' bits are loaded kAhead rows ahead of their use.
+template <int N>
+__global__ __launch_bounds__(64) void k_vn_order(float *vtx, int nw, int W, int H) {
     constexpr int kAhead = 16;
     const int lane = threadIdx.x;
     unsigned long long up[N], nxt[kAhead][N];
@@ -318,7 +358,7 @@ __global__ __launch_bounds__(64) void k_vn_order(unsigned long long *bits, int n
 #pragma unroll
             for (int q = 0; q < N; ++q) {
                 const int k = lane * N + q;
-                nxt[a][q] = (k < nw && row0 + a < H) ? ldg(bits, (size_t)(row0 + a) * nw + k) : 0ull;
+                nxt[a][q] = (k < nw && row0 + a < H) ? ld_word(vn_row(vtx, W, row0 + a), k) : 0ull;
             }
     };
     fetch(0);
@@ -331,33 +371,53 @@ __global__ __launch_bounds__(64) void k_vn_order(unsigned long long *bits, int n
         fetch(row0 + kAhead);
 #pragma unroll
         for (int a = 0; a < kAhead; ++a) {
-            unsigned long long r[N], sum[N];
-#pragma unroll
-            for (int q = 0; q < N; ++q) r[q] = cur[a][q] & ~up[q];
-            // last bit of the previous lane's words
-            unsigned prev = __shfl_up((unsigned)(r[N - 1] >> 63), 1, 64);
-            if (lane == 0) prev = 0u;
-            bool carry = false, prop = true;
 #pragma unroll
             for (int q = 0; q < N; ++q) {
-                const unsigned long long first = r[q] & ~((r[q] << 1) | prev);
-                const unsigned long long s = r[q] + (first & 0x5555555555555555ull);
-                sum[q] = s + (carry ? 1ull : 0ull);
-                carry = s < r[q] || sum[q] < s;
-                prop &= sum[q] == ~0ull;
-                prev = (unsigned)(r[q] >> 63);
-            }
-            const unsigned long long G = __ballot(carry), Pr = __ballot(prop);
-            bool in = ((((G << 1) + Pr) ^ Pr) >> lane) & 1ull;  // carry into this lane's first word
-#pragma unroll
-            for (int q = 0; q < N; ++q) {
-                sum[q] += in ? 1ull : 0ull;
-                in = in && sum[q] == 0ull;
-                up[q] = r[q] & ((~sum[q] & 0x5555555555555555ull) | (sum[q] & 0xAAAAAAAAAAAAAAAAull));
                 const int k = lane * N + q;
-                if (k < nw && row0 + a < H) stg(bits, (size_t)(row0 + a) * nw + k, up[q]);
+                if (k < nw && row0 + a < H) st_word(vn_row(vtx, W, row0 + a), nw + k, up[q]);
             }
+            vn_order_row<N>(cur[a], up, lane);
         }
+    }
+}
+
+// The maps, one workgroup per row: its ordered bits and the row above's into
+// LDS by the first wave, then the row's pixels over what they were read from.
+// A thread per pixel of the row while the workgroup holds them.
+template <int N>
+__global__ __launch_bounds__(1024) void k_vnmap_rows(const SessParams *__restrict__ SP, int l, float *vtx,
+                                                              float *nrm, int nw) {
+    __shared__ unsigned long long here[64 * N], above[64 * N];
+    const SessParams &P = SP[0];
+    const LevelDesc &L = P.lev[l];
+    const int W = L.W, y = blockIdx.x;
+    unsigned long long c[N], up[N];
+    if (threadIdx.x < 64) {
+        const uint32_t *row = vn_row(vtx, W, y);
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+            const int k = threadIdx.x * N + q;
+            c[q] = k < nw ? ld_word(row, k) : 0ull;
+            up[q] = k < nw ? ld_word(row, nw + k) : 0ull;
+        }
+    }
+    int x = threadIdx.x;
+    VnPixel r{};
+    if (x < W) r = vn_pixel(P.filt[l], L.K, W, L.H, x, y);  // its loads in flight with the bits
+    if (threadIdx.x < 64) {
+#pragma unroll
+        for (int q = 0; q < N; ++q) above[threadIdx.x * N + q] = up[q];
+        vn_order_row<N>(c, up, threadIdx.x);
+#pragma unroll
+        for (int q = 0; q < N; ++q) here[threadIdx.x * N + q] = up[q];
+    }
+    __syncthreads();
+    const auto bit = [](const unsigned long long *b, int i) -> bool { return i >= 0 && ((b[i >> 6] >> (i & 63)) & 1ull); };
+    while (x < W) {
+        r.normal &= !(bit(here, x - 1) || bit(above, x));
+        put_vn(r, bit(here, x), vtx, nrm, (size_t)y * W + x);
+        x += blockDim.x;
+        if (x < W) r = vn_pixel(P.filt[l], L.K, W, L.H, x, y);
     }
 }
 
@@ -430,21 +490,20 @@ void launch_pyramid(const SessParams *P, const WorkItem *const work[kMaxLevels],
 }
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int l, float *vtx, float *nrm, hipStream_t s) {
     if (n > 0)
-        hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm,
-                           (const unsigned long long *)nullptr, 0);
+        hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm);
 }
-void launch_vnmap_inplace(const SessParams *P, const WorkItem *work, int n, int l, int W, int H,
-                          unsigned long long *bits, float *vtx, float *nrm, hipStream_t s) {
-    if (n <= 0) return;
+void launch_vnmap_inplace(const SessParams *P, int l, int W, int H, float *vtx, float *nrm, hipStream_t s) {
     const int nw = vn_words(W);  // at most 128 (frames are at most 8192 wide)
     const size_t items = (size_t)nw * H, per = kTileThreads / 64;
-    hipLaunchKernelGGL(k_vn_graze, dim3((unsigned)((items + per - 1) / per)), dim3(kTileThreads), 0, s, P, l, bits, nw);
-    if (nw <= 64)
-        hipLaunchKernelGGL(k_vn_order<1>, dim3(1), dim3(64), 0, s, bits, nw, H);
-    else
-        hipLaunchKernelGGL(k_vn_order<2>, dim3(1), dim3(64), 0, s, bits, nw, H);
-    hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm,
-                       (const unsigned long long *)bits, nw);
+    const dim3 row(std::min(nw * 64, 1024));
+    hipLaunchKernelGGL(k_vn_graze, dim3((unsigned)((items + per - 1) / per)), dim3(kTileThreads), 0, s, P, l, vtx, nw);
+    if (nw <= 64) {
+        hipLaunchKernelGGL(k_vn_order<1>, dim3(1), dim3(64), 0, s, vtx, nw, W, H);
+        hipLaunchKernelGGL(k_vnmap_rows<1>, dim3(H), row, 0, s, P, l, vtx, nrm, nw);
+    } else {
+        hipLaunchKernelGGL(k_vn_order<2>, dim3(1), dim3(64), 0, s, vtx, nw, W, H);
+        hipLaunchKernelGGL(k_vnmap_rows<2>, dim3(H), row, 0, s, P, l, vtx, nrm, nw);
+    }
 }
 
 }  // namespace vs
