@@ -1125,6 +1125,14 @@ vs_status sync_last(vs_session *s) {
     return VS_OK;
 }
 
+// Before s's stream is destroyed, its work complete: a batched step without a
+// caller's stream runs on its first session's stream, which the other sessions
+// then hold as their last one.
+void release_stream_of(const vs_session *s) {
+    for (vs_session *o : s->ctx->sessions)
+        if (o != s && o->last == s->stream) o->last = o->stream;
+}
+
 // A NULL frame keeps the raw buffer as it is (set by vs_set_depth or a pre-step).
 vs_status copy_depth(vs_session *s, const void *depth, int is_host, hipStream_t st) {
     if (!depth) return VS_OK;
@@ -1513,6 +1521,12 @@ vs_status vs_session_destroy(vs_session *s) {
         // the steps in flight, and its memory is freed in stream order after
         // them; the host waits for neither.
         vs_server *v = s->server;
+        // work outside the slot table (single operators, a batched step) on
+        // the sessions' own streams is not in that order: it is waited for
+        (void)hipStreamSynchronize(s->stream);
+        for (vs_session *o : s->ctx->sessions)
+            if (o != s && s->last == o->stream) (void)hipStreamSynchronize(o->stream);
+        release_stream_of(s);
         server_forget(s);
         drop_batches_with(s->ctx, s);
         free_batch_graph(s->self);
@@ -1533,11 +1547,7 @@ vs_status vs_session_destroy(vs_session *s) {
         return VS_OK;
     }
     (void)sync_last(s);
-    // a batched step without a caller's stream runs on its first session's
-    // stream, which the other sessions then hold as their last one: that
-    // work has just completed, and the handle ends here
-    for (vs_session *o : s->ctx->sessions)
-        if (o != s && o->last == s->stream) o->last = o->stream;
+    release_stream_of(s);
     drop_batches_with(s->ctx, s);
     free_batch_graph(s->self);
     s->timer.destroy();
