@@ -375,7 +375,9 @@ struct HostStates {
 // fresh arrays; a second stream makes it 6.4, pieces of 1 MB 4.9, eight lanes
 // change nothing.) The lanes (16 MB page-locked, one stream) are made by the
 // first large download and kept until the context ends; downloads of one
-// context take turns.
+// context take turns. Other destinations keep the runtime's copy, which moves
+// them by DMA alone (page-locked: 4.9 ms against 7.7 through the lanes, which
+// copy once more) or is the only one that may (device memory).
 constexpr int kLanes = 4;
 constexpr size_t kPiece = (size_t)2 << 20;
 constexpr size_t kStagedDownload = (size_t)16 << 20;  // smaller ones: the runtime's copy (no threads to start)
@@ -384,6 +386,13 @@ struct Download {
     const void *src;
     size_t bytes;
 };
+// Whether p is ordinary host memory, unknown to the runtime.
+bool pageable(const void *p) {
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+    (void)hipGetLastError();  // how some runtimes report such memory
+    return true;
+}
 struct Downloader {
     std::mutex m;
     hipStream_t s = nullptr;
@@ -406,20 +415,24 @@ struct Downloader {
             size_t bytes;
         };
         std::vector<Part> parts;
+        std::vector<Download> whole;  // by the runtime's copy
         size_t total = 0;
         for (const Download &d : list) {
+            if (!pageable(d.dst)) {
+                whole.push_back(d);
+                continue;
+            }
             total += d.bytes;
             for (size_t o = 0; o < d.bytes; o += kPiece)
                 parts.push_back({(char *)d.dst + o, (const char *)d.src + o, std::min(kPiece, d.bytes - o)});
         }
         std::lock_guard<std::mutex> hold(m);
-        if (total < kStagedDownload || init() != hipSuccess) {
-            for (const Download &d : list) {
-                const hipError_t e = hipMemcpy(d.dst, d.src, d.bytes, hipMemcpyDeviceToHost);
-                if (e != hipSuccess) return e;
-            }
-            return hipSuccess;
+        const bool lanes = total >= kStagedDownload && init() == hipSuccess;
+        for (const Download &d : lanes ? whole : list) {
+            const hipError_t e = hipMemcpy(d.dst, d.src, d.bytes, hipMemcpyDeviceToHost);
+            if (e != hipSuccess) return e;
         }
+        if (!lanes) return hipSuccess;
         std::atomic<int> err{hipSuccess};
         const auto work = [&](int w) {
             char *buf = pinned + (size_t)w * 2 * kPiece;
