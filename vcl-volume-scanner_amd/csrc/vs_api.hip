@@ -407,32 +407,40 @@ struct Downloader {
         if (e == hipSuccess && !pinned) e = hipHostMalloc((void **)&pinned, kLanes * 2 * kPiece, hipHostMallocDefault);
         return e;
     }
+    static hipError_t plain(const std::vector<Download> &list) {
+        for (const Download &d : list) {
+            const hipError_t e = hipMemcpy(d.dst, d.src, d.bytes, hipMemcpyDeviceToHost);
+            if (e != hipSuccess) return e;
+        }
+        return hipSuccess;
+    }
     // The device data is complete (the caller has waited for it).
     hipError_t run(int device, const std::vector<Download> &list) {
+        std::vector<Download> staged, whole;
+        size_t total = 0;
+        for (const Download &d : list) {
+            const bool p = pageable(d.dst);
+            (p ? staged : whole).push_back(d);
+            total += p ? d.bytes : 0;
+        }
+        if (total < kStagedDownload) return plain(list);
+        const hipError_t we = plain(whole);
+        if (we != hipSuccess) return we;
         struct Part {
             char *dst;
             const char *src;
             size_t bytes;
         };
         std::vector<Part> parts;
-        std::vector<Download> whole;  // by the runtime's copy
-        size_t total = 0;
-        for (const Download &d : list) {
-            if (!pageable(d.dst)) {
-                whole.push_back(d);
-                continue;
-            }
-            total += d.bytes;
+        for (const Download &d : staged)
             for (size_t o = 0; o < d.bytes; o += kPiece)
                 parts.push_back({(char *)d.dst + o, (const char *)d.src + o, std::min(kPiece, d.bytes - o)});
+        // from here on the lanes: one download at a time; smaller copies wait for nobody
+        std::unique_lock<std::mutex> hold(m);
+        if (init() != hipSuccess) {
+            hold.unlock();
+            return plain(staged);
         }
-        std::lock_guard<std::mutex> hold(m);
-        const bool lanes = total >= kStagedDownload && init() == hipSuccess;
-        for (const Download &d : lanes ? whole : list) {
-            const hipError_t e = hipMemcpy(d.dst, d.src, d.bytes, hipMemcpyDeviceToHost);
-            if (e != hipSuccess) return e;
-        }
-        if (!lanes) return hipSuccess;
         std::atomic<int> err{hipSuccess};
         const auto work = [&](int w) {
             char *buf = pinned + (size_t)w * 2 * kPiece;
