@@ -393,6 +393,17 @@ bool pageable(const void *p) {
     (void)hipGetLastError();  // how some runtimes report such memory
     return true;
 }
+// The calling thread's device for the scope's length.
+struct DeviceScope {
+    int before = -1;
+    explicit DeviceScope(int device) {
+        if (hipGetDevice(&before) != hipSuccess || before == device) before = -1;
+        (void)hipSetDevice(device);
+    }
+    ~DeviceScope() {
+        if (before >= 0) (void)hipSetDevice(before);
+    }
+};
 struct Downloader {
     std::mutex m;
     hipStream_t s = nullptr;
@@ -435,9 +446,15 @@ struct Downloader {
         for (const Download &d : staged)
             for (size_t o = 0; o < d.bytes; o += kPiece)
                 parts.push_back({(char *)d.dst + o, (const char *)d.src + o, std::min(kPiece, d.bytes - o)});
+        std::vector<std::thread> pool;
+        std::vector<int> mine;
+        pool.reserve(kLanes);
+        mine.reserve(kLanes);
         // from here on the lanes: one download at a time; smaller copies wait for nobody
         std::unique_lock<std::mutex> hold(m);
+        const DeviceScope scope(device);
         if (init() != hipSuccess) {
+            (void)hipGetLastError();  // the copy below stands in: no later call may report it
             hold.unlock();
             return plain(staged);
         }
@@ -460,8 +477,7 @@ struct Downloader {
             if (e != hipSuccess) err = e;
         };
         // lanes whose thread cannot be started are this thread's
-        std::vector<std::thread> pool;
-        std::vector<int> mine{0};
+        mine.push_back(0);
         for (int w = 1; w < kLanes; ++w) {
             try {
                 pool.emplace_back(work, w);
