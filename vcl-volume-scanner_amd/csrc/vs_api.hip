@@ -393,6 +393,14 @@ bool pageable(const void *p) {
     (void)hipGetLastError();  // how some runtimes report such memory
     return true;
 }
+// Whether a kernel on `device` can store floats at p: aligned memory of that device.
+bool kernel_writes(const void *p, int device) {
+    hipPointerAttribute_t a{};
+    if (((uintptr_t)p & 3) != 0) return false;
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeDevice && a.device == device;
+    (void)hipGetLastError();
+    return false;
+}
 // The calling thread's device for the scope's length.
 struct DeviceScope {
     int before = -1;
@@ -1685,8 +1693,13 @@ vs_status vs_bilateral_filter_depth(vs_session *s, const void *depth_in, int in_
     hipStream_t h = pick(s, stream);
     vs_status r = copy_depth(s, depth_in, in_is_host, h);
     if (r != VS_OK) return r;
-    launch_bilateral(s->self.dP, s->self.dWork[0], s->self.nWork[0], 1, depth_out_dev, h);
+    // the filter writes a buffer that its stores reach; other memory (the host's,
+    // another device's, not aligned to floats) takes a copy
+    const bool direct = depth_out_dev && kernel_writes(depth_out_dev, s->ctx->device);
+    launch_bilateral(s->self.dP, s->self.dWork[0], s->self.nWork[0], 1, direct ? depth_out_dev : nullptr, h);
     HIP_TRY(hipGetLastError());
+    if (depth_out_dev && !direct)
+        HIP_TRY(hipMemcpyAsync(depth_out_dev, s->hp.filt[0], (size_t)s->d.width * s->d.height * 4, hipMemcpyDefault, h));
     return VS_OK;
 }
 
