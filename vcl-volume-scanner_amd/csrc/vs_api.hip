@@ -297,6 +297,7 @@ struct Batch {
     uint32_t bricks = 0;    // capacity of the brick list
     uint32_t max_words = 0; // longest visible-brick bitmap of a member (32-bit words)
     int addr = kAddr64;     // how the raycast addresses the members' voxels (VoxAddr)
+    int march_groups = 0;   // raycast workgroups of the launch that a captured step makes (the largest part's)
     int integ_grid = 1;     // default integrate grid
     Shape shape;
     std::string size_class;
@@ -696,6 +697,8 @@ struct ListSet {
     vs_status settle(Batch &B, int integ_max) const {
         B.levels = levels;
         B.pyr_pair = !two_levels;
+        B.march_groups = 0;
+        for (int l = 0; l < kMaxLevels; ++l) B.march_groups += (int)tile[l].size();
         B.sd_slices = sd_slices;
         for (int l = 0; l < kMaxLevels; ++l) B.max_iters[l] = max_iters[l];
         B.bricks = bricks;
@@ -970,7 +973,7 @@ void enqueue_step(const Batch &B, hipStream_t s, Timer *timed) {
     launch_integrate(B.dP, B.n, B.bl, B.tt, B.wt, integ_grid(B), B.sd_slices, s);
     mark(5);
     const LevelWork lw = level_work(B.dWork, B.nWork, B.levels);
-    launch_raycast_march(B.dP, lw, B.tt, B.wt, nullptr, B.shape.march, B.addr, s);
+    launch_raycast_march(B.dP, lw, B.tt, B.wt, nullptr, B.shape.march, B.march_groups, B.addr, s);
     mark(6);
     launch_raycast_shade(B.dP, lw, B.tt, B.wt, nullptr, kShadeOpts[B.shape.shade].block,
                          kShadeOpts[B.shape.shade].waves, B.addr, s);
@@ -1846,6 +1849,9 @@ vs_status vs_fuse_batch(vs_ctx *ctx, vs_session *const *sessions, const uint16_t
                 nb->sub.emplace_back(new Batch());
                 r = make_ctx_batch(part, *nb->sub.back());
             }
+            // eager steps of the whole (tuned or timed) march in the form that its parts will
+            nb->march_groups = 0;
+            for (const auto &b : nb->sub) nb->march_groups = std::max(nb->march_groups, b->march_groups);
         }
         if (r != VS_OK) {
             release_batch(*nb);
@@ -2169,7 +2175,7 @@ vs_status restore_session(vs_ctx *ctx, const void *buf, size_t bytes, bool poole
         const Batch &B = s->self;
         LevelWork lw = level_work(B.dWork, B.nWork, B.levels);
         lw.force = 1;
-        launch_raycast_march(B.dP, lw, B.tt, B.wt, nullptr, kRay8x8, B.addr, s->stream);
+        launch_raycast_march(B.dP, lw, B.tt, B.wt, nullptr, kRay8x8, 0, B.addr, s->stream);
         launch_raycast_shade(B.dP, lw, B.tt, B.wt, nullptr, kRay8x8, 4, B.addr, s->stream);
         s->last = s->stream;
         if (hipGetLastError() != hipSuccess) r = fail(VS_EHIP, "restore: the render could not be launched");

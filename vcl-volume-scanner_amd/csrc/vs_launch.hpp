@@ -112,9 +112,10 @@ LevelWork level_work(const WorkItem *const work[kMaxLevels], const int n[kMaxLev
 void launch_sdist(const SessParams *P, int nsess, int sd_slices, int force, hipStream_t s);
 // Ray block of one wave in the raycast kernels (same results for each).
 enum RayBlock { kRay8x8 = 0, kRay16x4 = 1, kRay32x2 = 2 };
+// groups: the workgroups that decide the march's form (0: the launch's own);
 // addr: VoxAddr
 void launch_raycast_march(const SessParams *P, const LevelWork &lw, int tsdf_type, int weight_type,
-                          unsigned long long *stats, int ray_block, int addr, hipStream_t s);
+                          unsigned long long *stats, int ray_block, int groups, int addr, hipStream_t s);
 // waves: the waves per SIMD its registers aim for (4 or 5); addr: VoxAddr
 void launch_raycast_shade(const SessParams *P, const LevelWork &lw, int tsdf_type, int weight_type,
                           unsigned long long *stats, int ray_block, int waves, int addr, hipStream_t s);

@@ -1637,26 +1637,24 @@ __host__ constexpr int latency_groups(int addr, int rec_bytes) {
     return addr != kAddrSmall ? 2048 : rec_bytes == 4 ? 32768 : 8192;
 }
 template <class TV, class TW>
-static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int addr,
+static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int groups, int addr,
                     hipStream_t s) {
     const int n = lw.blocks();
     if (n <= 0) return;
-#define VS_MARCH_A(RB_, AD_) \
-    hipLaunchKernelGGL((k_raycast<TV, TW, false, RB_, AD_, false>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats)
-#define VS_MARCH_L(AD_) \
-    hipLaunchKernelGGL((k_raycast<TV, TW, false, kRay8x8, AD_, true>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats)
-#define VS_MARCH(RB_)                                        \
-    do {                                                     \
-        if (addr == kAddrSmall) VS_MARCH_A(RB_, kAddrSmall); \
-        else if (addr == kAddr32) VS_MARCH_A(RB_, kAddr32);  \
-        else VS_MARCH_A(RB_, kAddr64);                       \
+    const bool lat = (groups ? groups : n) <= latency_groups(addr, (int)sizeof(typename VoxRec<TV, TW>::T));
+#define VS_MARCH_A(RB_, AD_, LAT_) \
+    hipLaunchKernelGGL((k_raycast<TV, TW, false, RB_, AD_, LAT_>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats)
+#define VS_MARCH(RB_)                                                    \
+    do {                                                                 \
+        if (lat && addr != kAddr64) VS_MARCH_A(RB_, kAddr32, true);      \
+        else if (lat) VS_MARCH_A(RB_, kAddr64, true);                    \
+        else if (addr == kAddrSmall) VS_MARCH_A(RB_, kAddrSmall, false); \
+        else if (addr == kAddr32) VS_MARCH_A(RB_, kAddr32, false);       \
+        else VS_MARCH_A(RB_, kAddr64, false);                            \
     } while (0)
     if (stats)
         hipLaunchKernelGGL((k_raycast<TV, TW, true, kRay8x8, kAddr64, false>), dim3(n), dim3(kTileThreads), 0, s, P, lw, stats);
-    else if (n <= latency_groups(addr, (int)sizeof(typename VoxRec<TV, TW>::T))) {
-        if (addr != kAddr64) VS_MARCH_L(kAddr32);
-        else VS_MARCH_L(kAddr64);
-    } else if (rb == kRay16x4)
+    else if (rb == kRay16x4)
         VS_MARCH(kRay16x4);
     else if (rb == kRay32x2)
         VS_MARCH(kRay32x2);
@@ -1664,7 +1662,6 @@ static void march_t(const SessParams *P, const LevelWork &lw, unsigned long long
         VS_MARCH(kRay8x8);
 #undef VS_MARCH
 #undef VS_MARCH_A
-#undef VS_MARCH_L
 }
 template <class TV, class TW>
 static void shade_t(const SessParams *P, const LevelWork &lw, unsigned long long *stats, int rb, int waves,
@@ -1714,8 +1711,8 @@ LevelWork level_work(const WorkItem *const work[kMaxLevels], const int n[kMaxLev
     return lw;
 }
 void launch_raycast_march(const SessParams *P, const LevelWork &lw, int tt, int wt, unsigned long long *stats,
-                          int rb, int addr, hipStream_t s) {
-    VS_DISPATCH(tt, wt, march_t, P, lw, stats, rb, addr, s);
+                          int rb, int groups, int addr, hipStream_t s) {
+    VS_DISPATCH(tt, wt, march_t, P, lw, stats, rb, groups, addr, s);
 }
 void launch_raycast_shade(const SessParams *P, const LevelWork &lw, int tt, int wt, unsigned long long *stats,
                           int rb, int waves, int addr, hipStream_t s) {
@@ -1735,13 +1732,13 @@ static LevelWork one_level(const WorkItem *work, int n, int level) {
 void launch_raycast(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt, int addr,
                     const MapsOut *out, hipStream_t s) {
     const LevelWork lw = one_level(work, n, level);
-    launch_raycast_march(P, lw, tt, wt, nullptr, kRay8x8, addr, s);
+    launch_raycast_march(P, lw, tt, wt, nullptr, kRay8x8, 0, addr, s);
     VS_DISPATCH(tt, wt, shade_t, P, lw, nullptr, kRay8x8, 4, addr, out, s);
 }
 void launch_raycast_stats(const SessParams *P, const WorkItem *work, int n, int level, int tt, int wt,
                           unsigned long long *stats, hipStream_t s) {
     const LevelWork lw = one_level(work, n, level);
-    launch_raycast_march(P, lw, tt, wt, stats, kRay8x8, kAddr64, s);
+    launch_raycast_march(P, lw, tt, wt, stats, kRay8x8, 0, kAddr64, s);
     launch_raycast_shade(P, lw, tt, wt, stats, kRay32x2, 4, kAddr64, s);
 }
 
