@@ -436,8 +436,11 @@ struct Downloader {
     }
     // The device data is complete (the caller has waited for it).
     hipError_t run(int device, const std::vector<Download> &list) {
-        std::vector<Download> staged, whole;
         size_t total = 0;
+        for (const Download &d : list) total += d.bytes;
+        if (total < kStagedDownload) return plain(list);
+        std::vector<Download> staged, whole;
+        total = 0;
         for (const Download &d : list) {
             const bool p = pageable(d.dst);
             (p ? staged : whole).push_back(d);
