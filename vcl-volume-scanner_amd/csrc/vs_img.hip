@@ -445,8 +445,9 @@ __global__ __launch_bounds__(256) void k_gather_depth(const SessParams *__restri
 }
 
 // Image buffers of a new session: empty pyramid, images and textures, model
-// maps at the -100 sentinel, the reprojection's keys empty, in one launch (a fill per buffer had cost an open
-// ~12 launches). Every buffer is 256-byte aligned and padded.
+// maps at the -100 sentinel, the reprojection's keys empty, in one launch (a
+// fill per buffer had cost an open ~12 launches). Every buffer is 256-byte
+// aligned and padded.
 __global__ __launch_bounds__(256) void k_session_init(const SessParams *__restrict__ SP, uint32_t *keys) {
     const SessParams &P = SP[0];
     const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
@@ -478,8 +479,9 @@ void launch_pyramid(const SessParams *P, const WorkItem *const work[kMaxLevels],
                     bool pair, int force, hipStream_t s) {
     if (levels == 3 && pair) {
         if (n[2] <= 0) return;
-        // 16 waves a tile while that leaves a CU for nearly every one of them
-        if (n[2] <= 1024)
+        // 16 waves a tile against 4, us in a step: 75 tiles 7.5 / 11.0, 300 8.4 / 11.4,
+        // 600 11.8 / 12.5, 975 13.9 / 13.2, 1200 16.7 / 13.7, 4800 44.1 / 35.6
+        if (n[2] <= 768)
             hipLaunchKernelGGL(k_pyr_down2<1024>, dim3(n[2]), dim3(1024), 0, s, P, work[2], force);
         else
             hipLaunchKernelGGL(k_pyr_down2<kTileThreads>, dim3(n[2]), dim3(kTileThreads), 0, s, P, work[2], force);
