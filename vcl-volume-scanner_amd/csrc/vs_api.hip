@@ -197,7 +197,7 @@ size_t frame_bytes(const vs_session_desc &d) {
 // ---------------------------------------------------------------------------
 // Events around the stages of one frame step:
 //   [0,1) track setup + bilateral   [1,2) pyramid    [2,3) ICP + finalize
-//   [3,4) brick clear + mark        [4,5) integrate  [5,6) raycast march, all levels
+//   [3,4) brick mark + list         [4,5) integrate  [5,6) raycast march, all levels
 //   [6,7) raycast shading, all levels                [7,8) empty
 constexpr int kMarks = 9;
 struct Timer {

@@ -8,7 +8,9 @@
 // FP64 partial of the 29 sums per group of tiles, then k_icp_solve (one
 // workgroup per session) sums them in FP64 in a fixed order, solves the 6x6
 // system (Cholesky, FP64), applies the SE(3) update and publishes the FP32
-// pose the next iteration reads. Convergence (|x|_inf < 5e-7) and failure are
+// pose the next iteration reads. Small launches take one launch per iteration,
+// in which every workgroup solves the last one's system before its sums
+// (k_icp_step, the same results). Convergence (|x|_inf < 5e-7) and failure are
 // flags the following launches test, so the host enqueues a fixed launch
 // sequence that can be captured in a graph.
 #include "vs_device.hpp"

@@ -11,8 +11,8 @@
 //
 // Per-session bitmaps: `bvis` (bricks touched by the current frame, rebuilt
 // each frame from the per-brick flags `vmask`), `bocc` (bricks holding any
-// voxel of weight > 0; weights never
-// decrease, so the bit is set once and kept) and the band bits `bband` /
+// voxel of weight > 0; weights never decrease, so the bit is set once and
+// kept) and the band bits `bband` /
 // `sband` (bricks / superbricks that may hold a voxel of weight > 0 and a value
 // other than 1.0; set when an update writes such a value, and kept).
 #include <type_traits>
@@ -79,13 +79,11 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_mark(const SessParams *__r
 // the batch's brick list. Workgroup (c, s) takes bricks [c, c + 1) *
 // kVisListBricks of session s: each thread packs the flags of 32 * WPT
 // consecutive bricks (16-byte loads) into WPT bit words and stores them
-// (clearing the flags it found set),
-// then the workgroup ranks the set bits (popcounts and a prefix sum),
-// reserves their range with one atomic on the list counter (8 workgroups of WPT 4 for
-// a 512^3 session) and writes (session, brick) in brick order, each thread
-// its own bricks.
+// (clearing the flags it found set), then the workgroup ranks the set bits
+// (popcounts and a prefix sum), reserves their range with one atomic on the
+// list counter (8 workgroups of WPT 4 for a 512^3 session) and writes
+// (session, brick) in brick order, each thread its own bricks.
 template <int WPT>
-
 __global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__restrict__ SP, BrickList bl, int force) {
     constexpr uint32_t kVisListBricks = 32u * WPT * kTileThreads;
     __shared__ unsigned wsum[kTileThreads / 64];
@@ -98,7 +96,7 @@ __global__ __launch_bounds__(kTileThreads) void k_vis_list(const SessParams *__r
     const uint32_t b0 = blockIdx.x * kVisListBricks + threadIdx.x * (32u * WPT);
     if (blockIdx.x * kVisListBricks >= nb) return;
     uint32_t w[WPT] = {};
-    if (b0 < nb) {  // flags padded to 128 bricks: the 128 read here are in the buffer
+    if (b0 < nb) {  // flags padded to 128 bricks: the 32 * WPT read here are in the buffer
         vs_u4 *f = (vs_u4 *)(P.vmask + b0);
         vs_u4 fl[2 * WPT];
 #pragma unroll
@@ -263,9 +261,10 @@ __device__ __forceinline__ void st_rec4(void *base, size_t i, const typename Vox
 }
 
 // The integrate walks the brick list in chunks of up to kIntegChunk
-// consecutive entries. The list comes from k_vis_mark in (session, image tile) order, so
-// a chunk's bricks mostly belong to one session and lie behind one small
-// patch of its depth frame. Workgroup g runs on XCD g % 8 (workgroups are
+// consecutive entries. The list comes from k_vis_list, whose workgroups write
+// runs of one session's bricks in brick order, so a chunk's bricks mostly
+// belong to one session and, neighbours along x, lie behind one small patch of
+// its depth frame. Workgroup g runs on XCD g % 8 (workgroups are
 // dealt to the eight XCDs in turn), and the workgroups of one XCD take the
 // chunks of one contiguous eighth of the list: the depth rows that
 // neighbouring bricks read are then fetched into that XCD's L2 once, not
@@ -791,12 +790,13 @@ constexpr float kSkipMargin = 0.25f;
 // the grid leaves it for good, and the iteration after the skip ends it as the
 // miss that it is. With t = (reach - sign(rd) (v - m)) / |rd|, ri the ray's
 // reciprocal direction, an axis costs 6 operations; an axis the ray does not
-// move along gives NaN or infinity, which the minimum passes over. (Bounds picked by the direction's sign and clipped
-// to the grid, and the trilinear corners as brick and in-brick offsets, had
-// been 100 of ~400 vector operations of a loop iteration: 64-session step 6.62
-// -> 6.32 ms, 1280x960 scan into 1024^3 1166 -> 1127 us, 640x480 scan 413 ->
-// 403, 264x200x312 render 100 -> 95; reciprocals once per ray instead of three
-// per skip then 6.20 -> 6.15 ms, 397 -> 394 us, 104 -> 102.)
+// move along gives NaN or infinity, which the minimum passes over. (Bounds
+// picked by the direction's sign and clipped to the grid, and the trilinear
+// corners as brick and in-brick offsets, had been 100 of ~400 vector operations
+// of a loop iteration: 64-session step 6.62 -> 6.32 ms, 1280x960 scan into
+// 1024^3 1166 -> 1127 us, 640x480 scan 413 -> 403, 264x200x312 render 100 -> 95;
+// reciprocals once per ray instead of three per skip then 6.20 -> 6.15 ms, 397 ->
+// 394 us, 104 -> 102.)
 __device__ __forceinline__ int steps_in_box(f3 v, f3 ri, float S, const FreeBox &box) {
     const float unit = (float)(1 << box.sh), mid = 0.5f * unit - 0.5f;
     const float reach = (float)box.r * unit + (0.5f * unit - kSkipMargin);
@@ -973,8 +973,9 @@ __device__ __forceinline__ bool cast_ray(const Vol<TV, TW, AD> &V, const RayCons
 // branches, and up to three dependent rounds of loads. Here the sizes stay in
 // vector registers, the tests are flags, and one round loads the band word,
 // the nearest record and the eight trilinear corners together (the corners of
-// a stencil that leaves the grid read the origin's and count as failed). Decisions and values are cast_ray's: the same FP32 operations on
-// the same operands.
+// a stencil that leaves the grid read the origin's and count as failed).
+// Decisions and values are cast_ray's: the same FP32 operations on the same
+// operands.
 template <class TV, class TW, int AD>
 __device__ __forceinline__ bool cast_ray_latency(const Vol<TV, TW, AD> &V, const RayConst &C, const float *Tcg,
                                                  float px, float py, f3 &hit) {
@@ -1595,7 +1596,9 @@ void launch_vis_mark(const SessParams *P, const WorkItem *work, int n, int nsess
     hipLaunchKernelGGL(k_vis_mark, dim3(n), dim3(kTileThreads), 0, s, P, work, force);
     // 32 bricks a thread while that keeps the launch small (a thread writes its
     // bricks one after another, and one session's surface crosses few threads'
-    // ranges: 640x480 scan 423 -> 418 us), else 128 and a quarter of the atomics
+    // ranges), else 128 and a quarter of the atomics. The visibility stage with
+    // 32 / 128: 32 workgroups of the former 15.7 / 21.6 us, 256 39.4 / 44.6, 512 67.5 /
+    // 71.1, 768 97.6 / 98.5, 1024 127.3 / 126.0, 2048 244.4 / 241.1
     const auto blocks = [&](uint32_t wpt) { return (max_words + wpt * kTileThreads - 1) / (wpt * kTileThreads); };
     if (blocks(1) * (uint32_t)nsess <= 512u)
         hipLaunchKernelGGL(k_vis_list<1>, dim3(blocks(1), nsess), dim3(kTileThreads), 0, s, P, bl, force);
@@ -1621,18 +1624,26 @@ void launch_integrate(const SessParams *P, int nsess, BrickList bl, int tt, int 
     launch_sdist(P, nsess, sd_slices, 0, s);
 }
 
-// Launches of up to this many workgroups take the latency form of the march.
-// 2048, the 8 per CU that are resident at once on 256 CUs, for any grid (fused
-// frame with a 1200-workgroup preview: 1575 workgroups at 640x480 / 256^3, 427
-// us in the wide form and 402 in the latency form; 1443 at 603x451 in colour,
-// 503 / 431; three levels of 1260, 300 and 75, 116 / 102). Above it the waves'
-// own number hides their latency, and what counts is each form's work per ray:
-// grids of small superbricks, whose boxes are short, gain from the latency
-// form's fewer branches (6300 workgroups at 1280x960 / 512^3 with 4-byte records
-// 1069 / 992, 3 sessions of 640x480 / 256^3 764 / 703, 16 of 384^3 2039 / 1960,
-// a server's 24168 1112 / 1076; 8-byte records 4700 workgroups 556 / 532, 6300
-// 756 / 751, 12600 equal; 4-byte 33075 equal), larger grids lose (6300 at
-// 1280x960 / 1024^3 1036 / 1074).
+// Launches of up to this many workgroups take the latency form of the march
+// (of a batch that a captured step runs in parts: the largest part's). Measured
+// crossovers (the form's 5 to 7 waves per SIMD hold 1280 to 1792 workgroups at
+// once).
+// Any grid, 2048: fused frame with a 1200-workgroup preview, 1575 workgroups at
+// 640x480 / 256^3 427 us in the wide form and 402 in the latency form, 1443 at
+// 603x451 in colour 503 / 431, three levels of 1260, 300 and 75 116 / 102; 6300
+// at 1280x960 / 1024^3 1036 / 1074.
+// Grids of small superbricks, whose boxes are short, gain from the latency
+// form's fewer branches and its loads in flight together, the more so the colder
+// the volumes. 8-byte records, 8192: 4700 workgroups 556 / 532 us, 6300 756 /
+// 751, 12600 907 / 910, 25200 1385 / 1417. 4-byte records, 32768, in steps over
+// volumes that other sessions' steps displace from the caches, address
+// translations included (three sets of sessions in turn): 12 sessions of 640x480 / 256^3 1437 /
+// 1353, 15 of 512^3 2142 / 2046, 16 of 384^3 2124 / 2034, 40 of 512^3 4153 / 4013,
+// a server's 24168 1112 / 1076. One set of sessions alone, step after step, is
+// equal up to 16000 workgroups (8 of 512^3 1076 / 1062, 10 of 256^3 1039 / 1038)
+// and a little slower from there to the line (16 of 384^3 1532 / 1542, 24 of 256^3
+// 1915 / 1964, 40 of 512^3 3750 / 3794), as is a set's first step (1 to 3%); the
+// line is where the first kind's gain ends (33075 equal).
 __host__ constexpr int latency_groups(int addr, int rec_bytes) {
     return addr != kAddrSmall ? 2048 : rec_bytes == 4 ? 32768 : 8192;
 }
