@@ -169,8 +169,9 @@ vs_status vs_vertex_normal_maps(vs_session *s, int level, float *vtx_dev, float 
  * left or upper neighbour was invalidated gets no normal (and, if grazing
  * itself, keeps its vertex). vs_vertex_normal_maps evaluates every pixel on
  * the input map instead (order-independent); the two differ only next to
- * grazing pixels. vtx_dev also holds the ordering's bits until the call has run:
- * calls on several streams need nothing but buffers of their own. */
+ * grazing pixels. With a stream of the caller's, vtx_dev also holds the ordering's
+ * bits until the call has run: calls on several streams need nothing but buffers
+ * of their own. */
 vs_status vs_vertex_normal_maps_inplace(vs_session *s, int level, float *vtx_dev, float *nrm_dev,
                                         vs_stream stream);
 /* A8-A12: projective point-to-plane ICP of the frame pyramid against the

@@ -71,6 +71,7 @@ struct Layout {
     size_t state, raw, filt[kMaxLevels], mvn[kMaxLevels], mimg[kMaxLevels];
     size_t vox, bvis, vmask, bocc, bband, sband, sdist, sdtmp, icp_part, diag_part, diag_mask, lists, params, stats, keys;
     size_t vcol, rgb, mtex[kMaxLevels];  // colour sessions only (0 otherwise)
+    size_t vnbits[kMaxLevels];            // in-place normal maps on the session's own stream: one bit per pixel
     size_t wtab;                          // voxel-centre world coordinates, x then y then z
     size_t total;
     size_t nvox;
@@ -132,6 +133,7 @@ Layout make_layout(const vs_session_desc &d) {
         L.filt[l] = take(n * 4);
         L.mvn[l] = take((n + 1) * 2 * sizeof(MapXYZ));  // vertex + normal per pixel, one padding pixel
         L.mimg[l] = take(n);
+        L.vnbits[l] = take((size_t)vn_words(Wl) * Hl * 8);
     }
     // value and weight of a voxel in one record (4 bytes for FP16 + u8, 8
     // otherwise)
@@ -541,6 +543,7 @@ struct vs_session {
     SessParams hp{};
     SessState *st = nullptr;
     HostState *host = nullptr;
+    std::mutex vn_turn;  // vs_vertex_normal_maps_inplace on the own stream
     hipStream_t stream = nullptr;
     hipStream_t last = nullptr;
     Batch self;
@@ -1733,7 +1736,12 @@ vs_status vs_vertex_normal_maps_inplace(vs_session *s, int level, float *vtx_dev
     if (level < 0 || level >= s->d.levels) return fail(VS_EINVAL, "level %d", level);
     hipStream_t h = pick(s, stream);
     const LevelDesc &ld = s->hp.lev[level];
-    launch_vnmap_inplace(s->self.dP, level, ld.W, ld.H, vtx_dev, nrm_dev, h);
+    // the session's scratch serves its own stream, where one call follows another
+    // (whole: threads that call at once take turns); calls on other streams share nothing
+    std::unique_lock<std::mutex> whole(s->vn_turn, std::defer_lock);
+    if (!stream) whole.lock();
+    launch_vnmap_inplace(s->self.dP, s->self.dWork[level], s->self.nWork[level], level, ld.W, ld.H,
+                         stream ? nullptr : s->mem + s->L.vnbits[level], vtx_dev, nrm_dev, h);
     HIP_TRY(hipGetLastError());
     return VS_OK;
 }

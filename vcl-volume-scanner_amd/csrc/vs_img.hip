@@ -245,10 +245,13 @@ __device__ __forceinline__ void put_vn(const VnPixel &r, bool gone, float *vtx, 
     stg(nrm, 3 * t + 1, r.normal ? r.n.y : -100.f);
     stg(nrm, 3 * t + 2, r.normal ? r.n.z : -100.f);
 }
-// Every pixel evaluated on the input vertex map (the order-independent form).
+// Without `inv`: every pixel evaluated on the input vertex map (the
+// order-independent form). With it (the reference loop's in-place order,
+// below): one bit per pixel, rows of `nw` 64-bit words, set where the loop
+// invalidates the vertex.
 __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__restrict__ SP,
                                                         const WorkItem *__restrict__ work, int l, float *vtx,
-                                                        float *nrm) {
+                                                        float *nrm, const unsigned long long *inv, int nw) {
     const WorkItem wi = work[blockIdx.x];
     const SessParams &P = SP[wi.sess];
     const LevelDesc &L = P.lev[l];
@@ -256,8 +259,16 @@ __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__rest
     const int x = (wi.tile % L.tiles_x) * kTileW + threadIdx.x % kTileW;
     const int y = (wi.tile / L.tiles_x) * kTileH + threadIdx.x / kTileW;
     if (x >= W || y >= H) return;
-    const VnPixel r = vn_pixel(P.filt[l], L.K, W, H, x, y);
-    put_vn(r, r.grazing, vtx, nrm, (size_t)y * W + x);
+    VnPixel r = vn_pixel(P.filt[l], L.K, W, H, x, y);
+    bool gone = r.grazing;
+    if (inv) {
+        auto bit = [&](int xx, int yy) -> bool {
+            return xx >= 0 && yy >= 0 && ((ldg(inv, (size_t)yy * nw + (xx >> 6)) >> (xx & 63)) & 1ull);
+        };
+        gone = bit(x, y);
+        r.normal &= !(bit(x - 1, y) || bit(x, y - 1));
+    }
+    put_vn(r, gone, vtx, nrm, (size_t)y * W + x);
 }
 
 // The reference CPU loop's in-place order (enm_Estimate_Normal_Map,
@@ -276,15 +287,22 @@ __global__ __launch_bounds__(kTileThreads) void k_vnmap(const SessParams *__rest
 // level: frame preparation and the maps of three levels of a 640x480 frame,
 // alone, 9.31 -> 0.19 ms.)
 //
-// The bits live in the caller's vertex map until the last launch writes it, so
-// calls on several streams share nothing: row y's 12 W bytes begin with its
-// bits of c (vn_words(W) words of 64 pixels, bit 0 the leftmost), followed by
-// the ordered bits of row y - 1. The last launch's workgroup for a row finds
-// both in the row that it alone overwrites, and takes the recurrence's step for
-// its row once more. (Bits in a scratch of the session's were 1 us of 54 faster
-// for the 640x480 frame's preparation, and made calls for one session and level
-// on two streams race.) A map is aligned to 4 bytes, hence the half words.
-__device__ __forceinline__ uint32_t *vn_row(float *vtx, int W, int y) { return (uint32_t *)vtx + (size_t)y * 3 * W; }
+// Where the bits are, a row's vn_words(W) words of 64 pixels, bit 0 the leftmost:
+//   calls on the session's own stream, which follow one another: in a scratch
+//   of the session's, where the ordered bits of a row replace its bits of c;
+//   calls on a caller's stream, of which several may run at once (MAP): in the
+//   caller's vertex map, until the last launch writes it. Row y's 12 W bytes
+//   begin with its bits of c, followed by the ordered bits of row y - 1; the
+//   last launch's workgroup for a row finds both in the row that it alone
+//   overwrites, and takes the recurrence's step for its row once more. (640x480
+//   frame preparation 54.0 us with the scratch, 55.0 so.) A map is aligned to
+//   4 bytes, hence the half words.
+template <bool MAP>
+struct VnBits {
+    static __device__ __forceinline__ uint32_t *row(uint32_t *bits, int nw, int W, int y) {
+        return bits + (size_t)y * (MAP ? 3 * W : 2 * nw);
+    }
+};
 __device__ __forceinline__ unsigned long long ld_word(const uint32_t *row, int k) {
     return (unsigned long long)ldg(row, 2 * k) | (unsigned long long)ldg(row, 2 * k + 1) << 32;
 }
@@ -294,7 +312,8 @@ __device__ __forceinline__ void st_word(uint32_t *row, int k, unsigned long long
 }
 
 // One wave per 64 pixels of a row: word k of row y = bits of c.
-__global__ __launch_bounds__(kTileThreads) void k_vn_graze(const SessParams *__restrict__ SP, int l, float *vtx,
+template <bool MAP>
+__global__ __launch_bounds__(kTileThreads) void k_vn_graze(const SessParams *__restrict__ SP, int l, uint32_t *bits,
                                                            int nw) {
     const SessParams &P = SP[0];
     const LevelDesc &L = P.lev[l];
@@ -304,7 +323,7 @@ __global__ __launch_bounds__(kTileThreads) void k_vn_graze(const SessParams *__r
     const int x = k * 64 + (threadIdx.x & 63);
     const bool c = x < L.W && vn_pixel(P.filt[l], L.K, L.W, L.H, x, y).grazing;
     const unsigned long long m = __ballot(c);
-    if ((threadIdx.x & 63) == 0) st_word(vn_row(vtx, L.W, y), k, m);
+    if ((threadIdx.x & 63) == 0) st_word(VnBits<MAP>::row(bits, nw, L.W, y), k, m);
 }
 
 // One step of the recurrence by one wave, lane k holding words k * N .. k * N +
@@ -342,11 +361,12 @@ __device__ __forceinline__ void vn_order_row(const unsigned long long *c, unsign
     }
 }
 
-// The recurrence over all rows by one wave: the ordered bits of the row above
-// into each row. Bound: a chain of ~25 dependent instructions per row; the
-// rows' bits are loaded kAhead rows ahead of their use.
-template <int N>
-__global__ __launch_bounds__(64) void k_vn_order(float *vtx, int nw, int W, int H) {
+// The recurrence over all rows by one wave: a row's ordered bits in place, or
+// (MAP) those of the row above behind its bits of c. Bound: a chain of ~25
+// dependent instructions per row; the rows' bits are loaded kAhead rows ahead
+// of their use.
+template <int N, bool MAP>
+__global__ __launch_bounds__(64) void k_vn_order(uint32_t *bits, int nw, int W, int H) {
     constexpr int kAhead = 16;
     const int lane = threadIdx.x;
     unsigned long long up[N], nxt[kAhead][N];
@@ -358,7 +378,7 @@ __global__ __launch_bounds__(64) void k_vn_order(float *vtx, int nw, int W, int 
 #pragma unroll
             for (int q = 0; q < N; ++q) {
                 const int k = lane * N + q;
-                nxt[a][q] = (k < nw && row0 + a < H) ? ld_word(vn_row(vtx, W, row0 + a), k) : 0ull;
+                nxt[a][q] = (k < nw && row0 + a < H) ? ld_word(VnBits<MAP>::row(bits, nw, W, row0 + a), k) : 0ull;
             }
     };
     fetch(0);
@@ -371,17 +391,19 @@ __global__ __launch_bounds__(64) void k_vn_order(float *vtx, int nw, int W, int 
         fetch(row0 + kAhead);
 #pragma unroll
         for (int a = 0; a < kAhead; ++a) {
+            if (!MAP) vn_order_row<N>(cur[a], up, lane);
 #pragma unroll
             for (int q = 0; q < N; ++q) {
                 const int k = lane * N + q;
-                if (k < nw && row0 + a < H) st_word(vn_row(vtx, W, row0 + a), nw + k, up[q]);
+                if (k < nw && row0 + a < H)
+                    st_word(VnBits<MAP>::row(bits, nw, W, row0 + a), MAP ? nw + k : k, up[q]);
             }
-            vn_order_row<N>(cur[a], up, lane);
+            if (MAP) vn_order_row<N>(cur[a], up, lane);
         }
     }
 }
 
-// The maps, one workgroup per row: its ordered bits and the row above's into
+// The maps from bits in the vertex map, one workgroup per row: its ordered bits and the row above's into
 // LDS by the first wave, then the row's pixels over what they were read from.
 // A thread per pixel of the row while the workgroup holds them.
 template <int N>
@@ -393,7 +415,7 @@ __global__ __launch_bounds__(1024) void k_vnmap_rows(const SessParams *__restric
     const int W = L.W, y = blockIdx.x;
     unsigned long long c[N], up[N];
     if (threadIdx.x < 64) {
-        const uint32_t *row = vn_row(vtx, W, y);
+        const uint32_t *row = VnBits<true>::row((uint32_t *)vtx, nw, W, y);
 #pragma unroll
         for (int q = 0; q < N; ++q) {
             const int k = threadIdx.x * N + q;
@@ -492,18 +514,32 @@ void launch_pyramid(const SessParams *P, const WorkItem *const work[kMaxLevels],
 }
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int l, float *vtx, float *nrm, hipStream_t s) {
     if (n > 0)
-        hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm);
+        hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm,
+                           (const unsigned long long *)nullptr, 0);
 }
-void launch_vnmap_inplace(const SessParams *P, int l, int W, int H, float *vtx, float *nrm, hipStream_t s) {
+void launch_vnmap_inplace(const SessParams *P, const WorkItem *work, int n, int l, int W, int H, void *scratch,
+                          float *vtx, float *nrm, hipStream_t s) {
+    if (n <= 0) return;
     const int nw = vn_words(W);  // at most 128 (frames are at most 8192 wide)
-    const size_t items = (size_t)nw * H, per = kTileThreads / 64;
+    const size_t per = kTileThreads / 64, grid = ((size_t)nw * H + per - 1) / per;
+    uint32_t *bits = (uint32_t *)(scratch ? scratch : vtx);
+    if (scratch) {
+        hipLaunchKernelGGL(k_vn_graze<false>, dim3((unsigned)grid), dim3(kTileThreads), 0, s, P, l, bits, nw);
+        if (nw <= 64)
+            hipLaunchKernelGGL((k_vn_order<1, false>), dim3(1), dim3(64), 0, s, bits, nw, W, H);
+        else
+            hipLaunchKernelGGL((k_vn_order<2, false>), dim3(1), dim3(64), 0, s, bits, nw, W, H);
+        hipLaunchKernelGGL(k_vnmap, dim3(n), dim3(kTileThreads), 0, s, P, work, l, vtx, nrm,
+                           (const unsigned long long *)scratch, nw);
+        return;
+    }
     const dim3 row(std::min(nw * 64, 1024));
-    hipLaunchKernelGGL(k_vn_graze, dim3((unsigned)((items + per - 1) / per)), dim3(kTileThreads), 0, s, P, l, vtx, nw);
+    hipLaunchKernelGGL(k_vn_graze<true>, dim3((unsigned)grid), dim3(kTileThreads), 0, s, P, l, bits, nw);
     if (nw <= 64) {
-        hipLaunchKernelGGL(k_vn_order<1>, dim3(1), dim3(64), 0, s, vtx, nw, W, H);
+        hipLaunchKernelGGL((k_vn_order<1, true>), dim3(1), dim3(64), 0, s, bits, nw, W, H);
         hipLaunchKernelGGL(k_vnmap_rows<1>, dim3(H), row, 0, s, P, l, vtx, nrm, nw);
     } else {
-        hipLaunchKernelGGL(k_vn_order<2>, dim3(1), dim3(64), 0, s, vtx, nw, W, H);
+        hipLaunchKernelGGL((k_vn_order<2, true>), dim3(1), dim3(64), 0, s, bits, nw, W, H);
         hipLaunchKernelGGL(k_vnmap_rows<2>, dim3(H), row, 0, s, P, l, vtx, nrm, nw);
     }
 }

@@ -28,9 +28,12 @@ void launch_bilateral(const SessParams *P, const WorkItem *work, int n, int forc
 void launch_pyramid(const SessParams *P, const WorkItem *const work[kMaxLevels], const int n[kMaxLevels], int levels,
                     bool pair, int force, hipStream_t s);
 void launch_vnmap(const SessParams *P, const WorkItem *work, int n, int level, float *vtx, float *nrm, hipStream_t s);
-// single session (P[0]), the reference loop's in-place order of a W x H level
+// single session (P[0]), the reference loop's in-place order of a W x H level;
+// scratch: vn_words(W) * H 64-bit words that no other call uses meanwhile, null:
+// the vertex map serves
 constexpr int vn_words(int W) { return (W + 63) / 64; }
-void launch_vnmap_inplace(const SessParams *P, int level, int W, int H, float *vtx, float *nrm, hipStream_t s);
+void launch_vnmap_inplace(const SessParams *P, const WorkItem *work, int n, int level, int W, int H, void *scratch,
+                          float *vtx, float *nrm, hipStream_t s);
 
 // tracker (vs_icp.hip); nsess = sessions in the batch
 void launch_track_setup(const SessParams *P, int nsess, const double *T_init, hipStream_t s);
