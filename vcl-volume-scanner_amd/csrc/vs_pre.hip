@@ -59,6 +59,7 @@ __global__ __launch_bounds__(256) void k_depth_reproject(const T *__restrict__ s
     for (int r = 0; r < kRepRows; ++r) {
         const float td = depth_value<T>(raw[r]);
         tx[r] = -1;
+        ty[r] = 0;
         if (td > 0.0f) {
             const float x = (float)x0, y = (float)(y0 + r);
             const f3 p = {td * (x - Ks[2]) / Ks[0], td * (y - Ks[3]) / Ks[1], td};
